@@ -9,45 +9,57 @@
 // Operands.  P is recomputed from the forward's per-token codes exactly as the
 // forward scores them, s = acc * qd * kd (qd carrying sm_scale*log2(e)),
 // p = 2^(s - lse) with the forward's base-2 LSE.  The quantization kernel
-// supplies the Q and smoothed-K codes and scales and, given dO in place of V,
-// the T image of dO; one preparation launch (bwd_prep_kernel) writes the T
-// images of Q and K~, the R images of dO and V and D = rowsum(dO * O).
+// supplies the Q and smoothed-K codes and scales; one preparation launch
+// (bwd_prep_kernel) writes the rows K~ = bf16(k - mean), -D = -rowsum(dO * O)
+// and the LSE padded to whole blocks.  Q, dO, V and K~ are read as the plain
+// bf16 rows they are.
 //
-// T image of bf16 rows X [N, D]: per 64-token block, chunks (j, b, tt) of 64
-// lanes x 8 bf16, element 4jj + i of lane 32hh + r holding
-// X[32b + 16tt + 8jj + 4hh + i][32j + r].  It is the operand of
-// v_mfma_f32_32x32x16_bf16 for a contraction over tokens whose other operand
-// comes straight from a 32x32 accumulator (lane (h, r) holding rows
-// 8J + 4h + i, element 4J + i): lane half h supplies the same 8 tokens to both
-// operands.  The forward's bf16 V operand is the T image of V.
-// R image: per 32-token block and 16-channel group, lane (h, r) holds the 16
-// bytes X[r][8h, +8) of the group: the row operand of the same instruction for
-// a contraction over channels.
+// Rows in LDS.  One copy of a 32-row block serves both as the row operand of
+// v_mfma_f32_32x32x16_bf16 (contraction over channels: lane (h, r) reads the
+// 16 bytes of row r, channels [16c2 + 8h, +8)) and, through the transposing
+// LDS read (ds_read_b64_tr_b16: a group of 16 lanes reads 4 rows x 16 channels
+// and each lane gets one channel's 4 rows), as the operand of a contraction
+// over rows, in exactly the row order in which a lane of a 32x32 accumulator
+// holds its rows (8J + 4h + i): P and dS go from the accumulator registers
+// into the next product without a shuffle.  The order of the copy (struct
+// Rows) keeps both reads free of bank conflicts and every address one
+// lane-constant base plus an immediate.
 //
-// Workgroups have 8 waves, two per SIMD; stages pass through a two-stage LDS
-// ring filled by direct global -> LDS loads issued one stage ahead (one
-// barrier per stage).  Work items are dealt to XCDs in contiguous ranges.
-// One launch (bwd_kernel) runs the dK/dV items, then the dQ items.
+// Two independent workgroups of 4 waves share a CU (at most 80 KB of LDS and
+// 256 registers each): they meet at no common barrier, so one's vector work
+// (exp, rounding) runs beside the other's matrix work.  Stages pass through a
+// two-stage LDS ring filled by direct global -> LDS loads issued one stage
+// ahead, one barrier per stage.  Against one 8-wave workgroup per CU whose
+// waves all ran the same phase between two barriers, with separate row and
+// transposed images of each operand, the kernel takes 1056 -> 862 us at
+// 1x30x4416x128 and 1808 -> 1127 us on the packed 1x30x6912 batch with document
+// ids, and the preparation 51 -> 23 us.  What bounds it now is the power limit:
+// 27.4 M MFMAs of random data run at 18.2 ns each per SIMD alone (1.79 GHz,
+// 489 us), 20.4 ns beside six vector instructions each (546 us).
+// Work items are dealt to XCDs in contiguous ranges.  One launch (bwd_kernel)
+// runs the dK/dV items, then the dQ items.
 //
-// dQ pass: a workgroup is the forward's 128-query tile; wave w takes queries
-// 32 (w % 4) and key half w / 4 of every 64-key tile.  Per wave and tile, in
-// the S^T layout (lane (h, r) = query r, keys 8J + 4h + i):
+// dQ pass: a workgroup is the forward's 128-query tile, 32 queries per wave;
+// keys stream in steps of 32.  Per wave and step, in the S^T layout (lane
+// (h, r) = query r, keys 8J + 4h + i):
 //   S^T = K . Q^T (int8 / fp8 MFMA, the forward's operands),
-//   dP^T = V . dO^T (bf16 MFMA; V from the stage, the wave's dO rows in registers),
-//   dS^T = P^T (dP^T - D), dQ += dS . K~ (A = dS from the registers, B = T image of K~);
-// the two key halves' dQ are added, then dQ * sm_scale is rounded to bf16
-// (sage_kernels.py:1720).
-// dK/dV pass: a workgroup owns 128 keys; wave w takes keys 32 (w % 4) and
-// query half w / 4 of every 64-query step.  Per wave and step, in the S
-// layout (lane (h, r) = key r, queries 8J + 4h + i):
-//   S = Q . K^T and dP = dO . V^T (the wave's K codes in registers, the
-//   workgroup's V rows in LDS for the whole launch),
-//   dS = P (dP - D), dV^T += dO^T . bf16(P), dK^T += Q^T . bf16(dS * sm_scale)
-// (A = the T images of dO and Q, B = P and dS from the registers); the two
-// query halves' dK and dV are added at the end.
-// Both kernels skip (query tile, key tile) pairs the reference tile mask turns
-// off; with document ids they skip pairs whose summaries show no visible pair
-// and give hidden pairs p = 0.
+//   dP^T - D = V . dO^T - D (bf16 MFMA started from -D; the wave's dO rows in registers),
+//   dS^T = P^T (dP^T - D), dQ += dS . K~ (A = dS from the registers, B = K~ transposed);
+// dQ * sm_scale is rounded to bf16 at the end (sage_kernels.py:1720).
+// dK/dV pass: a workgroup owns 128 keys, 32 per wave; queries stream in steps
+// of 32.  Per wave and step, in the S layout (lane (h, r) = key r, queries
+// 8J + 4h + i):
+//   S = Q . K^T and dP - D = dO . V^T - D (the wave's K codes and V rows in
+//   registers),
+//   dS = P (dP - D), dV^T += dO^T . bf16(P), dK^T += Q^T . bf16(dS);
+// dK * sm_scale is rounded to bf16 at the end (the reference scales dS before
+// its bf16 rounding, :1595: the same relative rounding of the same value).
+//
+// Both passes skip (query tile, key tile) pairs the reference tile mask turns
+// off; with document ids they skip pairs whose summaries show no visible pair,
+// and only pairs whose summaries are mixed test every element.  The steps'
+// activity is read 64 steps at a time (a lane per step, ballots), so a skipped
+// step costs nothing.
 #include <type_traits>
 
 #include "sage_common.h"
@@ -61,10 +73,10 @@ __device__ __forceinline__ uint32_t word_at(const uint4& w, int i) {
   return i == 0 ? w.x : i == 1 ? w.y : i == 2 ? w.z : w.w;
 }
 
-__device__ __forceinline__ uint4 zero_if(bool z, uint4 w) { return z ? make_uint4(0, 0, 0, 0) : w; }
-
 // 16-byte unit as a native vector: its copies are plain loads and stores.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
 
 template <int QK>
 struct BAcc {
@@ -99,85 +111,108 @@ __device__ __forceinline__ typename BAcc<QK>::type score_block(const i32x4* a, c
 
 __device__ __forceinline__ bool doc_visible(int dq, int dk) { return dk >= 0 && (dq == dk || dq < 0); }
 
+// Waves of a backward workgroup; two workgroups share a CU.
+constexpr int kBwdWaves = 4;
+constexpr int kBwdThreads = 64 * kBwdWaves;
+
+// bf16 rows of D channels in LDS: 1 KiB blocks of RPB rows, `stride` bytes
+// apart, each one direct global -> LDS load of a wave (64 chunks of 16 bytes)
+// that reads 1 KiB of consecutive rows.  Inside a block the rows' 64-byte
+// runs are ordered (run, row): four lanes of the load read one run, which
+// costs the vector cache a quarter of the accesses that single chunks of four
+// rows do (measured: 3.2e8 -> 1.4e8 accesses per launch).  The 16 bytes
+// between blocks put rows t and t + RPB in neighbouring chunk columns; with 8
+// rows a block (D = 64) rows 4..7 also swap their runs' halves: the 16 lanes
+// of a row read and the 32 of a transposed read then touch 256 different
+// bytes modulo the banks.
+template <int D>
+struct Rows {
+  static constexpr int RPB = 512 / D;
+  static constexpr int stride = 1024 + 16;
+  static constexpr int blocks32 = 32 / RPB;
+  static constexpr int bytes32 = blocks32 * stride;  // a 32-row block
+
+  static __device__ __forceinline__ int swap(int row_in_block) { return (row_in_block >> 2) * 2; }
+  // byte offset in its source block of the chunk that lane `lane` of the load moves
+  static __device__ __forceinline__ int src_off(int lane) {
+    const int t = (lane >> 2) % RPB, run = (lane >> 2) / RPB;
+    return t * (2 * D) + run * 64 + ((lane & 3) ^ swap(t)) * 16;
+  }
+  // row operand: lane (h, r) reads row r, channels [16 c2 + 8h, +8) at
+  // row_off(lane, c2 % 2) + row_imm(c2)
+  static __device__ __forceinline__ int row_off(int lane, int odd) {
+    const int h = lane >> 5, r = lane & 31, t = r % RPB;
+    return (r / RPB) * stride + t * 64 + ((2 * odd + h) ^ swap(t)) * 16;
+  }
+  static constexpr int row_imm(int c2) { return c2 / 2 * RPB * 64; }
+  // transposed operand: lane (hh, r) gets channel 32c + r of rows 16tt + 8jj +
+  // 4hh + 0..3; lane l of a group of 16 reads channels 4 (l % 4) .. +3 (of the
+  // group's 16) of row l / 4
+  static __device__ __forceinline__ int tr_off(int lane) {
+    const int l = lane & 15, g = (lane >> 4) & 1, hh = lane >> 5, t = 4 * hh % RPB + (l >> 2);
+    return (4 * hh / RPB) * stride + t * 64 + ((2 * g + ((l & 3) >> 1)) ^ swap(t)) * 16 + (l & 1) * 8;
+  }
+  static constexpr int tr_imm(int c, int tt, int jj) { return (16 * tt + 8 * jj) / RPB * stride + c * RPB * 64; }
+};
+
+// One direct global -> LDS load of 64 chunks: lane l's 16 bytes land at lds + 16 l.
+__device__ __forceinline__ void dma_16(uint8_t* lds, __amdgpu_buffer_rsrc_t rs, int off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, lds, 16, off, 0, 0, 0);
+}
+
+// Rows [0, 32) of `rows` (row-major, contiguous; rows past `left` read as
+// zeros) into the LDS block at `lds`, by waves `wave`, wave + WAVES, ...  The
+// whole offset sits in the range-checked vector operand.
+template <int D, int WAVES>
+__device__ __forceinline__ void dma_rows32(uint8_t* lds, int wave, int src_off, const uint16_t* rows, int64_t left) {
+  using R = Rows<D>;
+  const int valid = (int)(left < 0 ? 0 : left > 32 ? 32 : left);
+  const __amdgpu_buffer_rsrc_t rs = raw_rsrc(rows, (uint32_t)(valid * D * 2));
+#pragma unroll
+  for (int j0 = 0; j0 < R::blocks32; j0 += WAVES) {
+    const int j = j0 + wave;
+    if (R::blocks32 % WAVES == 0 || j < R::blocks32)
+      dma_16(lds + j * R::stride, rs, src_off + j * 1024);
+  }
+}
+
+// 32 consecutive 4-byte values into LDS by one wave: 16-byte aligned ones by
+// its first 8 lanes, others (rows past `left` read as zeros) by 32 lanes.
+__device__ __forceinline__ void dma_words32(uint8_t* lds, int lane, const void* src) {
+  const __amdgpu_buffer_rsrc_t rs = raw_rsrc(src, 128);
+  if (lane < 8) dma_16(lds, rs, lane * 16);
+}
+__device__ __forceinline__ void dma_words32_unaligned(uint8_t* lds, int lane, const void* src, int64_t left) {
+  const int valid = (int)(left < 0 ? 0 : left > 32 ? 32 : left);
+  const __amdgpu_buffer_rsrc_t rs = raw_rsrc(src, (uint32_t)(valid * 4));
+  if (lane < 32) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, lds, 4, lane * 4, 0, 0, 0);
+}
+
+// The operand of v_mfma_f32_32x32x16_bf16 that contracts 16 rows (tt): two
+// transposed reads of 4 rows each per lane.  `base` is restrict so that the
+// reads carry alias information, like plain LDS loads (type-based there):
+// without any, the compiler waits for every direct global -> LDS load in
+// flight, the next stage's, before each of them.
+template <int D>
+__device__ __forceinline__ bf16x8 tr_frag(const uint8_t* __restrict__ base, int c, int tt) {
+  typedef __attribute__((address_space(3))) s16x4* LdsPtr;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(base + Rows<D>::tr_imm(c, tt, 0)));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(base + Rows<D>::tr_imm(c, tt, 1)));
+  return __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+}
+
+// Activity of up to 64 steps: bit i of each mask is step base + i.
+struct StepMasks {
+  uint64_t wg;    // some wave of the workgroup has work
+  uint64_t on;    // this wave has work
+  uint64_t mixed; // this wave tests every element
+};
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
 // Preparation
 // ---------------------------------------------------------------------------
-
-// T image of 64-token block bx of head bh of job z (of up to two bf16
-// [BH, N, D] tensors), rows past N zero.  With mu set, the rows are
-// bf16(x - mu) (the quantization's smoothed K, sage_attention.py:63-71).
-// img: 2 * 64 * D bytes of LDS.
-template <int D>
-__device__ __forceinline__ void timage_block(const TImageJobs& jobs, int z, int bh, int64_t bx, int64_t n, int64_t np,
-                                             uint8_t* img) {
-  constexpr int LPR = D / 8;
-  constexpr int VTHREADS = 16 * LPR;  // 16 groups of 4 tokens
-  const int tid = threadIdx.x;
-  const int64_t tok0 = bx * 64;
-  const uint16_t* x = jobs.x[z] + (int64_t)bh * n * D;
-  const uint16_t* mu = jobs.mu[z];
-  if (tid < VTHREADS) {
-    const int g = tid / LPR, c8 = tid % LPR;
-    uint4 w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t tok = tok0 + 4 * g + i;
-      w[i] = zero_if(tok >= n, *reinterpret_cast<const uint4*>(x + min(tok, n - 1) * D + c8 * 8));
-    }
-    float m8[8];
-    if (mu) {
-      const uint4 mw = *reinterpret_cast<const uint4*>(mu + (int64_t)bh * D + c8 * 8);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) m8[e] = bf16_to_f32((uint16_t)(word_at(mw, e >> 1) >> ((e & 1) * 16)));
-    }
-    const int b = g >> 3, tt = (g >> 2) & 1, jj = (g >> 1) & 1, hh = g & 1;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int d = c8 * 8 + e, j = d >> 5, r = d & 31;
-      uint32_t t4[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t u = (word_at(w[i], e >> 1) >> ((e & 1) * 16)) & 0xffffu;
-        if (mu && tok0 + 4 * g + i < n) u = f32_to_bf16_rne(bf16_to_f32((uint16_t)u) - m8[e]);
-        t4[i] = u;
-      }
-      uint2 pk;
-      pk.x = t4[0] | (t4[1] << 16);
-      pk.y = t4[2] | (t4[3] << 16);
-      *reinterpret_cast<uint2*>(img + (((((j * 2 + b) * 2 + tt) * 64 + 32 * hh + r) * 8) + 4 * jj) * 2) = pk;
-    }
-  }
-  __syncthreads();
-  uint4* o = reinterpret_cast<uint4*>(jobs.out[z] + ((int64_t)bh * np + tok0) * D);
-#pragma unroll
-  for (int i = tid; i < 64 * D * 2 / 16; i += 256) o[i] = reinterpret_cast<const uint4*>(img)[i];
-}
-
-// R images of up to two bf16 [BH, N, D] tensors (grid.z selects the job): per
-// 32-token block rb, 16-channel group c2 and lane L = 32h + r, the 16 bytes
-// X[32 rb + r][16 c2 + 8h, +8) at chunk (rb * D/16 + c2) * 64 + L, rows past N
-// zero.  It is the row operand of v_mfma_f32_32x32x16_bf16 contracting the
-// channels (lane (h, r) = row r, channels 8h.. of the 16-channel step), so a
-// stage is a contiguous copy and a fragment read is one 16-byte load per lane.
-// One 64-token block (bx) of head bh of job z, one thread per chunk.
-template <int D>
-__device__ __forceinline__ void rimage_block(const TImageJobs& jobs, int z, int bh, int64_t bx, int64_t n,
-                                             int64_t np) {
-  constexpr int G = D / 16;           // 16-channel groups
-  constexpr int kChunks = 64 * D / 8;  // 16-byte chunks of a 64-token block
-  const int64_t tok0 = bx * 64;
-  const uint16_t* x = jobs.x[z] + (int64_t)bh * n * D;
-  uint4* o = reinterpret_cast<uint4*>(jobs.out[z] + ((int64_t)bh * np + tok0) * D);
-#pragma unroll
-  for (int c = threadIdx.x; c < kChunks; c += 256) {
-    const int lane = c & 63, g = (c >> 6) % G, rb = (c >> 6) / G;
-    const int64_t row = tok0 + 32 * rb + (lane & 31);
-    const uint4 w = *reinterpret_cast<const uint4*>(x + min(row, n - 1) * D + 16 * g + 8 * (lane >> 5));
-    o[c] = zero_if(row >= n, w);
-  }
-}
 
 // Item of workgroup b of a 1D grid of `total` items: the hardware hands
 // workgroup b to XCD b % 8, and each XCD has its own L2, so every XCD takes a
@@ -189,13 +224,16 @@ __device__ __forceinline__ int xcd_item(int b, int total) {
   return x * per + min(x, rem) + local;
 }
 
-// D = rowsum(dO * O) per token in fp32 (sage_kernels.py:321-349), zero past N.
-// Lane (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps; the products
-// are fp32, summed per lane then over the token's lanes.  One 64-token
-// block (bx) of head bh.
+// -D = -rowsum(dO * O) per token in fp32 (sage_kernels.py:321-349), zero past
+// N, and the LSE with +inf for rows without a gradient (past N, or no visible
+// key in the forward): 2^(s - inf) = 0 needs no per-element test.  Lane
+// (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps; the products are
+// fp32, summed per lane then over the token's lanes.  One 64-token block (bx)
+// of head bh.
 template <int D>
 __device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, const uint16_t* __restrict__ out,
-                                            int bh, int64_t bx, int64_t n, int64_t np, float* __restrict__ delta) {
+                                            const float* __restrict__ lse, int bh, int64_t bx, int64_t n, int64_t np,
+                                            float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
   constexpr int LPR = D / 8, RPP = 256 / LPR, PASSES = 64 / RPP;
   const int tid = threadIdx.x, c8 = tid % LPR, rr = tid / LPR;
   const int64_t tok0 = bx * 64;
@@ -213,7 +251,40 @@ __device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, c
     }
 #pragma unroll
     for (int off = 1; off < LPR; off <<= 1) s += __shfl_xor(s, off);
-    if (c8 == 0) delta[(int64_t)bh * np + t] = t < n ? s : 0.0f;
+    if (c8 == 0) {
+      const float l = lse[(int64_t)bh * n + min(t, n - 1)];
+      neg_delta[(int64_t)bh * np + t] = t < n ? -s : 0.0f;
+      lse_pad[(int64_t)bh * np + t] = t < n && l > -INFINITY ? l : INFINITY;
+    }
+  }
+}
+
+// K~ = bf16(k - mean) of one 64-token block (the quantization's smoothed K,
+// sage_attention.py:63-71), one thread per 16-byte chunk.
+template <int D>
+__device__ __forceinline__ void smooth_block(const uint16_t* __restrict__ k, const uint16_t* __restrict__ mu, int bh,
+                                             int64_t bx, int64_t n, uint16_t* __restrict__ kt) {
+  constexpr int CPR = D / 8;
+  const int64_t rows = min((int64_t)64, n - bx * 64);
+  const int64_t at = ((int64_t)bh * n + bx * 64) * D;
+  const uint4* src = reinterpret_cast<const uint4*>(k + at);
+  uint4* dst = reinterpret_cast<uint4*>(kt + at);
+  const uint4 m = reinterpret_cast<const uint4*>(mu + (int64_t)bh * D)[threadIdx.x % CPR];
+#pragma unroll
+  for (int c0 = 0; c0 < 64 * CPR; c0 += 256) {
+    const int c = c0 + (int)threadIdx.x;
+    if (c < rows * CPR) {
+      const uint4 x = src[c];
+      uint32_t o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t w = word_at(x, i), mw = word_at(m, i);
+        const uint16_t lo = f32_to_bf16_rne(bf16_to_f32((uint16_t)w) - bf16_to_f32((uint16_t)mw));
+        const uint16_t hi = f32_to_bf16_rne(bf16_to_f32((uint16_t)(w >> 16)) - bf16_to_f32((uint16_t)(mw >> 16)));
+        o[i] = lo | ((uint32_t)hi << 16);
+      }
+      dst[c] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
   }
 }
 
@@ -221,55 +292,39 @@ __device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, c
 // dQ
 // ---------------------------------------------------------------------------
 
-// LDS stage of one 64-key tile: K codes (row fragments, as stored), the R
-// image of V, the T image of K~, per-key K scales, per-key document ids.
+// LDS stage of one 32-key step: K codes (row fragments, as stored), V rows,
+// K~ rows, per-key K scales, per-key document ids.
 template <int D>
 struct DqStage {
-  static constexpr int kcBytes = 64 * D;
-  static constexpr int rowBytes = 64 * 2 * D;
-  static constexpr int offV = kcBytes;
-  static constexpr int offT = offV + rowBytes;
-  static constexpr int offKd = offT + rowBytes;
-  static constexpr int offDoc = offKd + 256;
-  static constexpr int bytes = offDoc + 256;
-  static constexpr int cKc = kcBytes / 16, cRow = rowBytes / 16;  // 16-byte chunks
+  static constexpr int offV = 32 * D;
+  static constexpr int offT = offV + Rows<D>::bytes32;
+  static constexpr int offKd = offT + Rows<D>::bytes32;
+  static constexpr int offDoc = offKd + 128;
+  static constexpr int bytes = offDoc + 128;
 };
 
-// Threads of the backward workgroups: 8 waves, two per SIMD, so one wave's
-// vector work overlaps the other's matrix and LDS work.
-constexpr int kBwdThreads = 512;
-
-// Direct global -> LDS copies by the 8 waves of a backward workgroup.
-template <int C, typename Src>
-__device__ __forceinline__ void dma_chunks(uint8_t* lds, int wave, int lane, Src src) {
-  sage::dma_chunks<C, kBwdThreads / 64>(lds, wave, lane, src);
-}
-
-// dQ of item (bh, 128-query tile), in `smem` (2 * DqStage<D>::bytes).  Wave
-// w covers queries 32 * (w % 4) of the tile and key half w / 4 of every
-// 64-key tile; the two key halves' partial dQ are summed (half 0 + half 1) at
-// the end.
-// Key tiles [t_begin, t_end) of the item; with cut >= 0 the item is cut item
-// `cut` (AttnParams-style in-kernel merge): the half's fp32 dQ goes to its
-// slot, and the last half to arrive sums both slots (first half + second
-// half) and stores dQ.
+// dQ of item (bh, 128-query tile), in `smem` (2 * DqStage<D>::bytes), over
+// 32-key steps [s_begin, s_end).  With cut >= 0 the item is cut item `cut`
+// (an in-kernel merge as the forward's split items): the half's fp32 dQ goes
+// to its slot, and the last half to arrive sums both slots (first half +
+// second half) and stores dQ.
 template <int D, int QK, int MASK>
-__device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int item, int t_begin, int t_end,
-                                        int cut, int half) {
+__device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int item, int s_begin, int s_end, int cut,
+                                        int half) {
   using St = DqStage<D>;
+  using R = Rows<D>;
   using SAcc = typename BAcc<QK>::type;
   constexpr int NC = D / 32, CPR = D / 8;
-  static_assert(4 * NC * 16 * 64 * 4 <= 2 * St::bytes, "partial dQ exchange must fit in the ring");
+  static_assert(kRowsPerWG * D * 2 <= 2 * St::bytes, "the output staging must fit in the ring");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
   const int h = lane >> 5, r = lane & 31;
-  const int qg = wave & 3, b = wave >> 2;  // query group, key half
   const int nq = (int)(p.np / kRowsPerWG);
   const int bh = item / nq, qt = item % nq;
   const int bidx = bh / p.h;
   const int64_t n = p.n, np = p.np;
   const int nt = (int)((n + 63) / 64);
-  const int64_t q0 = (int64_t)qt * kRowsPerWG + 32 * qg;
+  const int64_t q0 = (int64_t)qt * kRowsPerWG + 32 * wave;
   const bool wave_live = q0 < n;
   const int64_t qrow = q0 + r;
 
@@ -287,220 +342,192 @@ __device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int i
     for (int c2 = 0; c2 < 2 * NC; ++c2) dof[c2] = *reinterpret_cast<const bf16x8*>(dr + 16 * c2);
   }
   const float qd = p.qs[(int64_t)bh * np + qrow];
-  // +inf for rows with no gradient (past N, or no visible key in the forward):
-  // 2^(s - inf) = 0 needs no per-element test
-  const float lse_r = qrow < n ? p.lse[(int64_t)bh * n + qrow] : -INFINITY;
-  const float lse_b = lse_r > -INFINITY ? lse_r : INFINITY;
-  const float dl = p.delta[(int64_t)bh * np + qrow];
+  const float lse_b = p.lse_pad[(int64_t)bh * np + qrow];
+  f32x16 nd;  // -D of the lane's query, the start of the dP sums
+  {
+    const float d = p.neg_delta[(int64_t)bh * np + qrow];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) nd[e] = d;
+  }
   const int dq_doc = (MASK & 2) ? (qrow < n ? p.doc[(int64_t)bidx * n + qrow] : -1) : 0;
   f32x16 acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = f32x16{0};
 
-  // document-id summaries: the workgroup's 128 queries and this wave's 32
+  // ---- active steps: tile t = s / 2 against the workgroup's 128 queries and this wave's 32 ----
   int4 qsum128 = make_int4(0, 0, 0, 0), qsum32 = make_int4(0, 0, 0, 0);
   if constexpr (MASK & 2) {
-    qsum128 = p.q_sum128[(int64_t)bidx * nq + qt];
-    qsum32 = p.q_sum[(int64_t)bidx * (np / 32) + (q0 >> 5)];
+    qsum128 = load_uniform(p.q_sum128, (int64_t)bidx * nq + qt);
+    qsum32 = load_uniform(p.q_sum, (int64_t)bidx * (np / 32) + (q0 >> 5));
   }
-  auto active = [&](int t) __attribute__((always_inline)) -> bool {
-    bool on = true;
-    if constexpr (MASK & 1)
-      on = load_uniform_u8(p.tile_mask, (int64_t)bh * p.mask_stride_z + (int64_t)qt * p.mask_nkv + t) != 0;
-    if constexpr (MASK & 2) on = on && classify(qsum128, load_uniform(p.kv_sum, (int64_t)bidx * nt + t)) != 0;
-    return on;
-  };
-  auto next_active = [&](int t) __attribute__((always_inline)) -> int {
-    while (t < t_end && !active(t)) ++t;
-    return t;
-  };
-
-  // ---- staging: bulk by direct global -> LDS loads, scales / ids through registers ----
-  u32x4 psm = u32x4{0, 0, 0, 0};
-  auto load_tile = [&](int t, int stage) __attribute__((always_inline)) {
-    const int64_t key0 = (int64_t)t * 64;
-    uint8_t* sb = smem + stage * St::bytes;
-    const uint8_t* kcs = p.kc + ((int64_t)bh * np + key0) * D;
-    const uint8_t* tks = reinterpret_cast<const uint8_t*>(p.tk + ((int64_t)bh * np + key0) * D);
-    const uint8_t* rvs = reinterpret_cast<const uint8_t*>(p.rv + ((int64_t)bh * np + key0) * D);
-    if (tid < 32) {
-      // one path for lanes 0..31 (see the dK/dV kernel): K scales (g=0),
-      // key document ids (g=1, -1 past N)
-      const int g = tid >> 4;
-      const int64_t k = key0 + 4 * (tid & 15);
-      const uint32_t* base = g == 0 ? reinterpret_cast<const uint32_t*>(p.ks + (int64_t)bh * np)
-                             : (MASK & 2) ? reinterpret_cast<const uint32_t*>(p.doc + (int64_t)bidx * n)
-                                          : reinterpret_cast<const uint32_t*>(p.ks);  // not read
-      const int64_t lim = g == 0 ? np : (MASK & 2) ? n : 0;
-      const uint32_t dflt = g == 1 ? 0xffffffffu : 0u;
-      u32x4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = k + i < lim ? base[k + i] : dflt;
-      psm = v;
+  StepMasks sm{0, 0, 0};
+  int sm_base = -1;
+  auto find = [&](int s) __attribute__((always_inline)) -> int {
+    if constexpr (MASK == 0) return s;
+    while (s < s_end) {
+      if ((s & ~63) != sm_base) {
+        sm_base = s & ~63;
+        const int t = (sm_base + lane) >> 1;
+        bool wg = sm_base + lane < s_end, on = wg, mixed = false;
+        if constexpr (MASK & 1)
+          wg = wg && p.tile_mask[(int64_t)bh * p.mask_stride_z + (int64_t)qt * p.mask_nkv + min(t, nt - 1)] != 0;
+        on = wg;
+        if constexpr (MASK & 2) {
+          const int4 ks = p.kv_sum[(int64_t)bidx * nt + min(t, nt - 1)];
+          const int c = classify(qsum32, ks);
+          on = wg && c != 0;
+          mixed = c == 2;
+          wg = wg && classify(qsum128, ks) != 0;
+        }
+        sm.wg = __ballot(wg);
+        sm.on = __ballot(on);
+        sm.mixed = __ballot(mixed);
+      }
+      const uint64_t m = sm.wg >> (s & 63);
+      if (m) return s + __builtin_ctzll(m);
+      s = sm_base + 64;
     }
-    // the stage loads after the small ones (see the dK/dV kernel)
-    dma_chunks<St::cKc>(sb, wave, lane, [&](int x) { return kcs + (uint32_t)(x * 16); });
-    dma_chunks<St::cRow>(sb + St::offT, wave, lane, [&](int x) { return tks + (uint32_t)(x * 16); });
-    dma_chunks<St::cRow>(sb + St::offV, wave, lane, [&](int x) { return rvs + (uint32_t)(x * 16); });
-  };
-  auto store_small = [&](int stage) __attribute__((always_inline)) {
-    uint8_t* sb = smem + stage * St::bytes;
-    if (tid < 16)
-      reinterpret_cast<u32x4*>(sb + St::offKd)[tid] = psm;
-    else if ((MASK & 2) && tid < 32)
-      reinterpret_cast<u32x4*>(sb + St::offDoc)[tid - 16] = psm;
+    return s_end;
   };
 
-  int t = next_active(t_begin);
-  if (t < t_end) {
-    load_tile(t, 0);
-    store_small(0);
-  }
-  wait_vmem();
-  __syncthreads();
+  // ---- staging -------------------------------------------------------------------
+  const int src_off = R::src_off(lane);
+  auto load_step = [&](int s, int stage) __attribute__((always_inline)) {
+    const int64_t key0 = (int64_t)s * 32;
+    uint8_t* sb = smem + stage * St::bytes;
+    dma_chunks_buf<2 * D, kBwdWaves>(sb, wave, lane, raw_rsrc(p.kc + ((int64_t)bh * np + key0) * D, 32 * D), 0);
+    dma_rows32<D, kBwdWaves>(sb + St::offV, wave, src_off, p.v + ((int64_t)bh * n + key0) * D, n - key0);
+    dma_rows32<D, kBwdWaves>(sb + St::offT, wave, src_off, p.kt + ((int64_t)bh * n + key0) * D, n - key0);
+    if (wave == 2) dma_words32(sb + St::offKd, lane, p.ks + (int64_t)bh * np + key0);
+    if constexpr (MASK & 2) {
+      if (wave == 3) dma_words32_unaligned(sb + St::offDoc, lane, p.doc + (int64_t)bidx * n + key0, n - key0);
+    }
+  };
+  const int row_off[2] = {R::row_off(lane, 0), R::row_off(lane, 1)}, tr_off = R::tr_off(lane);
+
+  int s = find(s_begin);
+  if (s < s_end) load_step(s, 0);
   int stage = 0;
-  while (t < t_end) {
-    const int tn = next_active(t + 1);
-    if (tn < t_end) load_tile(tn, stage ^ 1);
-    bool wave_on = wave_live;
-    if constexpr (MASK & 2)
-      wave_on = wave_on && classify(qsum32, load_uniform(p.kv_sum, (int64_t)bidx * nt + t)) != 0;
-    if (wave_on) {
+  while (s < s_end) {
+    const bool on = wave_live && (MASK == 0 || ((sm.on >> (s & 63)) & 1));
+    const bool mixed = (MASK & 2) && ((sm.mixed >> (s & 63)) & 1);
+    const int sn = find(s + 1);
+    wait_vmem();
+    __syncthreads();  // stage complete; every wave is past the step that used the other stage
+    if (sn < s_end) load_step(sn, stage ^ 1);
+    if (on) {
       const uint8_t* sb = smem + stage * St::bytes;
-      // S^T = K . Q^T for keys 32b + (lane-local rows) x this wave's queries
+      // S^T = K . Q^T for keys (lane-local rows) x this wave's queries
       i32x4 ka[NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) ka[c] = reinterpret_cast<const i32x4*>(sb)[(b * NC + c) * 64 + lane];
-      const SAcc s = score_block<D, QK>(ka, qf);
-      // dP^T = V . dO^T
-      f32x16 dp = f32x16{0};
-      const u32x4* vl = reinterpret_cast<const u32x4*>(sb + St::offV);
-      u32x4 vf[2 * NC];  // V[key 32b + r][16c2 + 8h, +8), read two MFMAs ahead
-      vf[0] = vl[(b * 2 * NC + 0) * 64 + lane];
-      vf[1] = vl[(b * 2 * NC + 1) * 64 + lane];
+      for (int c = 0; c < NC; ++c) ka[c] = reinterpret_cast<const i32x4*>(sb)[c * 64 + lane];
+      const SAcc sc = score_block<D, QK>(ka, qf);
+      // dP^T - D = V . dO^T - D, its MFMAs issued under the exponentials of P
+      f32x16 dp = nd;
+      const f32x4* kdl = reinterpret_cast<const f32x4*>(sb + St::offKd);
+      const int4* dkl = reinterpret_cast<const int4*>(sb + St::offDoc);
+      const int kmax = (int)min((int64_t)32, n - (int64_t)s * 32);  // valid keys of this step
+      const uint8_t* vl = sb + St::offV;
+      bf16x8 vf[2 * NC];
+      vf[0] = *reinterpret_cast<const bf16x8*>(vl + row_off[0]);
+      vf[1] = *reinterpret_cast<const bf16x8*>(vl + row_off[1]);
+      f32x4 kd4[4];
+#pragma unroll
+      for (int J = 0; J < 4; ++J) kd4[J] = kdl[2 * J + h];
+      float pr[16];
+      // s - lse = acc * (qd * kd) - lse
+      constexpr int kPer = 16 / (2 * NC);  // scores per MFMA
 #pragma unroll
       for (int c2 = 0; c2 < 2 * NC; ++c2) {
         __builtin_amdgcn_sched_barrier(0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[c2]), dof[c2], dp, 0, 0, 0);
-        if (c2 + 2 < 2 * NC) vf[c2 + 2] = vl[(b * 2 * NC + c2 + 2) * 64 + lane];
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c2], dof[c2], dp, 0, 0, 0);
+        if (c2 + 2 < 2 * NC) vf[c2 + 2] = *reinterpret_cast<const bf16x8*>(vl + row_off[c2 & 1] + R::row_imm(c2 + 2));
+#pragma unroll
+        for (int e = kPer * c2; e < kPer * c2 + kPer; ++e)
+          pr[e] = __builtin_amdgcn_exp2f(fmaf((float)sc[e], qd * kd4[e >> 2][e & 3], -lse_b));
       }
-      // P^T, dS^T (bf16, packed as the A operand of dS . K~)
-      const f32x4* kdl = reinterpret_cast<const f32x4*>(sb + St::offKd);
-      const int4* dkl = reinterpret_cast<const int4*>(sb + St::offDoc);
-      const int kmax = (int)min((int64_t)64, n - (int64_t)t * 64);  // valid keys of this tile
-      // the K~ operands of dQ += dS . K~, read before the P / dS vector work
-      // so their LDS latency hides under it
-      const bf16x8* tkl = reinterpret_cast<const bf16x8*>(sb + St::offT);
-      bf16x8 tkf[NC][2];
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) tkf[c][tt] = tkl[((c * 2 + b) * 2 + tt) * 64 + lane];
-      bf16x8 dsa[2];
-      // s - lse = acc * (qd * kd) - lse; keys past N (the last tile only) are
-      // hidden by a test taken on that tile alone
-      auto scores = [&](auto ragged) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      // keys past N (the last step only) and, in mixed pairs, hidden keys: p = 0
+      if (kmax < 32 || mixed) {
 #pragma unroll
         for (int J = 0; J < 4; ++J) {
-          const f32x4 kd4 = kdl[8 * b + 2 * J + h];
           int4 dk4 = make_int4(0, 0, 0, 0);
-          if constexpr (MASK & 2) dk4 = dkl[8 * b + 2 * J + h];
+          if constexpr (MASK & 2) dk4 = dkl[2 * J + h];
           const int dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int e = 4 * J + i;
-            float pr = __builtin_amdgcn_exp2f(fmaf((float)s[e], qd * kd4[i], -lse_b));
-            if constexpr (decltype(ragged)::value) pr = 32 * b + 8 * J + 4 * h + i < kmax ? pr : 0.0f;
-            if constexpr (MASK & 2) pr = doc_visible(dq_doc, dk[i]) ? pr : 0.0f;
-            dsa[e >> 3][e & 7] = (__bf16)(pr * (dp[e] - dl));
+            bool vis = 8 * J + 4 * h + i < kmax;
+            if constexpr (MASK & 2) vis = vis && doc_visible(dq_doc, dk[i]);
+            pr[4 * J + i] = vis ? pr[4 * J + i] : 0.0f;
           }
         }
-      };
-      if (kmax < 64)
-        scores(std::true_type{});
-      else
-        scores(std::false_type{});
-      // dQ += dS . K~ over this key half
+      }
+      // dQ += dS . K~ (A = dS, rounded to bf16), the first 16 keys' products under the others' rounding
+      const uint8_t* tl = sb + St::offT + tr_off;
+      bf16x8 dsa[2];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dsa[0][e] = (__bf16)(pr[e] * dp[e]);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[0], tr_frag<D>(tl, c, 0), acc[c], 0, 0, 0);
+#pragma unroll
+        for (int e = 8 / NC * c; e < 8 / NC * (c + 1); ++e) dsa[1][e] = (__bf16)(pr[8 + e] * dp[8 + e]);
+      }
 #pragma unroll
       for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-          acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[tt], tkf[c][tt], acc[c], 0, 0, 0);
+        acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsa[1], tr_frag<D>(tl, c, 1), acc[c], 0, 0, 0);
     }
-    if (tn < t_end) store_small(stage ^ 1);
-    wait_vmem();
-    __syncthreads();
     stage ^= 1;
-    t = tn;
+    s = sn;
   }
+  wait_vmem();
+  __syncthreads();  // the ring is free
 
-  // ---- epilogue: dQ = (half 0 + half 1) * sm_scale -> bf16 ---------------------------
+  // ---- epilogue: dQ * sm_scale -> bf16 ------------------------------------------------
   // acc lane (h, r) holds channel 32c + r of rows 8J + 4h + i (element 4J + i)
-  float* xch = reinterpret_cast<float*>(smem) + qg * NC * 16 * 64;
-  if (b == 1) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) xch[(c * 16 + e) * 64 + lane] = acc[c][e];
-  }
-  __syncthreads();
-  if (b == 0) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[c][e] += xch[(c * 16 + e) * 64 + lane];
-  }
-  __syncthreads();
   if (cut >= 0) {
     // a half of a cut item: its dQ through to the coherence point, complete
     // before it counts; the last half sums the two slots in key order
     constexpr int kSlot = 4 * NC * 16 * 64;
     uint32_t* slots = reinterpret_cast<uint32_t*>(p.dq_part + (int64_t)cut * 2 * kSlot);
-    if (b == 0) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int e = 0; e < 16; ++e)
-          __hip_atomic_store(slots + half * kSlot + ((qg * NC + c) * 16 + e) * 64 + lane, __float_as_uint(acc[c][e]),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+      for (int e = 0; e < 16; ++e)
+        __hip_atomic_store(slots + half * kSlot + ((wave * NC + c) * 16 + e) * 64 + lane, __float_as_uint(acc[c][e]),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     wait_vmem();
     __syncthreads();
     int* last = reinterpret_cast<int*>(smem);
     if (tid == 0) *last = arrive_last(p.dq_ctr + cut, p.dq_tag, 2) ? 1 : 0;
     __syncthreads();
     if (*last == 0) return;
-    if (b == 0) {
-      auto ld = [](const uint32_t* a) __attribute__((always_inline)) {
-        return __uint_as_float(__hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      };
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int at = ((qg * NC + c) * 16 + e) * 64 + lane;
-          acc[c][e] = ld(slots + at) + ld(slots + kSlot + at);
-        }
-    }
-    if (tid == 0)
-      __hip_atomic_store(p.dq_ctr + cut, p.dq_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();  // every wave has read `last` before the staging below reuses the LDS
-  }
-  uint16_t* stg = reinterpret_cast<uint16_t*>(smem) + qg * 32 * D;
-  if (b == 0) {
+    auto ld = [](const uint32_t* a) __attribute__((always_inline)) {
+      return __uint_as_float(__hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int row = 8 * (e >> 2) + 4 * h + (e & 3);
-        stg[row * D + 32 * c + r] = f32_to_bf16_rne(acc[c][e] * p.sm_scale);
+        const int at = ((wave * NC + c) * 16 + e) * 64 + lane;
+        acc[c][e] = ld(slots + at) + ld(slots + kSlot + at);
       }
+    if (tid == 0)
+      __hip_atomic_store(p.dq_ctr + cut, p.dq_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();  // every wave has read `last` before the staging below reuses the LDS
   }
-  __syncthreads();
-  // all 8 waves store: wave w writes half (w / 4) of the rows of query group w % 4
+  uint16_t* stg = reinterpret_cast<uint16_t*>(smem) + wave * 32 * D;  // the wave's own rows
 #pragma unroll
-  for (int i = 0; i < 16 * CPR / 64; ++i) {
-    const int x = 16 * CPR * b + lane + 64 * i, row = x / CPR, ch = x % CPR;
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = 8 * (e >> 2) + 4 * h + (e & 3);
+      stg[row * D + 32 * c + r] = f32_to_bf16_rne(acc[c][e] * p.sm_scale);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 32 * CPR / 64; ++i) {
+    const int x = lane + 64 * i, row = x / CPR, ch = x % CPR;
     const int64_t q = q0 + row;
     if (q < n)
       *reinterpret_cast<uint4*>(p.dq + ((int64_t)bh * n + q) * D + ch * 8) =
@@ -512,53 +539,51 @@ __device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int i
 // dK, dV
 // ---------------------------------------------------------------------------
 
-// LDS stage of one 64-query step: Q codes (row fragments), the R image of dO,
-// T images of dO and Q, per-query Q scale, LSE (+inf for rows without
-// gradient), D, document ids.
+// LDS stage of one 32-query step: Q codes (row fragments), Q rows, dO rows,
+// per-query Q scale, LSE, -D, document ids.
 template <int D>
 struct DkvStage {
-  static constexpr int qcBytes = 64 * D;
-  static constexpr int rowBytes = 64 * 2 * D;
-  static constexpr int offDo = qcBytes;
-  static constexpr int offTdo = offDo + rowBytes;
-  static constexpr int offTq = offTdo + rowBytes;
-  static constexpr int offQd = offTq + rowBytes;
-  static constexpr int offLse = offQd + 256;
-  static constexpr int offDl = offLse + 256;
-  static constexpr int offDoc = offDl + 256;
-  static constexpr int bytes = offDoc + 256;
-  static constexpr int cQc = qcBytes / 16, cRow = rowBytes / 16;
+  static constexpr int offQ = 32 * D;
+  static constexpr int offDo = offQ + Rows<D>::bytes32;
+  static constexpr int offQd = offDo + Rows<D>::bytes32;
+  static constexpr int offLse = offQd + 128;
+  static constexpr int offNd = offLse + 128;
+  static constexpr int offDoc = offNd + 128;
+  static constexpr int bytes = offDoc + 128;
 };
 
-// LDS of a dK/dV item: two step stages, then the R image of the workgroup's
-// 128 V rows, read as the B operand of dP by the waves that own them.
-template <int D>
-constexpr int kDkvLds = 2 * DkvStage<D>::bytes + kRowsPerWG * 2 * D;
+// The wave's 32 V rows, the column operand of dP in every step, stay in
+// registers (D/4 of them), except with document ids at D = 128: the mixed
+// steps' registers leave no room there (4-8 spilled), so the rows stay in LDS
+// behind the ring.  Measured at 1x30x4416x128 without ids: 903.8 -> 891.4 us.
+template <int D, int MASK>
+constexpr bool kVInRegs = D == 64 || (MASK & 2) == 0;
 
-// dK, dV of item (bh, 128-key block), in `smem` (kDkvLds<D>).  Wave w owns
-// keys 32 * (w % 4) of the workgroup's 128 keys and query half w / 4 of every
-// 64-query step; the two query halves' partial dK and dV are summed (half 0 +
-// half 1) at the end.
+// LDS of a dK/dV item: two step stages, then the V rows if they are there.
+template <int D, int MASK>
+constexpr int kDkvLds = 2 * DkvStage<D>::bytes + (kVInRegs<D, MASK> ? 0 : kBwdWaves * Rows<D>::bytes32);
+
+// dK, dV of item (bh, 128-key block), in `smem` (kDkvLds<D, MASK>).  Wave w owns
+// keys 32w .. +31 of the block.
 template <int D, int QK, int MASK>
 __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int item) {
   using St = DkvStage<D>;
+  using R = Rows<D>;
   using SAcc = typename BAcc<QK>::type;
   constexpr int NC = D / 32, CPR = D / 8;
-  constexpr int kVOff = 2 * St::bytes;
-  static_assert(4 * NC * 16 * 64 * 4 <= 2 * St::bytes, "partial dK/dV exchange must fit in the ring");
+  constexpr int kOutStride = 2 * D + 16;  // bytes of a staged output row: no bank is hit by two rows' 8-byte pieces
+  static_assert(kBwdWaves * 32 * kOutStride <= 2 * St::bytes, "the output staging must fit in the ring");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar registers
   const int h = lane >> 5, r = lane & 31;
-  const int kg = wave & 3, a = wave >> 2;  // key group, query half
   const int nkb = (int)(p.np / kRowsPerWG);
   const int bh = item / nkb, kb = item % nkb;
   const int bidx = bh / p.h;
   const int64_t n = p.n, np = p.np;
   const int nkv = (int)((n + 63) / 64);
-  const int nsteps = (int)((n + 63) / 64);  // 64-query steps holding a query below N
-  const int64_t k0 = (int64_t)kb * kRowsPerWG + 32 * kg;
+  const int nsteps = (int)((n + 31) / 32);  // 32-query steps holding a query below N
+  const int64_t k0 = (int64_t)kb * kRowsPerWG + 32 * wave;
   const int64_t krow = k0 + r;
-  const int my_tile = 2 * kb + (kg >> 1);  // reference KV tile of this wave's keys
   const bool wave_live = k0 < n;
 
   // ---- per-wave key state -------------------------------------------------------------
@@ -568,15 +593,19 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
 #pragma unroll
     for (int c = 0; c < NC; ++c) kf[c] = *reinterpret_cast<const i32x4*>(kbp + (c * 64 + lane) * 16);
   }
-  {
-    // the R image of V rows [kb*128, +128) into the persistent region
-    const uint8_t* rvs = reinterpret_cast<const uint8_t*>(p.rv + ((int64_t)bh * np + (int64_t)kb * kRowsPerWG) * D);
-    dma_chunks<kRowsPerWG * CPR>(smem + kVOff, wave, lane, [&](int x) { return rvs + (uint32_t)(x * 16); });
+  const int src_off = R::src_off(lane), tr_off = R::tr_off(lane);
+  const int row_off[2] = {R::row_off(lane, 0), R::row_off(lane, 1)};
+  bf16x8 vf[2 * NC];                                         // V[krow][16c2 + 8h, +8)
+  uint8_t* vlds = smem + 2 * St::bytes + wave * R::bytes32;  // or the wave's V rows
+  if constexpr (kVInRegs<D, MASK>) {
+    const uint16_t* vr = p.v + ((int64_t)bh * n + min(krow, n - 1)) * D + 8 * h;
+#pragma unroll
+    for (int c2 = 0; c2 < 2 * NC; ++c2) vf[c2] = *reinterpret_cast<const bf16x8*>(vr + 16 * c2);
+  } else if (wave_live) {
+    dma_rows32<D, 1>(vlds, 0, src_off, p.v + ((int64_t)bh * n + k0) * D, n - k0);
   }
-  const u32x4* vrl = reinterpret_cast<const u32x4*>(smem + kVOff);
   const float kd = p.ks[(int64_t)bh * np + krow];
-  const bool key_ok = krow < n;
-  const int dk_doc = (MASK & 2) ? (key_ok ? p.doc[(int64_t)bidx * n + krow] : -1) : 0;
+  const int dk_doc = (MASK & 2) ? (krow < n ? p.doc[(int64_t)bidx * n + krow] : -1) : 0;
   f32x16 dva[NC], dka[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
@@ -584,9 +613,7 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
     dka[c] = f32x16{0};
   }
 
-  const uint8_t* mrow = (MASK & 1) ? p.tile_mask + (int64_t)bh * p.mask_stride_z : nullptr;
-  // document-id summaries of the workgroup's two key tiles
-  const int4* qs32 = (MASK & 2) ? p.q_sum + (int64_t)bidx * (np / 32) : nullptr;
+  // ---- active steps: 32-query block s against the workgroup's two key tiles, this wave's one ----
   int4 ksum[2] = {make_int4(0, 0, 0, 0), make_int4(0, 0, 0, 0)};
   if constexpr (MASK & 2) {
 #pragma unroll
@@ -594,209 +621,176 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
       ksum[i] = 2 * kb + i < nkv ? load_uniform(p.kv_sum, (int64_t)bidx * nkv + 2 * kb + i)
                                  : make_int4(0x7fffffff, -0x7fffffff, 0, 0);
   }
-  auto wave_active = [&](int s) __attribute__((always_inline)) -> bool {
-    bool on = true;
-    if constexpr (MASK & 1) on = my_tile < nkv && load_uniform_u8(mrow, (int64_t)(s >> 1) * p.mask_nkv + my_tile) != 0;
-    if constexpr (MASK & 2) on = on && classify(load_uniform(qs32, 2 * s + a), ksum[kg >> 1]) != 0;
-    return on;
-  };
-  auto active = [&](int s) __attribute__((always_inline)) -> bool {
-    bool on = true;
-    if constexpr (MASK & 1) {
-      const uint8_t* m = mrow + (int64_t)(s >> 1) * p.mask_nkv;
-      on = load_uniform_u8(m, 2 * kb) != 0 || (2 * kb + 1 < nkv && load_uniform_u8(m, 2 * kb + 1) != 0);
+  StepMasks sm{0, 0, 0};
+  int sm_base = -1;
+  auto find = [&](int s) __attribute__((always_inline)) -> int {
+    if constexpr (MASK == 0) return s;
+    while (s < nsteps) {
+      if ((s & ~63) != sm_base) {
+        sm_base = s & ~63;
+        const int st = min(sm_base + lane, nsteps - 1);
+        bool on0 = sm_base + lane < nsteps, on1 = on0 && 2 * kb + 1 < nkv;
+        if constexpr (MASK & 1) {
+          const uint8_t* m = p.tile_mask + (int64_t)bh * p.mask_stride_z + (int64_t)(st >> 2) * p.mask_nkv + 2 * kb;
+          on0 = on0 && m[0] != 0;
+          on1 = on1 && m[on1 ? 1 : 0] != 0;
+        }
+        bool mixed = false;
+        if constexpr (MASK & 2) {
+          const int4 qs = p.q_sum[(int64_t)bidx * (np / 32) + st];
+          const int c0 = classify(qs, ksum[0]), c1 = classify(qs, ksum[1]);
+          on0 = on0 && c0 != 0;
+          on1 = on1 && c1 != 0;
+          mixed = (wave >> 1 ? c1 : c0) == 2;
+        }
+        sm.wg = __ballot(on0 || on1);
+        sm.on = __ballot(wave >> 1 ? on1 : on0);
+        sm.mixed = __ballot(mixed);
+      }
+      const uint64_t m = sm.wg >> (s & 63);
+      if (m) return s + __builtin_ctzll(m);
+      s = sm_base + 64;
     }
-    if constexpr (MASK & 2) {
-      const int4 q64 = merge_summary(load_uniform(qs32, 2 * s), load_uniform(qs32, 2 * s + 1));
-      on = on && (classify(q64, ksum[0]) != 0 || classify(q64, ksum[1]) != 0);
-    }
-    return on;
-  };
-  auto next_active = [&](int s) __attribute__((always_inline)) -> int {
-    while (s < nsteps && !active(s)) ++s;
-    return s;
+    return nsteps;
   };
 
-  // ---- staging: bulk by direct global -> LDS loads, per-query values through registers ----
-  u32x4 psm = u32x4{0, 0, 0, 0};
+  // ---- staging -----------------------------------------------------------------------
   auto load_step = [&](int s, int stage) __attribute__((always_inline)) {
-    const int64_t m0 = (int64_t)s * 64;
+    const int64_t m0 = (int64_t)s * 32;
     uint8_t* sb = smem + stage * St::bytes;
-    const uint8_t* qcs = p.qc + ((int64_t)bh * np + m0) * D;
-    const uint8_t* tds = reinterpret_cast<const uint8_t*>(p.tdo + ((int64_t)bh * np + m0) * D);
-    const uint8_t* tqs = reinterpret_cast<const uint8_t*>(p.tq + ((int64_t)bh * np + m0) * D);
-    const uint8_t* rds = reinterpret_cast<const uint8_t*>(p.rdo + ((int64_t)bh * np + m0) * D);
-    if (tid < 64) {
-      // one path for the 64 lanes of wave 0 (no per-lane branches writing the
-      // same registers, which would make the compiler wait for loads in
-      // flight, the stage loads included): lanes 16g .. 16g+15 take values
-      // 4(lane&15) .. +3 of the Q scales (g=0), LSE (g=1, -inf past N), D
-      // (g=2) or query document ids (g=3, -1 past N)
-      const int g = tid >> 4;
-      const int64_t m = m0 + 4 * (tid & 15);
-      const uint32_t* base = g == 0   ? reinterpret_cast<const uint32_t*>(p.qs + (int64_t)bh * np)
-                             : g == 1 ? reinterpret_cast<const uint32_t*>(p.lse + (int64_t)bh * n)
-                             : g == 2 ? reinterpret_cast<const uint32_t*>(p.delta + (int64_t)bh * np)
-                             : (MASK & 2) ? reinterpret_cast<const uint32_t*>(p.doc + (int64_t)bidx * n)
-                                          : reinterpret_cast<const uint32_t*>(p.qs);  // not read
-      const int64_t lim = (g == 0 || g == 2) ? np : (g == 1 || (MASK & 2)) ? n : 0;
-      const uint32_t dflt = g == 1 ? __float_as_uint(-INFINITY) : g == 3 ? 0xffffffffu : 0u;
-      u32x4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = m + i < lim ? base[m + i] : dflt;
-      psm = v;
+    dma_chunks_buf<2 * D, kBwdWaves>(sb, wave, lane, raw_rsrc(p.qc + ((int64_t)bh * np + m0) * D, 32 * D), 0);
+    dma_rows32<D, kBwdWaves>(sb + St::offDo, wave, src_off, p.dout + ((int64_t)bh * n + m0) * D, n - m0);
+    dma_rows32<D, kBwdWaves>(sb + St::offQ, wave, src_off, p.q + ((int64_t)bh * n + m0) * D, n - m0);
+    if (wave < 3) {
+      const float* src = wave == 0 ? p.qs : wave == 1 ? p.lse_pad : p.neg_delta;
+      dma_words32(sb + St::offQd + wave * 128, lane, src + (int64_t)bh * np + m0);
+    } else if constexpr (MASK & 2) {
+      dma_words32_unaligned(sb + St::offDoc, lane, p.doc + (int64_t)bidx * n + m0, n - m0);
     }
-    // the stage loads after the small ones: a wait for the small values then
-    // leaves the stage loads in flight
-    dma_chunks<St::cQc>(sb, wave, lane, [&](int x) { return qcs + (uint32_t)(x * 16); });
-    dma_chunks<St::cRow>(sb + St::offTdo, wave, lane, [&](int x) { return tds + (uint32_t)(x * 16); });
-    dma_chunks<St::cRow>(sb + St::offTq, wave, lane, [&](int x) { return tqs + (uint32_t)(x * 16); });
-    dma_chunks<St::cRow>(sb + St::offDo, wave, lane, [&](int x) { return rds + (uint32_t)(x * 16); });
-  };
-  auto store_small = [&](int stage) __attribute__((always_inline)) {
-    uint8_t* sb = smem + stage * St::bytes;
-    u32x4 v = psm;
-    if (tid >= 16 && tid < 32) {
-      // +inf for rows with no gradient (past N, or no visible key in the
-      // forward): 2^(s - inf) = 0 needs no per-element test
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(v[i]) > -INFINITY ? v[i] : __float_as_uint(INFINITY);
-    }
-    if (tid < 48 || ((MASK & 2) && tid < 64)) reinterpret_cast<u32x4*>(sb + St::offQd)[tid] = v;
   };
 
-  int s = next_active(0);
-  if (s < nsteps) {
-    load_step(s, 0);
-    store_small(0);
-  }
-  wait_vmem();
-  __syncthreads();
+  int s = find(0);
+  if (s < nsteps) load_step(s, 0);
   int stage = 0;
   while (s < nsteps) {
-    const int sn = next_active(s + 1);
+    const bool on = wave_live && (MASK == 0 || ((sm.on >> (s & 63)) & 1));
+    const bool mixed = (MASK & 2) && ((sm.mixed >> (s & 63)) & 1);
+    const int sn = find(s + 1);
+    wait_vmem();
+    __syncthreads();  // stage complete; every wave is past the step that used the other stage
     if (sn < nsteps) load_step(sn, stage ^ 1);
-    if (wave_live && wave_active(s)) {
+    if (on) {
       const uint8_t* sb = smem + stage * St::bytes;
       const f32x4* qdl = reinterpret_cast<const f32x4*>(sb + St::offQd);
       const f32x4* lsl = reinterpret_cast<const f32x4*>(sb + St::offLse);
-      const f32x4* dll = reinterpret_cast<const f32x4*>(sb + St::offDl);
+      const f32x4* ndl = reinterpret_cast<const f32x4*>(sb + St::offNd);
       const int4* dql = reinterpret_cast<const int4*>(sb + St::offDoc);
-      const u32x4* dol = reinterpret_cast<const u32x4*>(sb + St::offDo);
-      const bf16x8* tdl = reinterpret_cast<const bf16x8*>(sb + St::offTdo);
-      const bf16x8* tql = reinterpret_cast<const bf16x8*>(sb + St::offTq);
-      // S = Q . K^T: rows = queries 32a + (lane-local rows), columns = this wave's keys
+      // S = Q . K^T: rows = queries, columns = this wave's keys
       i32x4 qa[NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) qa[c] = reinterpret_cast<const i32x4*>(sb)[(a * NC + c) * 64 + lane];
+      for (int c = 0; c < NC; ++c) qa[c] = reinterpret_cast<const i32x4*>(sb)[c * 64 + lane];
       const SAcc sacc = score_block<D, QK>(qa, kf);
-      // dP = dO . V^T, operands read two MFMAs ahead of their use
-      f32x16 dp = f32x16{0};
-      u32x4 wf[2 * NC], vf[2 * NC];
+      // dP - D = dO . V^T - D
+      f32x16 dp;
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+        const f32x4 d4 = ndl[2 * J + h];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dp[4 * J + i] = d4[i];
+      }
+      // ... its MFMAs issued under the exponentials of P
+      const uint8_t* dol = sb + St::offDo;
+      bf16x8 wf[2 * NC];
       auto dpfrag = [&](int c2) __attribute__((always_inline)) {
-        wf[c2] = dol[(a * 2 * NC + c2) * 64 + lane];   // dO[query 32a + r][16c2 + 8h, +8)
-        vf[c2] = vrl[(kg * 2 * NC + c2) * 64 + lane];  // V[krow][16c2 + 8h, +8)
+        wf[c2] = *reinterpret_cast<const bf16x8*>(dol + row_off[c2 & 1] + R::row_imm(c2));
+        if constexpr (!kVInRegs<D, MASK>)
+          vf[c2] = *reinterpret_cast<const bf16x8*>(vlds + row_off[c2 & 1] + R::row_imm(c2));
       };
       dpfrag(0);
       dpfrag(1);
+      float pr[16];
+      bf16x8 pb[2], db[2];
+      // s - lse = acc * (qd * kd) - lse; keys past N need no test: their
+      // column only feeds their own dK / dV rows, which are not stored
+      constexpr int kPer = 16 / (2 * NC);  // scores per MFMA
+      f32x4 qd4, ls4;
 #pragma unroll
       for (int c2 = 0; c2 < 2 * NC; ++c2) {
         __builtin_amdgcn_sched_barrier(0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wf[c2]),
-                                                     __builtin_bit_cast(bf16x8, vf[c2]), dp, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[c2], vf[c2], dp, 0, 0, 0);
         if (c2 + 2 < 2 * NC) dpfrag(c2 + 2);
-      }
-      bf16x8 pb[2], db[2];
 #pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        const f32x4 qd4 = qdl[8 * a + 2 * J + h];
-        const f32x4 ls4 = lsl[8 * a + 2 * J + h];
-        const f32x4 dl4 = dll[8 * a + 2 * J + h];
-        int4 dq4 = make_int4(0, 0, 0, 0);
-        if constexpr (MASK & 2) dq4 = dql[8 * a + 2 * J + h];
-        const int dqd[4] = {dq4.x, dq4.y, dq4.z, dq4.w};
-        // s - lse = acc * (qd * kd) - lse; keys past N need no test: their
-        // column only feeds their own dK / dV rows, which are not stored
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int e = 4 * J + i;
-          float pr = __builtin_amdgcn_exp2f(fmaf((float)sacc[e], qd4[i] * kd, -ls4[i]));
-          if constexpr (MASK & 2) pr = doc_visible(dqd[i], dk_doc) ? pr : 0.0f;
-          const float ds = pr * (dp[e] - dl4[i]);
-          pb[e >> 3][e & 7] = (__bf16)pr;
-          db[e >> 3][e & 7] = (__bf16)(ds * p.sm_scale);
+        for (int e = kPer * c2; e < kPer * c2 + kPer; ++e) {
+          const int J = e >> 2, i = e & 3;
+          if (i == 0) {
+            qd4 = qdl[2 * J + h];
+            ls4 = lsl[2 * J + h];
+          }
+          pr[e] = __builtin_amdgcn_exp2f(fmaf((float)sacc[e], qd4[i] * kd, -ls4[i]));
+          if constexpr ((MASK & 2) == 0) pb[e >> 3][e & 7] = (__bf16)pr[e];
         }
       }
-      // dV^T += dO^T . P, dK^T += Q^T . dS over this query half; operand
-      // fragments read two MFMA pairs ahead of their use
-      constexpr int kPairs = NC * 2, kAhead = 2;
-      bf16x8 tdf[kPairs], tqf[kPairs];
-      auto frag = [&](int i) __attribute__((always_inline)) {
-        const int ci = (((i >> 1) * 2 + a) * 2 + (i & 1)) * 64 + lane;  // c = i / 2, tt = i % 2
-        tdf[i] = tdl[ci];
-        tqf[i] = tql[ci];
-      };
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (MASK & 2) {
+        if (mixed) {  // hidden keys: p = 0
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) frag(i);
+          for (int J = 0; J < 4; ++J) {
+            const int4 dq4 = dql[2 * J + h];
+            const int dqd[4] = {dq4.x, dq4.y, dq4.z, dq4.w};
 #pragma unroll
-      for (int i = 0; i < kPairs; ++i) {
-        __builtin_amdgcn_sched_barrier(0);
-        const int c = i >> 1, tt = i & 1;
-        dva[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tdf[i], pb[tt], dva[c], 0, 0, 0);
-        dka[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tqf[i], db[tt], dka[c], 0, 0, 0);
-        if (i + kAhead < kPairs) frag(i + kAhead);
+            for (int i = 0; i < 4; ++i) pr[4 * J + i] = doc_visible(dqd[i], dk_doc) ? pr[4 * J + i] : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) pb[e >> 3][e & 7] = (__bf16)pr[e];
       }
+      // dV^T += dO^T . P under the rounding of dS, then dK^T += Q^T . dS
+      const uint8_t* tdl = sb + St::offDo + tr_off;
+      const uint8_t* tql = sb + St::offQ + tr_off;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          dva[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(tdl, c, tt), pb[tt], dva[c], 0, 0, 0);
+#pragma unroll
+          for (int e = 8 / NC * c; e < 8 / NC * (c + 1); ++e) db[tt][e] = (__bf16)(pr[8 * tt + e] * dp[8 * tt + e]);
+        }
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          dka[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag<D>(tql, c, tt), db[tt], dka[c], 0, 0, 0);
     }
-    if (sn < nsteps) store_small(stage ^ 1);
-    wait_vmem();
-    __syncthreads();
     stage ^= 1;
     s = sn;
   }
+  wait_vmem();
+  __syncthreads();  // the ring is free
 
-  // ---- epilogue: (half 0 + half 1), lane (h, r) holds key r, channels 32c + 8J + 4h + i ----
-  float* xch = reinterpret_cast<float*>(smem) + kg * NC * 16 * 64;
-  if (a == 1) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) xch[(c * 16 + e) * 64 + lane] = dva[c][e];
-  }
-  __syncthreads();
-  if (a == 0) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) dva[c][e] += xch[(c * 16 + e) * 64 + lane];
-  }
-  __syncthreads();
-  if (a == 1) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) xch[(c * 16 + e) * 64 + lane] = dka[c][e];
-  }
-  __syncthreads();
-  if (a == 0 && key_ok) {
-    uint16_t* dvr = p.dv + ((int64_t)bh * n + krow) * D;
-    uint16_t* dkr = p.dk + ((int64_t)bh * n + krow) * D;
+  // ---- epilogue: lane (h, r) holds key r, channels 32c + 8J + 4h + i; rows staged in LDS ----
+  uint8_t* stg = smem + wave * 32 * kOutStride;  // the wave's own rows
+  auto store_rows = [&](const f32x16* x, float scale, uint16_t* out) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int J = 0; J < 4; ++J) {
-        const int ch = 32 * c + 8 * J + 4 * h;
-        float kk[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) kk[i] = dka[c][4 * J + i] + xch[(c * 16 + 4 * J + i) * 64 + lane];
-        uint2 va, ka2;
-        va.x = f32_to_bf16_rne(dva[c][4 * J + 0]) | ((uint32_t)f32_to_bf16_rne(dva[c][4 * J + 1]) << 16);
-        va.y = f32_to_bf16_rne(dva[c][4 * J + 2]) | ((uint32_t)f32_to_bf16_rne(dva[c][4 * J + 3]) << 16);
-        ka2.x = f32_to_bf16_rne(kk[0]) | ((uint32_t)f32_to_bf16_rne(kk[1]) << 16);
-        ka2.y = f32_to_bf16_rne(kk[2]) | ((uint32_t)f32_to_bf16_rne(kk[3]) << 16);
-        *reinterpret_cast<uint2*>(dvr + ch) = va;
-        *reinterpret_cast<uint2*>(dkr + ch) = ka2;
+        uint2 w;
+        w.x = f32_to_bf16_rne(x[c][4 * J + 0] * scale) | ((uint32_t)f32_to_bf16_rne(x[c][4 * J + 1] * scale) << 16);
+        w.y = f32_to_bf16_rne(x[c][4 * J + 2] * scale) | ((uint32_t)f32_to_bf16_rne(x[c][4 * J + 3] * scale) << 16);
+        *reinterpret_cast<uint2*>(stg + r * kOutStride + (32 * c + 8 * J + 4 * h) * 2) = w;
       }
-  }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 32 * CPR / 64; ++i) {
+      const int y = lane + 64 * i, row = y / CPR, ch = y % CPR;
+      if (k0 + row < n)
+        *reinterpret_cast<uint4*>(out + ((int64_t)bh * n + k0 + row) * D + ch * 8) =
+            *reinterpret_cast<const uint4*>(stg + row * kOutStride + ch * 16);
+    }
+    __syncthreads();
+  };
+  store_rows(dva, 1.0f, p.dv);
+  store_rows(dka, p.sm_scale, p.dk);
 }
 
 // The two gradient passes in one launch: workgroups [0, kv_wgs) take the
@@ -808,57 +802,56 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
 // items come last.  Each part deals its items to the XCDs like a launch of
 // its own (xcd_item): kv_wgs is a multiple of the XCD count, so a dQ
 // workgroup's XCD is its index within the part modulo 8.
-template <int D>
-constexpr int kBwdLds = kDkvLds<D> > 2 * DqStage<D>::bytes ? kDkvLds<D> : 2 * DqStage<D>::bytes;
+template <int D, int MASK>
+constexpr int kBwdLds = kDkvLds<D, MASK> > 2 * DqStage<D>::bytes ? kDkvLds<D, MASK> : 2 * DqStage<D>::bytes;
+static_assert(2 * kBwdLds<128, 2> <= 160 * 1024, "two workgroups per CU");
 
 template <int D, int QK, int MASK>
-__global__ void __launch_bounds__(kBwdThreads) bwd_kernel(BwdParams p, int items, int kv_wgs) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[kBwdLds<D>];
+__global__ void __launch_bounds__(kBwdThreads, 2) bwd_kernel(BwdParams p, int items, int kv_wgs) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[kBwdLds<D, MASK>];
   const int wg = (int)blockIdx.x;
-  const int nt = (int)((p.n + 63) / 64), mid = nt / 2;
   if (wg < kv_wgs) {
     if (wg < items) dkdv_item<D, QK, MASK>(p, smem, xcd_item(wg, items));
     return;
   }
+  const int steps = (int)((p.n + 31) / 32), mid = (int)((p.n + 63) / 64) / 2 * 2;  // 32-key steps; whole tiles first
   const int j = wg - kv_wgs, whole = items - p.dq_split;
-  if (j < whole)
-    dq_item<D, QK, MASK>(p, smem, xcd_item(j, items), 0, nt, -1, 0);
-  else if (j < items)
-    dq_item<D, QK, MASK>(p, smem, xcd_item(j, items), 0, mid, j - whole, 0);
-  else
-    dq_item<D, QK, MASK>(p, smem, xcd_item(j - p.dq_split, items), mid, nt, j - items, 1);
+  const bool second = j >= items, cut = j >= whole;
+  dq_item<D, QK, MASK>(p, smem, xcd_item(second ? j - p.dq_split : j, items), second ? mid : 0,
+                       cut && !second ? mid : steps, cut ? (second ? j - items : j - whole) : -1, second ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
 
-// The preparation in one launch, grid (np / 64, BH, 5): z = 0, 1 the T images
-// of tjobs, z = 2, 3 the R images of rjobs, z = 4 D.
+// The preparation in one launch, grid (np / 64, BH, 1 or 2): z = 0 the
+// per-query values, z = 1 the smoothed K rows.
 template <int D>
-__global__ void __launch_bounds__(256) bwd_prep_kernel(TImageJobs tjobs, TImageJobs rjobs,
-                                                       const uint16_t* __restrict__ dout,
-                                                       const uint16_t* __restrict__ out, int64_t n, int64_t np,
-                                                       float* __restrict__ delta) {
-  __shared__ __attribute__((aligned(16))) uint8_t img[2 * 64 * D];
-  const int z = blockIdx.z, bh = blockIdx.y;
+__global__ void __launch_bounds__(256) bwd_prep_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ mu,
+                                                       uint16_t* __restrict__ kt, const uint16_t* __restrict__ dout,
+                                                       const uint16_t* __restrict__ out,
+                                                       const float* __restrict__ lse, int64_t n, int64_t np,
+                                                       float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
+  const int bh = blockIdx.y;
   const int64_t bx = blockIdx.x;
-  if (z < 2)
-    timage_block<D>(tjobs, z, bh, bx, n, np, img);
-  else if (z < 4)
-    rimage_block<D>(rjobs, z - 2, bh, bx, n, np);
-  else
-    delta_block<D>(dout, out, bh, bx, n, np, delta);
+  if (blockIdx.z == 0)
+    delta_block<D>(dout, out, lse, bh, bx, n, np, neg_delta, lse_pad);
+  else if (bx * 64 < n)
+    smooth_block<D>(k, mu, bh, bx, n, kt);
 }
 
-hipError_t launch_bwd_prep(const TImageJobs& tjobs, const TImageJobs& rjobs, const uint16_t* dout,
-                           const uint16_t* out, int64_t bh, int64_t n, int64_t d, float* delta, hipStream_t st) {
+hipError_t launch_bwd_prep(const uint16_t* k, const uint16_t* mu, uint16_t* kt, const uint16_t* dout,
+                           const uint16_t* out, const float* lse, int64_t bh, int64_t n, int64_t d, float* neg_delta,
+                           float* lse_pad, hipStream_t st) {
   const int64_t np = padded_len(n);
-  const dim3 grid((unsigned)(np / 64), (unsigned)bh, 5u);
+  const dim3 grid((unsigned)(np / 64), (unsigned)bh, mu ? 2u : 1u);
   if (d == 128)
-    hipLaunchKernelGGL(bwd_prep_kernel<128>, grid, dim3(256), 0, st, tjobs, rjobs, dout, out, n, np, delta);
+    hipLaunchKernelGGL(bwd_prep_kernel<128>, grid, dim3(256), 0, st, k, mu, kt, dout, out, lse, n, np, neg_delta,
+                       lse_pad);
   else if (d == 64)
-    hipLaunchKernelGGL(bwd_prep_kernel<64>, grid, dim3(256), 0, st, tjobs, rjobs, dout, out, n, np, delta);
+    hipLaunchKernelGGL(bwd_prep_kernel<64>, grid, dim3(256), 0, st, k, mu, kt, dout, out, lse, n, np, neg_delta,
+                       lse_pad);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

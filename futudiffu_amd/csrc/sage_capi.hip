@@ -130,9 +130,10 @@ int check_producer(const void* qkv, const float* q_norm_w, const float* k_norm_w
 }
 
 // Backward workspace: byte offsets of the quantization's outputs (codes,
-// scales, K mean, column-sum partials), the T images of dO, Q and K~, and D.
+// scales, K mean, column-sum partials, the V operand), the smoothed K rows,
+// -D and the padded LSE.
 struct BwdWorkspace {
-  size_t qc, qs, kc, ks, kmean, quant, tdo, tq, tk, rdo, rv, delta, sums, dq_part, dq_ctr, bytes;
+  size_t qc, qs, kc, ks, kmean, quant, vop, kt, neg_delta, lse_pad, sums, dq_part, dq_ctr, bytes;
 };
 
 BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
@@ -150,12 +151,15 @@ BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
   w.ks = take(rows * 4);
   w.kmean = take((size_t)bh * d * 2);
   w.quant = take(sage::quant_workspace_bytes(bh, n, d));
-  w.tdo = take(rows * d * 2);
-  w.tq = take(rows * d * 2);
-  w.tk = take(rows * d * 2);
-  w.rdo = take(rows * d * 2);
-  w.rv = take(rows * d * 2);
-  w.delta = take(rows * 4);
+  // Five regions of one bf16 image each: the size is part of the interface
+  // (callers keep workspaces of it), the last three are not used in full
+  // since the passes read dO, Q and V as they are.
+  w.vop = take(rows * d * 2);
+  w.kt = take(rows * d * 2);
+  w.lse_pad = take(rows * d * 2);
+  take(rows * d * 2);
+  take(rows * d * 2);
+  w.neg_delta = take(rows * 4);
   // document-id summaries (used with doc_ids): key tiles, 32- and 128-row blocks
   w.sums = take((size_t)b * ((n + 63) / 64 + np / 32 + np / 128) * sizeof(int4));
   // fp32 partial dQ of the cut items' two key-tile halves, their counters
@@ -500,27 +504,17 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
   const auto* q16 = static_cast<const uint16_t*>(q);
   const auto* k16 = static_cast<const uint16_t*>(k);
   const auto* do16 = static_cast<const uint16_t*>(dout);
-  // codes, scales and the K mean of the forward's per-token quantization;
-  // dO takes the place of V, so the bf16 "V operand" written is dO's T image
+  // codes, scales and the K mean of the forward's per-token quantization
   hipError_t e = sage::launch_quantize(
       qk_kind, SAGE_PV_BF16, SAGE_GRAN_TOKEN, smooth_k != 0, q16, k16, do16, bh, n, d,
       sm_scale_log2e, reinterpret_cast<double*>(w + ws.quant), w + ws.qc,
-      reinterpret_cast<float*>(w + ws.qs), w + ws.kc, reinterpret_cast<float*>(w + ws.ks), w + ws.tdo, nullptr,
+      reinterpret_cast<float*>(w + ws.qs), w + ws.kc, reinterpret_cast<float*>(w + ws.ks), w + ws.vop, nullptr,
       reinterpret_cast<uint16_t*>(w + ws.kmean), sage::ProdArgs{}, stream);
   if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (quantize)");
-  sage::TImageJobs jobs{};
-  jobs.x[0] = q16;
-  jobs.out[0] = reinterpret_cast<uint16_t*>(w + ws.tq);
-  jobs.x[1] = k16;
-  jobs.mu[1] = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kmean) : nullptr;
-  jobs.out[1] = reinterpret_cast<uint16_t*>(w + ws.tk);
-  sage::TImageJobs rjobs{};
-  rjobs.x[0] = do16;
-  rjobs.out[0] = reinterpret_cast<uint16_t*>(w + ws.rdo);
-  rjobs.x[1] = static_cast<const uint16_t*>(v);
-  rjobs.out[1] = reinterpret_cast<uint16_t*>(w + ws.rv);
-  e = sage::launch_bwd_prep(jobs, rjobs, do16, static_cast<const uint16_t*>(out), bh, n, d,
-                            reinterpret_cast<float*>(w + ws.delta), stream);
+  const uint16_t* mean = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kmean) : nullptr;
+  e = sage::launch_bwd_prep(k16, mean, reinterpret_cast<uint16_t*>(w + ws.kt), do16, static_cast<const uint16_t*>(out),
+                            lse, bh, n, d, reinterpret_cast<float*>(w + ws.neg_delta),
+                            reinterpret_cast<float*>(w + ws.lse_pad), stream);
   if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (prep)");
   const int4* sums = reinterpret_cast<const int4*>(w + ws.sums);
   const int64_t np = sage::padded_len(n);
@@ -535,15 +529,12 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
   p.qs = reinterpret_cast<const float*>(w + ws.qs);
   p.kc = w + ws.kc;
   p.ks = reinterpret_cast<const float*>(w + ws.ks);
+  p.q = q16;
+  p.kt = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kt) : k16;
   p.v = static_cast<const uint16_t*>(v);
   p.dout = do16;
-  p.tq = reinterpret_cast<const uint16_t*>(w + ws.tq);
-  p.tk = reinterpret_cast<const uint16_t*>(w + ws.tk);
-  p.tdo = reinterpret_cast<const uint16_t*>(w + ws.tdo);
-  p.rdo = reinterpret_cast<const uint16_t*>(w + ws.rdo);
-  p.rv = reinterpret_cast<const uint16_t*>(w + ws.rv);
-  p.lse = lse;
-  p.delta = reinterpret_cast<const float*>(w + ws.delta);
+  p.lse_pad = reinterpret_cast<const float*>(w + ws.lse_pad);
+  p.neg_delta = reinterpret_cast<const float*>(w + ws.neg_delta);
   p.tile_mask = tile_mask;
   p.mask_stride_z = mask_stride_z;
   p.mask_nkv = mask_nkv;

@@ -183,23 +183,20 @@ hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t p
 
 // Backward (sage_kernels.py:321-349, :805-1030, :1491-1722).  Codes and
 // scales are the quantization's per-token outputs ([BH, Np] layout, Q scale
-// with sm_scale*log2(e)); tq / tk / tdo are T images [BH, Np, D] of Q, the
-// smoothed K and dO, rdo / rv R images of dO and V; v, dout, lse and the
-// gradients are unpadded [BH, N(, D)]; delta is [BH, Np].
+// with sm_scale*log2(e)); q, v, dout, kt (K~, the smoothed K: k itself without
+// smoothing) and the gradients are plain rows [BH, N, D]; lse_pad and
+// neg_delta are [BH, Np] (launch_bwd_prep).
 struct BwdParams {
   const uint8_t* qc;
   const float* qs;
   const uint8_t* kc;
   const float* ks;
+  const uint16_t* q;
+  const uint16_t* kt;
   const uint16_t* v;
   const uint16_t* dout;
-  const uint16_t* tq;
-  const uint16_t* tk;
-  const uint16_t* tdo;
-  const uint16_t* rdo;  // R images [BH, Np, D] of dO and V
-  const uint16_t* rv;
-  const float* lse;
-  const float* delta;
+  const float* lse_pad;
+  const float* neg_delta;
   const uint8_t* tile_mask;
   int64_t mask_stride_z;
   int64_t mask_nkv;
@@ -227,16 +224,12 @@ struct BwdParams {
 // multiple of 8, so both halves of an item run on one XCD).
 constexpr int kBwdDqSplit = 64;
 
-// Two operand-image jobs of one launch: x [BH, N, D] bf16 -> out [BH, Np, D]
-// (T or R image), with mu ([BH, D] bf16) subtracted when set (T images only).
-struct TImageJobs {
-  const uint16_t* x[2];
-  const uint16_t* mu[2];
-  uint16_t* out[2];
-};
-
-hipError_t launch_bwd_prep(const TImageJobs& tjobs, const TImageJobs& rjobs, const uint16_t* dout,
-                           const uint16_t* out, int64_t bh, int64_t n, int64_t d, float* delta, hipStream_t st);
+// The backward's own operands: kt = bf16(k - mu) rows [BH, N, D] (not written
+// when mu is null), neg_delta = -rowsum(dout * out) and the LSE with +inf for
+// rows without gradient, both [BH, Np].
+hipError_t launch_bwd_prep(const uint16_t* k, const uint16_t* mu, uint16_t* kt, const uint16_t* dout,
+                           const uint16_t* out, const float* lse, int64_t bh, int64_t n, int64_t d, float* neg_delta,
+                           float* lse_pad, hipStream_t st);
 hipError_t launch_bwd(int qk, int mask, const BwdParams& p, int64_t d, int64_t bh, hipStream_t st);
 hipError_t launch_doc_from_cu(const int32_t* cu, int64_t nb, int64_t nseg, int64_t n, int32_t* doc,
                               hipStream_t st);

@@ -288,8 +288,8 @@ int sage_doc_ids_from_cu_seqlens(const int32_t* cu_seqlens, int64_t b,
 
 /* Bytes of the workspace sage_attn_bwd needs for b*h heads of n tokens of
  * dimension D: the per-token Q / smoothed-K codes, scales and K mean, the
- * K column-sum partials, bf16 operand images of dO, Q and the smoothed K
- * (the bf16 v_codes layout above), D = rowsum(dO * O) (fp32 [BH, Np]), the
+ * K column-sum partials, five bf16 regions of [BH, Np, D] (the smoothed K, the
+ * padded LSE; part of them spare), -D = -rowsum(dO * O) (fp32 [BH, Np]), the
  * document-id summaries, and the fp32 partial dQ of the last dQ items, which
  * run as two key-tile halves (8 MB at D = 128).  No reference counterpart
  * (the Triton launcher allocates these with torch). */
@@ -302,7 +302,7 @@ size_t sage_attn_bwd_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d)
  * (:918-1030, tile-masked :1617-1722), int8 or fp8 QK (:356-590).  P is
  * recomputed from per-token codes of Q and of K (smoothed again when
  * smooth_k != 0, which must match the forward), p = 2^(s - lse):
- *   dV = bf16(P)^T dO, dK = bf16(dS * sm_scale)^T Q, dQ = (bf16(dS) K~) * sm_scale,
+ *   dV = bf16(P)^T dO, dK = (bf16(dS)^T Q) * sm_scale, dQ = (bf16(dS) K~) * sm_scale,
  *   dS = P (dO V^T - D), each output rounded once to bf16.
  *   q, k, v, out,
  *   dout, dq, dk, dv  bf16 [BH, N, D] contiguous (the [B, H, N, D] tensors).

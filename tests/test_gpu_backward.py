@@ -233,3 +233,31 @@ def test_backward_dq_halves_match_whole_items(cuda, monkeypatch):
         rq, _, _ = O.sage_backward(q[:, sl], k[:, sl], v[:, sl], out_c[:, sl], lse_c[hh:hh + 1], dout[:, sl], sm,
                                    head_chunk=1)
         _close(g1[0][:, sl], rq, f"head {hh} dq")
+
+
+@pytest.mark.parametrize("N", [1, 31, 33, 64, 65, 127, 129, 2100])
+@pytest.mark.parametrize("kind", ["none", "tile", "doc"])
+def test_backward_step_edges(cuda, N, kind):
+    """Sequence lengths around the 32-row steps, 64-key tiles and 128-row items
+    of both passes, and past the 64 steps whose activity is read at once (2048
+    tokens), with the active steps on both sides of that line; D alternates.
+    The bound is _close's: the rounding of P and dS to bf16 (2^-9 each) where a
+    different summation order moves a value across a tie."""
+    D = 128 if N % 2 else 64
+    B, H = 2, 1
+    q, k, v, dout = _inputs(B, H, N, D, seed=100 + N)
+    cuts = [N // 3, N - N // 3]
+    bm = O.build_block_mask(cuts, N) if kind == "tile" else None
+    doc = None
+    if kind == "doc":
+        doc = torch.cat([torch.full((B, cuts[0]), 0), torch.full((B, cuts[1]), 1)], 1).to(torch.int32)
+        doc[1, N // 2:] = -1
+        doc[1, 0] = 0  # a valid key for the padded queries
+    print(f"bwd edges N={N} D={D} {kind}", flush=True)
+    out, lse, dq, dk, dv = _run(cuda, q, k, v, dout, "int8", True, block_mask=bm, doc_ids=doc)
+    rq, rk, rv = O.sage_backward(q, k, v, out, lse, dout, 1.0 / math.sqrt(D), block_mask=bm, doc_ids=doc)
+    assert torch.isfinite(torch.stack([g.float().abs().max() for g in (dq, dk, dv)])).all()
+    _close(dv, rv, "dv")
+    if N > 1:  # one key: softmax is constant, dQ and dK are rounding only
+        _close(dq, rq, "dq")
+        _close(dk, rk, "dk")
