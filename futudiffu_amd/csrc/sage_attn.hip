@@ -596,6 +596,144 @@ __device__ __forceinline__ void pv_bf16_pair(const uint8_t* sb, const bf16x8 (&p
   }
 }
 
+// One iteration of the pipelined bf16 loop after its loads: the softmax of
+// tile t (scores from its S^T in s0 / s1, K scales in stage sb), the pending
+// product of the previous tile (P in pb, V in stage sbp, the first fragments
+// already in vf0) and the next tile's S^T (K in stage sbn) into s0 / s1, as
+// ten scheduling groups that each pair 2-3 MFMAs with the vector work of 4-8
+// scores and the LDS reads of the next group.
+//
+// The row max is not formed: P is exponentiated in the frame m_ref as it is,
+// and a row whose sum over a lane's 32 values exceeds 2^kTau (necessary for
+// a score above m_ref + kTau, where the frame moves; also taken by NaN and
+// overflow) sends the wave through the full softmax (softmax_bf16) on the kept
+// scores, whose frame decision and values are those of every tile before.  So
+// the results are the same bits, 25 vector instructions and the serial chain
+// max -> frame -> exp leave the loop, and each score's exp can start when it
+// is converted.  Measured against MFMAs and vector work in separate phases
+// with the row max (int8 QK): tile-masked 1x30x6912 packed batch 400 -> 377 us
+// per op, 1x30x4416 from the QKV projection 361 -> 341 us.  What bounds it now:
+// vector issue (about 190 instructions a tile, 0.46 of the cycles) and the
+// matrix cores (0.36) beside the waits of two waves per SIMD.  Returns whether
+// a move is pending (then its factor in alpha).
+constexpr int kVAhead = 2;  // V fragments read before the barrier that ends an iteration
+template <int D>
+__device__ __forceinline__ bf16x8 v_frag(const uint8_t* sb, int lane, int i) {
+  const bf16x8* vl = reinterpret_cast<const bf16x8*>(sb + Stage<D, kPV_BF16>::offV);
+  return vl[((i % (D / 32)) * 4 + i / (D / 32)) * 64 + lane];
+}
+
+template <int D, int QK, int GRAN>
+__device__ __forceinline__ bool tile_bf16(const uint8_t* sb, const uint8_t* sbp, const uint8_t* sbn, const i32x4* qf,
+                                          int lane, float kd_blk, typename SAccT<QK>::type& s0,
+                                          typename SAccT<QK>::type& s1, f32x16* o, const bf16x8 (&vf0)[kVAhead],
+                                          bf16x8 (&pb)[2][2], float wt, float& m_ref, float& l_acc, float& alpha) {
+  using St = Stage<D, kPV_BF16>;
+  constexpr int NC = D / 32;
+  constexpr int kPV = NC * 4;                          // P.V MFMAs: MFMA i is chunk i % NC, key step i / NC
+  constexpr int kQKh = QK == kQK_INT8 ? NC : NC / 2;   // S^T MFMAs per 32-key half
+  constexpr int kGroups = 10;
+  const int h = lane >> 5;
+  const i32x4* kl = reinterpret_cast<const i32x4*>(sbn);
+  const f32x4* kdl = reinterpret_cast<const f32x4*>(sb + St::offKd);
+  const float bias = -m_ref;
+  bf16x8 vf[kPV];
+#pragma unroll
+  for (int i = 0; i < kVAhead; ++i) vf[i] = vf0[i];
+  i32x4 kf[2][NC];
+  f32x4 kd4[8];
+  float u[2][16];
+  bf16x8 pn[2][2];
+  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // P.V MFMAs [pv_of(g), pv_of(g + 1)) belong to group g; S^T's half 0 to groups
+  // 2..5, half 1 to groups 6..9
+  auto pv_of = [](int g) constexpr { return (g >= 6 ? 6 + g : 2 * g) * kPV / 16; };
+  auto qk_of = [](int g) constexpr { return ((g >= 6 ? g - 6 : g - 2) * kQKh + 3) / 4; };  // first of group g's half
+  auto read_kd = [&](int x) __attribute__((always_inline)) {  // K scales of half x / 4, keys 8 (x % 4) ..
+    if constexpr (GRAN == kGRAN_TOKEN)
+      kd4[x] = kdl[8 * (x >> 2) + 2 * (x & 3) + h];
+    else
+      kd4[x] = f32x4{kd_blk, kd_blk, kd_blk, kd_blk};
+  };
+  auto read_k = [&](int b, int m) __attribute__((always_inline)) {  // operands of S^T MFMA m of half b
+    constexpr int per = NC / kQKh;
+#pragma unroll
+    for (int c = per * m; c < per * m + per; ++c) kf[b][c] = kl[(b * NC + c) * 64 + lane];
+  };
+  auto qk_mfma = [&](int b, int m) __attribute__((always_inline)) {
+    auto& acc = b ? s1 : s0;
+    if constexpr (QK == kQK_INT8) {
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[b][m], qf[m], m == 0 ? i32x16{0} : acc, 0, 0, 0);
+    } else {
+      const int c = 2 * m;
+      const i32x8 bq = {qf[c][0], qf[c][1], qf[c][2], qf[c][3], qf[c + 1][0], qf[c + 1][1], qf[c + 1][2], qf[c + 1][3]};
+      const i32x8 ka = {kf[b][c][0],     kf[b][c][1],     kf[b][c][2],     kf[b][c][3],
+                        kf[b][c + 1][0], kf[b][c + 1][1], kf[b][c + 1][2], kf[b][c + 1][3]};
+      acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ka, bq, m == 0 ? f32x16{0} : acc, 0, 0, 0, 0, 0, 0);
+    }
+  };
+  auto convert = [&](int b, int j) __attribute__((always_inline)) {
+    const auto& s = b ? s1 : s0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[b][4 * j + i] = (float)s[4 * j + i] * kd4[4 * b + j][i];
+  };
+  auto exps = [&](int b, int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = 4 * j + i;
+      const float pr = __builtin_amdgcn_exp2f(fmaf(u[b][e], wt, bias));
+      ls[i] += pr;
+      pn[b][e >> 3][e & 7] = (__bf16)pr;
+    }
+  };
+  read_kd(0);
+  read_kd(1);
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int half = g >= 6;
+#pragma unroll
+    for (int i = pv_of(g); i < pv_of(g + 1); ++i)
+      o[i % NC] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pb[i / NC >> 1][i / NC & 1], vf[i], o[i % NC], 0, 0, 0);
+    if (g >= 2) {
+#pragma unroll
+      for (int m = qk_of(g); m < (g == 5 || g == 9 ? kQKh : qk_of(g + 1)); ++m) qk_mfma(half, m);
+    }
+    // the next group's operands
+#pragma unroll
+    for (int i = pv_of(g + 1); i < pv_of(g + 2 > kGroups ? kGroups : g + 2); ++i)
+      if (i >= kVAhead) vf[i] = v_frag<D>(sbp, lane, i);
+    if (g + 1 >= 2 && g + 1 < kGroups) {
+#pragma unroll
+      for (int m = qk_of(g + 1); m < (g + 1 == 5 || g + 1 == 9 ? kQKh : qk_of(g + 2)); ++m) read_k(g + 1 >= 6, m);
+    }
+    if (g == 0) {
+      read_kd(2);
+      read_kd(3);
+    }
+    if (g >= 1 && g < 5) read_kd(3 + g);
+    if (g < 2) {
+      convert(0, 2 * g);
+      convert(0, 2 * g + 1);
+    } else if (g < 6) {
+      exps(0, g - 2);
+      convert(1, g - 2);
+    } else {
+      exps(1, g - 6);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const float sum = (ls[0] + ls[1]) + (ls[2] + ls[3]);
+  // 2^kTau: no score of the lane above m_ref + kTau
+  if (__any(!(sum <= 256.0f))) return softmax_bf16(u, wt, m_ref, l_acc, pb, alpha);
+  l_acc += sum;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) pb[b][tt] = pn[b][tt];
+  return false;
+}
+
 // The per-tile work of one wave in the general loop, as straight-line code
 // for the scheduler: scores of tile t from s0/s1, the next tile's S^T into
 // s0/s1 (both halves issued first, as two interleaved MFMA chains, so the
@@ -958,8 +1096,15 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     // vector work covers their LDS latency (the barrier waits for every LDS
     // access in flight)
     PvFrags pf0;
+    bf16x8 vf_p[kVAhead];  // bf16: its first V fragments
     auto prefetch_pending = [&]() __attribute__((always_inline)) {
-      if constexpr (PV == kPV_FP8) pf0 = pv_load<D>(sp(stage), lane, 0);  // the tile about to become pending
+      // the tile about to become pending
+      if constexpr (PV == kPV_FP8) {
+        pf0 = pv_load<D>(sp(stage), lane, 0);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kVAhead; ++i) vf_p[i] = v_frag<D>(sp(stage), lane, i);
+      }
     };
     float u[2][16];
     auto softmax_p = [&]() __attribute__((always_inline)) {
@@ -1002,15 +1147,20 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     auto iteration = [&]() __attribute__((always_inline)) {
       SAGE_PHASE(0);  // loop overhead since the last iteration's end
       issue_loads();
-      const uint8_t* sb = sp(stage);
-      const uint8_t* sbp = sp(stage_p);
-      const float kdb = kd_block(t);
-      dump(t, s0, s1);
-      auto scores = [&](int b_, float (&u_)[16]) __attribute__((always_inline)) {
-        half_scores<D, QK, PV, GRAN, false, kC0Start>(sb, b_ ? s1 : s0, b_, h, kdb, 64, false, dq, u_);
-      };
-      pending_move();
-      if constexpr (PV == kPV_FP8) {
+      if constexpr (PV == kPV_BF16) {
+        dump(t, s0, s1);
+        pending_move();
+        move_p = tile_bf16<D, QK, GRAN>(sp(stage), sp(stage_p), sp(next_stage(stage, 1)), qf, lane, kd_block(t), s0,
+                                        s1, o, vf_p, pb_p, w, m_ref, l_acc, alpha_p);
+        prefetch_pending();
+      } else {
+        const uint8_t* sb = sp(stage);
+        const uint8_t* sbp = sp(stage_p);
+        const float kdb = kd_block(t);
+        dump(t, s0, s1);
+        auto scores = [&](int b_, float (&u_)[16]) __attribute__((always_inline)) {
+          half_scores<D, QK, PV, GRAN, false, kC0Start>(sb, b_ ? s1 : s0, b_, h, kdb, 64, false, dq, u_);
+        };
         f32x16 p0, p1;
         f32x32 rv;
         pv_issue_f<D>(pf0, pa_p, rsc_p, p0, p1, rv);
@@ -1026,40 +1176,26 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
           scores(1, u[1]);
           pv_accum(o, 2, p0, p1, rv);
         }
-      } else {
-        // bf16: the first chunk pair's products under the score conversion
-        // (int8 QK, whose conversion is longer), the rest under the softmax
-        if constexpr (QK == kQK_INT8) pv_bf16_pair<D>(sbp, pb_p, lane, 0, o);
-        scores(0, u[0]);
-        scores(1, u[1]);
-      }
-      if constexpr (PV == kPV_FP8 && QK == kQK_FP8 && D == 128) {
-        // fp8 QK, D = 128: the frame decision ends a scheduling region (its
-        // rare O rescale is a branch); the next tile's S^T goes after it,
-        // among the exp / pack work of this tile (A/B at 1x30x4416x128
-        // fp8/fp8: 234.7 -> 230.7 us and 240.3 -> 235.7 us; with int8 QK the
-        // same order measured 247.7 -> 250.8 us: the other wave of the SIMD
-        // already covers the QK^T burst)
-        prefetch_pending();
-        const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
-        softmax_fp8_exp_qk<D>(u, w, bm, m_ref, l_acc, pa_p, rsc_p, sp(next_stage(stage, 1)), qf, lane, s0, s1);
-      } else {
-        SAGE_PHASE(1);  // the pending product and this tile's score conversion
-        qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
-        if constexpr (PV == kPV_BF16) {
-          if constexpr (QK != kQK_INT8) pv_bf16_pair<D>(sbp, pb_p, lane, 0, o);
-          if constexpr (NP == 2) pv_bf16_pair<D>(sbp, pb_p, lane, 2, o);
-        }
-        SAGE_PHASE(2);  // the next tile's QK^T issue
-        prefetch_pending();
-        if constexpr (PV == kPV_FP8) {
+        if constexpr (QK == kQK_FP8 && D == 128) {
+          // fp8 QK, D = 128: the frame decision ends a scheduling region (its
+          // rare O rescale is a branch); the next tile's S^T goes after it,
+          // among the exp / pack work of this tile (A/B at 1x30x4416x128
+          // fp8/fp8: 234.7 -> 230.7 us and 240.3 -> 235.7 us; with int8 QK the
+          // same order measured 247.7 -> 250.8 us: the other wave of the SIMD
+          // already covers the QK^T burst)
+          prefetch_pending();
+          const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
+          softmax_fp8_exp_qk<D>(u, w, bm, m_ref, l_acc, pa_p, rsc_p, sp(next_stage(stage, 1)), qf, lane, s0, s1);
+        } else {
+          SAGE_PHASE(1);  // the pending product and this tile's score conversion
+          qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
+          SAGE_PHASE(2);  // the next tile's QK^T issue
+          prefetch_pending();
           const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
           SAGE_PHASE(3);  // row max and frame decision
           softmax_fp8_exp(u, w, bm, m_ref, l_acc, pa_p, rsc_p);
-        } else {
-          softmax_p();
+          SAGE_PHASE(4);  // exp, row sums, P packing
         }
-        SAGE_PHASE(4);  // exp, row sums, P packing
       }
       stage_p = stage;
       publish();

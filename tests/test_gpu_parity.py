@@ -451,3 +451,25 @@ def test_split_items_merged_in_kernel_as_by_merge_kernel(cuda, monkeypatch, B, H
         torch.cuda.synchronize()
         _assert_bits_equal(out, want, f"out, call {i}")
         _assert_bits_equal(lse, want_lse, f"lse, call {i}")
+
+
+@pytest.mark.parametrize("qk", ["int8", "fp8"])
+@pytest.mark.parametrize("N", [64, 65, 128, 192, 250, 320, 500])
+def test_bf16_loop_without_row_max(cuda, N, qk):
+    """The pipelined bf16 loop exponentiates in the frame it has and forms the
+    row max only where a lane's sum of P exceeds 2^8: tile counts around the
+    peeled first and last tiles, with scores that rise along the keys by more
+    than 8 log2 units (the full softmax must take over) and, for D = 64, by more
+    than 128 (P overflows to infinity first).  One row's output follows a few
+    keys' V here, where one bf16 step is above the tight bound with fp8 QK
+    (test_frame_moves_inside_the_loop); the reference-scheme bounds hold."""
+    SA = _sa()
+    D = 64 if N % 64 else 128
+    q, k, v = _sharp_inputs(D, N, 1, 2, seed=200 + N)
+    if D == 64:
+        u = torch.randn(D, generator=torch.Generator().manual_seed(200 + N))
+        k = (k.float() + torch.linspace(0, 60, N).view(1, 1, N, 1) * (u / u.norm())).bfloat16()
+    print(f"bf16 loop N={N} D={D} {qk}", flush=True)
+    out, lse = SA.sage_forward(q.to(cuda), k.to(cuda), v.to(cuda), qk=qk, pv="bf16")
+    torch.cuda.synchronize()
+    _compare(out, lse, q, k, v, qk, "bf16", "token", tight=False)
