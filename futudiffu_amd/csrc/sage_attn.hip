@@ -1345,18 +1345,18 @@ __device__ __forceinline__ void store_partial_coherent(float* slot, const f32x16
 // operations of merge_split_kernel in the same order (so the same bits).  The
 // partials are read by agent-scope relaxed atomic loads (sc1), issued after
 // this piece's arrival was counted behind every other piece's, whose stores
-// had completed before they counted.  fac: LDS [8][128] floats.
+// had completed before they counted.  The item's slots are split_parts apart
+// from the next item's; its first `parts` are in use.  fac: LDS [8][128] floats.
 template <int D>
-__device__ __forceinline__ void merge_pieces(const AttnParams& p, int64_t si, float* fac) {
+__device__ __forceinline__ void merge_pieces(const AttnParams& p, int64_t si, int parts, float* fac) {
   constexpr int NC = D / 32;
   constexpr int kMaxParts = 8;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, h = lane >> 5, r = lane & 31;
-  const int parts = p.split_parts;
   const int nq = (int)(p.np / kRowsPerWG);
   const int64_t pos = p.n_whole + si;
   const int bh = (int)(pos / nq), qt = (int)(pos % nq);
   const int64_t q0 = (int64_t)qt * kRowsPerWG + 32 * w;
-  const uint32_t* slots = reinterpret_cast<const uint32_t*>(p.part + si * parts * kPartFloats<D>);
+  const uint32_t* slots = reinterpret_cast<const uint32_t*>(p.part + si * p.split_parts * kPartFloats<D>);
   auto ld = [](const uint32_t* a) __attribute__((always_inline)) {
     return __uint_as_float(__hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   };
@@ -1420,6 +1420,47 @@ __device__ __forceinline__ void merge_pieces(const AttnParams& p, int64_t si, fl
     }
 }
 
+// The tile-mask row of a work item, and what the item needs to know of it: 64
+// tiles at a time, a byte per lane and a ballot (every lane of a wave returns
+// the same).
+__device__ __forceinline__ const uint8_t* mask_row(const AttnParams& p, int bh, int qt) {
+  return p.tile_mask + (int64_t)bh * p.mask_stride_z + (int64_t)qt * p.mask_nkv;
+}
+__device__ __forceinline__ uint64_t active_64(const uint8_t* row, int nt, int t) {
+  const int i = t + (int)(threadIdx.x & 63);
+  return __ballot(i < nt && row[min(i, nt - 1)] != 0);
+}
+// (first active tile, one past the last); (nt, 0) with none
+__device__ __forceinline__ int2 active_ends(const uint8_t* row, int nt) {
+  int2 e = make_int2(nt, 0);
+  for (int t = 0; t < nt; t += 64) {
+    const uint64_t m = active_64(row, nt, t);
+    if (m != 0) {
+      e.x = min(e.x, t + __builtin_ctzll(m));
+      e.y = t + 64 - __builtin_clzll(m);
+    }
+  }
+  return e;
+}
+__device__ __forceinline__ int active_count(const uint8_t* row, int nt) {
+  int n = 0;
+  for (int t = 0; t < nt; t += 64) n += __builtin_popcountll(active_64(row, nt, t));
+  return n;
+}
+// the active tile with k active ones before it; nt if there is none
+__device__ __forceinline__ int nth_active(const uint8_t* row, int nt, int k) {
+  for (int t = 0; t < nt; t += 64) {
+    uint64_t m = active_64(row, nt, t);
+    const int n = __builtin_popcountll(m);
+    if (k < n) {
+      for (; k > 0; --k) m &= m - 1;
+      return t + __builtin_ctzll(m);
+    }
+    k -= n;
+  }
+  return nt;
+}
+
 template <int D, int QK, int PV, int GRAN, int MASK, bool DUMP = false>
 __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
   using SM = Smem<D, PV>;
@@ -1431,13 +1472,17 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
 
   int bh, qt;
   bool skip_listed = false;  // document ids: this workgroup leaves a listed split query tile to the first ones
-  if constexpr (MASK == 0) {
-    // Unmasked: items in head-major order.  Workgroups [0, n_whole) take whole
-    // items, dealt to XCDs (workgroup i runs on XCD i % 8) in contiguous
-    // ranges so that an XCD's resident workgroups share K/V tiles in its L2.
-    // Later workgroups, dispatched last, take the pieces of the split items
-    // and leave partials; the last piece of an item to arrive merges them
-    // (merge_pieces), or merge_split_kernel does after the launch.
+  if constexpr ((MASK & 2) == 0) {
+    // Without document ids: items in head-major order.  Workgroups [0,
+    // n_whole) take whole items, dealt to XCDs (workgroup i runs on XCD i % 8)
+    // in contiguous ranges so that an XCD's resident workgroups share K/V
+    // tiles in its L2.  Later workgroups, dispatched last, take the pieces of
+    // the split items and leave partials; the last piece of an item to arrive
+    // merges them (merge_pieces), or merge_split_kernel does after the launch
+    // (unmasked launches only).  A tile-masked item's pieces are equal shares
+    // of its active tiles, kMinPiece at least: it uses only as many of its
+    // workgroups as that gives, the others exit.
+    constexpr int kMinPiece = 4;
     const int64_t b = blockIdx.x;
     if (b >= p.n_whole) {
       const int64_t c = b - p.n_whole;
@@ -1446,10 +1491,24 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
       const int part = (int)(c % p.split_parts);
       bh = (int)(pos / nq);
       qt = (int)(pos % nq);
-      const int t0 = (int)((int64_t)part * p.nt / p.split_parts);
-      const int t1 = (int)((int64_t)(part + 1) * p.nt / p.split_parts);
-      item_tiles<D, QK, PV, GRAN, 0, DUMP>(p, smem, bh, qt, t0, t1, o, m_ref, l_acc);
-      if (p.merge_ctr == nullptr) {
+      int t0, t1, parts = p.split_parts;
+      if constexpr (MASK == 1) {
+        const uint8_t* row = mask_row(p, bh, qt);
+        const int count = active_count(row, p.nt);
+        parts = max(1, min(parts, count / kMinPiece));
+        if (part >= parts) return;
+        t0 = nth_active(row, p.nt, (int)((int64_t)part * count / parts));
+        t1 = part + 1 < parts ? nth_active(row, p.nt, (int)((int64_t)(part + 1) * count / parts)) : p.nt;
+      } else {
+        t0 = (int)((int64_t)part * p.nt / p.split_parts);
+        t1 = (int)((int64_t)(part + 1) * p.nt / p.split_parts);
+      }
+      item_tiles<D, QK, PV, GRAN, MASK, DUMP>(p, smem, bh, qt, t0, t1, o, m_ref, l_acc);
+      if (MASK == 1 && parts == 1) {  // too few active tiles to share
+        store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
+        return;
+      }
+      if (MASK == 0 && p.merge_ctr == nullptr) {
         store_partial<D>(p.part + c * kPartFloats<D>, o, m_ref, l_acc);
         return;
       }
@@ -1457,39 +1516,48 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
       wait_vmem();  // this piece's partial is at the coherence point before it counts
       __syncthreads();
       int* last = reinterpret_cast<int*>(smem);
-      if (threadIdx.x == 0) *last = arrive_last(p.merge_ctr + si, p.merge_tag, p.split_parts) ? 1 : 0;
+      if (threadIdx.x == 0) *last = arrive_last(p.merge_ctr + si, p.merge_tag, parts) ? 1 : 0;
       __syncthreads();
       if (*last == 0) return;
       __syncthreads();  // every wave has read the decision before the factors reuse the LDS
-      merge_pieces<D>(p, si, reinterpret_cast<float*>(smem));
+      merge_pieces<D>(p, si, parts, reinterpret_cast<float*>(smem));
       if (threadIdx.x == 0)
         __hip_atomic_store(p.merge_ctr + si, p.merge_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;
     }
-    const int x = (int)(b % 8);
-    const int64_t local = b / 8, per = p.n_whole / 8, rem = p.n_whole % 8;
-    const int64_t pos = x * per + (x < rem ? x : rem) + local;
-    bh = (int)(pos / nq);
-    qt = (int)(pos % nq);
-  } else {
-    const int id = blockIdx.x, total = gridDim.x;
-    if constexpr ((MASK & 2) != 0) {
-      // the first heavy_max * h workgroups: head id % h of listed split query
-      // tile id / h (doc_prefix_kernel); the others run the usual order and
-      // leave the listed items to them
-      const int reserved = p.heavy_max * p.h;
-      if (id < reserved) {
-        const int e = id / p.h;
-        if (e >= load_uniform(&p.heavy[0].x, 0)) return;
-        const int it = load_uniform(&p.heavy[1 + e].x, 0);
-        bh = (it / nq) * p.h + id % p.h;
-        qt = it % nq;
-      } else {
-        item_of(id - reserved, total - reserved, p.bh, nq, p.light_last, bh, qt);
-        skip_listed = true;
-      }
+    if (MASK == 0 || p.split_parts > 1) {
+      const int x = (int)(b % 8);
+      const int64_t local = b / 8, per = p.n_whole / 8, rem = p.n_whole % 8;
+      const int64_t pos = x * per + (x < rem ? x : rem) + local;
+      bh = (int)(pos / nq);
+      qt = (int)(pos % nq);
     } else {
-      item_of(id, total, p.bh, nq, p.light_last, bh, qt);
+      item_of((int)b, (int)gridDim.x, p.bh, nq, p.light_last, bh, qt);
+    }
+    if constexpr (MASK == 1) {
+      // the loop starts at the first active tile and ends after the last:
+      // walking the others one scalar load at a time took 10 us per short
+      // document of the packed 6912-token batch
+      const int2 ends = active_ends(mask_row(p, bh, qt), p.nt);
+      item_tiles<D, QK, PV, GRAN, MASK, DUMP>(p, smem, bh, qt, ends.x, ends.y, o, m_ref, l_acc);
+      store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
+      return;
+    }
+  } else {
+    // the first heavy_max * h workgroups: head id % h of listed split query
+    // tile id / h (doc_prefix_kernel); the others run the usual order and
+    // leave the listed items to them
+    const int id = blockIdx.x, total = gridDim.x;
+    const int reserved = p.heavy_max * p.h;
+    if (id < reserved) {
+      const int e = id / p.h;
+      if (e >= load_uniform(&p.heavy[0].x, 0)) return;
+      const int it = load_uniform(&p.heavy[1 + e].x, 0);
+      bh = (it / nq) * p.h + id % p.h;
+      qt = it % nq;
+    } else {
+      item_of(id - reserved, total - reserved, p.bh, nq, p.light_last, bh, qt);
+      skip_listed = true;
     }
   }
   if (!item_tiles<D, QK, PV, GRAN, MASK, DUMP>(p, smem, bh, qt, 0, p.nt, o, m_ref, l_acc, skip_listed)) return;
@@ -1574,10 +1642,9 @@ __global__ void __launch_bounds__(256) merge_split_kernel(AttnParams p) {
 template <int D, int QK, int PV, int GRAN>
 hipError_t launch_attn_g(int mask, const AttnParams& p, hipStream_t st) {
   const int64_t items = (int64_t)p.bh * (p.np / kRowsPerWG);
-  const int64_t n_split = mask == 0 ? items - p.n_whole : 0;
+  const int64_t n_split = items - p.n_whole;  // 0 with document ids
   // with document ids the first heavy_max * h workgroups take the listed split query tiles
-  const dim3 grid((unsigned)(mask == 0 ? p.n_whole + n_split * p.split_parts
-                                       : items + ((mask & 2) ? (int64_t)p.heavy_max * p.h : 0)));
+  const dim3 grid((unsigned)(p.n_whole + n_split * p.split_parts + ((mask & 2) ? (int64_t)p.heavy_max * p.h : 0)));
   // the accumulator dump exists for the per-token, unmasked kernels
   constexpr bool kDumpable = GRAN == kGRAN_TOKEN;
   if (p.s_dump != nullptr) {
@@ -1714,7 +1781,7 @@ hipError_t launch_attn(int qk, int pv, int gran, int mask, const AttnParams& p, 
   return hipErrorInvalidValue;
 }
 
-AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked) {
+AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked, size_t limit) {
   const int64_t np = padded_len(n);
   const int64_t nt = (n + 63) / 64;
   const int64_t items = b * h * (np / kRowsPerWG);
@@ -1725,7 +1792,14 @@ AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool ma
   // list of split query tiles (a count and kHeavyMax entries)
   w.heavy_off = (size_t)(b * (nt + np / 32 + np / 128 + np / 128)) * sizeof(int4);
   w.part_off = (w.heavy_off + (size_t)(1 + kHeavyMax) * sizeof(int4) + 255) & ~(size_t)255;
-  const int64_t split_items = !masked && w.split.parts > 1 ? items - w.split.whole : 0;
+  int64_t split_items = !masked && w.split.parts > 1 ? items - w.split.whole : 0;
+  if (limit != 0 && split_items > 0) {
+    const int64_t item_bytes = w.split.parts * (128 * d + 512) * (int64_t)sizeof(float) + (int64_t)sizeof(uint64_t);
+    const int64_t room = (int64_t)limit - (int64_t)w.part_off;
+    split_items = room > 0 ? std::min(split_items, room / item_bytes) : 0;
+    w.split.whole = items - split_items;
+    if (split_items == 0) w.split.parts = 1;
+  }
   const int64_t pieces = split_items * w.split.parts;
   // then one 8-byte arrival counter per split item (in-kernel merge)
   w.ctr_off = w.part_off + (size_t)pieces * (size_t)(128 * d + 512) * sizeof(float);

@@ -313,8 +313,19 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   if (doc_ids) mask |= 2;
   sage::AttnParams p;
   memset(&p, 0, sizeof(p));
-  // masked launches cut no item, so they need no partial slots
-  const sage::AttnWorkspace ws = sage::attn_workspace(b, h, n, d, mask != 0);
+  // Masked launches need no partial slots.  With a tile mask alone and a
+  // workspace that has room for them all the same (sage_attn_workspace_bytes,
+  // or the scratch of the allocation-free entry point), the last items are
+  // split as in an unmasked launch: the production op is always masked, and at
+  // 1x30x4416 its 1050 items leave a third round of 26.  The pieces' slots stay
+  // within that scratch, so every entry point cuts the same items.
+  sage::AttnWorkspace ws = sage::attn_workspace(b, h, n, d, mask != 0);
+  bool masked_split = false;
+  if (mask == 1 && merge_in_kernel()) {
+    const sage::AttnWorkspace split = sage::attn_workspace(b, h, n, d, false, SAGE_NOALLOC_SCRATCH_BYTES);
+    masked_split = workspace_bytes >= split.bytes;
+    if (masked_split) ws = split;
+  }
   if (!workspace || workspace_bytes < ws.bytes)
     return fail(SAGE_ERR_WORKSPACE, "workspace of %zu bytes needed, got %zu", ws.bytes, workspace_bytes);
   if (!aligned16(workspace)) return fail(SAGE_ERR_ALIGN, "workspace must be 16-byte aligned");
@@ -355,10 +366,10 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   p.bh = (int)(b * h);
   p.nt = (int)nkv;
   p.light_last = (nq > 1 && n - (nq - 1) * 128 <= 64) ? 1 : 0;
-  // unmasked launches cut the items of the last, partial dispatch round
+  // cut the items of the last, partial dispatch round
   p.n_whole = (int)(b * h * nq);
   p.split_parts = 1;
-  if (mask == 0) {
+  if (mask == 0 || masked_split) {
     p.n_whole = (int)ws.split.whole;
     p.split_parts = ws.split.parts;
     p.part = reinterpret_cast<float*>(wsp + ws.part_off);

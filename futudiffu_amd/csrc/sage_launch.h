@@ -41,8 +41,9 @@ struct AttnParams {
   int bh;          // B * H
   int nt;          // key tiles: ceil(N / 64)
   int light_last;  // last 128-row query tile holds <= 64 rows: schedule those items last
-  // unmasked launches: the items past n_whole (in schedule order) are cut into
-  // split_parts key-tile ranges whose partials a second kernel merges
+  // without document ids: the items past n_whole (in schedule order) are cut
+  // into (with a tile mask, at most) split_parts key-tile ranges, merged by the
+  // last range to finish or, unmasked, by a second kernel
   int n_whole;
   int split_parts;
   float* part;  // (items - n_whole) * split_parts slots of kPartFloats<D> floats
@@ -175,8 +176,9 @@ struct AttnWorkspace {
   TailSplit split;
 };
 // `masked`: a launch with a tile mask or document ids, which splits no item
-// and so needs no partial slots
-AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false);
+// and so needs no partial slots.  `limit` (0: none): split only as many of the
+// tail items as keep `bytes` within it, the others stay whole.
+AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false, size_t limit = 0);
 size_t attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false);
 hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t pad_fill, uint8_t* mask,
                             hipStream_t st);

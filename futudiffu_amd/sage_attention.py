@@ -281,7 +281,7 @@ def attn_from_quantized(qz: SageQuantized, B: int, H: int, *, block_mask: Tensor
         if doc_ids.shape != (B, N):
             raise ValueError(f"doc_ids must be [B, N] = [{B}, {N}], got {tuple(doc_ids.shape)}")
         doc_ids = doc_ids.to(device=dev, dtype=torch.int32).contiguous()
-    if bm is None and doc_ids is None:
+    if doc_ids is None:  # with a tile mask too: room for the split tail items
         wsb = int(lib.sage_attn_workspace_bytes(B, H, N, D))
     else:
         wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))

@@ -180,9 +180,11 @@ int sage_quantize_from_qkv(const void* qkv, const float* q_norm_w, const float* 
 size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
 /* Bytes of device workspace a sage_attn_fwd launch with a tile_mask or
- * doc_ids needs: the summaries only, since masked launches split no item
- * (a few KB; 7 KB for the packed 1x30x6912 batch).  No reference
- * counterpart. */
+ * doc_ids needs: the summaries only (a few KB; 7 KB for the packed 1x30x6912
+ * batch).  A tile-masked launch without doc_ids that is given room for them
+ * (sage_attn_workspace_bytes) splits its last items like an unmasked one: as
+ * many of them as keep the partials within SAGE_NOALLOC_SCRATCH_BYTES, so
+ * sage_attn_fwd_noalloc cuts the same ones.  No reference counterpart. */
 size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
 /* Fused attention forward over pre-quantized operands.

@@ -155,3 +155,56 @@ def test_packed_tile_mask_equal_serial_images(cuda, qk, pv):
                                f"max {(got.float() - o1.float()).abs().max().item():.3g}")
         assert torch.equal(lse.view(B * H, n)[:, sl].cpu(), l1.cpu()), f"segment at {off}: LSE differs"
         off += s
+
+
+@pytest.mark.parametrize("pv,D", [("bf16", 128), ("fp8", 128), ("bf16", 64)])
+def test_tile_masked_tail_split(cuda, pv, D):
+    """65 heads of 1000 tokens are 520 items: with room in the workspace the
+    last 8 run as up to four shares of their active tiles each.  A 3D mask
+    gives the split items 0 to 16 active tiles, scattered ones among them; the
+    results agree with the unsplit launch (a workspace of the masked size) to
+    the rounding of P in another frame, rows without a key give 0 and -inf,
+    and two heads match the oracle."""
+    from futudiffu_amd import _lib
+    from futudiffu_amd import sage_attention as SA
+    B, H, N = 1, 65, 1000
+    nq, nkv = 8, 16
+    lib = _lib.load()
+    q, k, v = O.make_inputs(B, H, N, D, seed=91)
+    g = torch.Generator().manual_seed(92)
+    mask = (torch.rand(H, nq, nkv, generator=g) < 0.5).to(torch.uint8)
+    for i, count in enumerate([0, 1, 3, 4, 7, 8, 15, 16]):  # the last head's items are the split ones
+        mask[H - 1, i] = 0
+        mask[H - 1, i, torch.randperm(nkv, generator=g)[:count]] = 1
+    print(f"masked tail split int8/{pv} D={D}", flush=True)
+    qz = SA.quantize_qkv(q.to(cuda), k.to(cuda), v.to(cuda), qk="int8", pv=pv)
+    mg = mask.to(cuda)
+    out, lse = SA.attn_from_quantized(qz, B, H, block_mask=mg)
+    out2, lse2 = SA.attn_from_quantized(qz, B, H, block_mask=mg)
+    wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))
+    assert wsb < int(lib.sage_attn_workspace_bytes(B, H, N, D))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+    o1 = torch.empty_like(out)
+    l1 = torch.empty_like(lse)
+    _lib.check(lib.sage_attn_fwd(
+        qz.q_codes.data_ptr(), qz.q_scale.data_ptr(), qz.k_codes.data_ptr(), qz.k_scale.data_ptr(),
+        qz.v_op.data_ptr(), SA._ptr(qz.v_scale), B, H, N, D, 0, SA._PV[pv], 0, mg.data_ptr(), nq * nkv, nq, nkv, None,
+        ws.data_ptr(), wsb, o1.data_ptr(), 0, l1.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)
+    assert torch.equal(out[:, :H - 1], o1[:, :H - 1]) and torch.equal(lse[:H - 1], l1[:H - 1])
+    assert not out[0, H - 1, :128].float().any() and torch.isinf(lse[H - 1, :128]).all()
+    assert (out.float() - o1.float()).abs().max().item() <= 8e-3
+    fin = torch.isfinite(l1)
+    assert torch.equal(fin, torch.isfinite(lse)) and (lse[fin] - l1[fin]).abs().max().item() <= 1e-4
+    for hh in (0, H - 1):
+        sl = slice(hh, hh + 1)
+        live = mask[hh].sum(1) > 0
+        m1 = mask[hh:hh + 1].clone()
+        m1[0, ~live] = 1
+        want, wl, _ = O.sage_forward(q[:, sl], k[:, sl], v[:, sl], 1.0 / math.sqrt(D), "int8", pv, "token", True, m1)
+        see = live.repeat_interleave(128)[:N]
+        got = out[:, sl].float().cpu()[:, :, see]
+        assert (got - want.float()[:, :, see]).abs().max().item() <= 2e-2
+        assert O.cosine(got, want[:, :, see]) >= 0.999
+        assert (lse[hh].cpu()[see] - wl[0][see]).abs().max().item() <= 2e-3
