@@ -65,6 +65,14 @@ def _fake_merged_heads(q: Tensor) -> tuple[Tensor, Tensor]:
     return q.new_empty(B, N, H * D), q.new_empty(B * H, N, dtype=torch.float32)
 
 
+def _grad_of(grad: Tensor | None, out: Tensor) -> Tensor:
+    """The incoming gradient of ``out``.  The formulas ask for no materialized
+    gradients, which would fill an LSE-sized tensor of zeros nobody reads on
+    every backward; a missing gradient of ``out`` itself (only the LSE was
+    used) still counts as zeros."""
+    return torch.zeros_like(out) if grad is None else grad
+
+
 def _to_bhnd(x: Tensor, shape) -> Tensor:
     """[B, N, H*D] -> contiguous [B, H, N, D]."""
     B, H, N, D = shape
@@ -130,6 +138,7 @@ def _fake_fwd_masked(q, k, v, block_mask, sm_scale):
 def _masked_setup_context(ctx, inputs, output):
     q, k, v, block_mask, sm_scale = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)
     ctx.save_for_backward(q, k, v, out, lse, block_mask)
     ctx.sm_scale = sm_scale
     ctx.smooth_k = _sa._SAGE_SMOOTH_K
@@ -137,8 +146,8 @@ def _masked_setup_context(ctx, inputs, output):
 
 def _masked_backward(ctx, grad_out, grad_lse):
     q, k, v, out, lse, block_mask = ctx.saved_tensors
-    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out.contiguous(), block_mask, None, ctx.sm_scale, "int8",
-                                 ctx.smooth_k)
+    grad_out = _grad_of(grad_out, out).contiguous()
+    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out, block_mask, None, ctx.sm_scale, "int8", ctx.smooth_k)
     return dq, dk, dv, None, None
 
 
@@ -159,6 +168,7 @@ def _fake_fwd(q, k, v, sm_scale):
 def _setup_context(ctx, inputs, output):
     q, k, v, sm_scale = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)
     ctx.save_for_backward(q, k, v, out, lse)
     ctx.sm_scale = sm_scale
     ctx.qk = _sa._SAGE_QK_QUANT
@@ -167,8 +177,8 @@ def _setup_context(ctx, inputs, output):
 
 def _backward(ctx, grad_out, grad_lse):
     q, k, v, out, lse = ctx.saved_tensors
-    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out.contiguous(), None, None, ctx.sm_scale, ctx.qk,
-                                 ctx.smooth_k)
+    grad_out = _grad_of(grad_out, out).contiguous()
+    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out, None, None, ctx.sm_scale, ctx.qk, ctx.smooth_k)
     return dq, dk, dv, None
 
 
@@ -194,6 +204,7 @@ def _fake_ext(q, k, v, block_mask, doc_ids, sm_scale, qk, pv, granularity, smoot
 def _ext_setup_context(ctx, inputs, output):
     q, k, v, block_mask, doc_ids, sm_scale, qk, pv, granularity, smooth_k, *rest = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)
     ctx.save_for_backward(q, k, v, out, lse, block_mask, doc_ids)
     ctx.args = (sm_scale, qk, smooth_k, rest[0] if rest else "bhnd")
     ctx.granularity = granularity
@@ -209,6 +220,7 @@ def _ext_backward(ctx, grad_out, grad_lse):
                          f"{ctx.granularity!r}")
     q, k, v, out, lse, block_mask, doc_ids = ctx.saved_tensors
     sm_scale, qk, smooth_k, layout = ctx.args
+    grad_out = _grad_of(grad_out, out)
     if layout == "bnhd":
         out, grad_out = _to_bhnd(out, q.shape), _to_bhnd(grad_out, q.shape)
     dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out.contiguous(), block_mask, doc_ids, sm_scale, qk,
@@ -237,6 +249,7 @@ def _fake_fwd_merged(q, k, v, block_mask, sm_scale):
 
 def _merged_backward(ctx, grad_out, grad_lse):
     q, k, v, out, lse, block_mask = ctx.saved_tensors
+    grad_out = _grad_of(grad_out, out)
     dq, dk, dv = sage_bwd_ext_op(q, k, v, _to_bhnd(out, q.shape), lse, _to_bhnd(grad_out, q.shape), block_mask,
                                  None, ctx.sm_scale, "int8", ctx.smooth_k)
     return dq, dk, dv, None, None
@@ -269,6 +282,7 @@ def _fake_qkv_masked(qkv, q_norm_weight, k_norm_weight, freqs_cis, block_mask, n
 def _qkv_masked_setup(ctx, inputs, output):
     qkv, q_norm_weight, k_norm_weight, freqs_cis, block_mask, n_heads, head_dim, norm_eps, sm_scale = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)
     ctx.save_for_backward(qkv, q_norm_weight, k_norm_weight, freqs_cis, block_mask, out, lse)
     ctx.args = (n_heads, head_dim, norm_eps, sm_scale)
     ctx.smooth_k = _sa._SAGE_SMOOTH_K
@@ -282,6 +296,7 @@ def _qkv_masked_backward(ctx, grad_out, grad_lse):
     n_heads, head_dim, norm_eps, sm_scale = ctx.args
     q, k, v = _sa.qkv_postprocess(qkv, qw, kw, freqs, n_heads, head_dim, norm_eps)
     shape = q.shape
+    grad_out = _grad_of(grad_out, out)
     dq, dk, dv = sage_bwd_ext_op(q, k, v, _to_bhnd(out, shape), lse, _to_bhnd(grad_out, shape), block_mask, None,
                                  sm_scale, "int8", ctx.smooth_k)
     dqkv = _sa.qkv_postprocess_backward(qkv, qw, kw, freqs, dq, dk, dv, n_heads, head_dim, norm_eps)

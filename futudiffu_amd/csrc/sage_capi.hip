@@ -169,6 +169,35 @@ BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
   return w;
 }
 
+// Workspace of sage_forward: the quantization's outputs (sized for per-token
+// scales, the larger granularity), its workspace, the attention's workspace.
+struct ForwardWorkspace {
+  size_t qc, qs, kc, ks, vop, vs, kmean, quant, attn, bytes;
+};
+
+ForwardWorkspace forward_workspace(int64_t b, int64_t h, int64_t n, int64_t d, int pv_kind, bool doc_ids) {
+  const int64_t bh = b * h;
+  const size_t np = (size_t)sage::padded_len(n), rows = (size_t)bh * np;
+  ForwardWorkspace w;
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off = (off + bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  w.qc = take(rows * d);
+  w.qs = take(rows * 4);
+  w.kc = take(rows * d);
+  w.ks = take(rows * 4);
+  w.vop = take(rows * d * (pv_kind == SAGE_PV_FP8 ? 1 : 2));
+  w.vs = take(pv_kind == SAGE_PV_FP8 ? rows / 64 * d * 4 : 0);
+  w.kmean = take((size_t)bh * d * 2);
+  w.quant = take(sage::quant_workspace_bytes(bh, n, d));
+  w.attn = off;
+  w.bytes = off + sage::attn_workspace_bytes(b, h, n, d, doc_ids);
+  return w;
+}
+
 }  // namespace
 
 extern "C" {
@@ -459,6 +488,33 @@ int sage_attn_fwd_noalloc(const void* q_codes, const float* q_scale, const void*
   return attn_fwd_impl(q_codes, q_scale, k_codes, k_scale, v_in, v_scale, b, h, n, d, qk_kind, pv_kind, granularity,
                        tile_mask, mask_stride_z, mask_nq, mask_nkv, doc_ids, ws, SAGE_NOALLOC_SCRATCH_BYTES, out,
                        out_layout, lse, nullptr, "sage_attn_fwd_noalloc", stream);
+}
+
+size_t sage_forward_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int pv_kind, int with_doc_ids) {
+  return forward_workspace(b, h, n, d, pv_kind, with_doc_ids != 0).bytes;
+}
+
+int sage_forward(const void* q, const void* k, const void* v, int64_t b, int64_t h, int64_t n, int64_t d, int qk_kind,
+                 int pv_kind, int granularity, int smooth_k, float sm_scale_log2e, const uint8_t* tile_mask,
+                 int64_t mask_stride_z, int64_t mask_nq, int64_t mask_nkv, const int32_t* doc_ids, void* workspace,
+                 size_t workspace_bytes, void* out, int out_layout, float* lse, hipStream_t stream) {
+  if (b <= 0 || h <= 0) return fail(SAGE_ERR_ARG, "b=%lld and h=%lld must be positive", (long long)b, (long long)h);
+  int st = check_common(b * h, n, d, qk_kind, pv_kind, granularity);
+  if (st) return st;
+  const ForwardWorkspace w = forward_workspace(b, h, n, d, pv_kind, doc_ids != nullptr);
+  if (!workspace || workspace_bytes < w.bytes)
+    return fail(SAGE_ERR_WORKSPACE, "workspace of %zu bytes needed, got %zu", w.bytes, workspace_bytes);
+  if (!aligned16(workspace)) return fail(SAGE_ERR_ALIGN, "workspace must be 16-byte aligned");
+  uint8_t* p = static_cast<uint8_t*>(workspace);
+  float* qs = reinterpret_cast<float*>(p + w.qs);
+  float* ks = reinterpret_cast<float*>(p + w.ks);
+  float* vs = pv_kind == SAGE_PV_FP8 ? reinterpret_cast<float*>(p + w.vs) : nullptr;
+  st = sage_quantize_qkv(q, k, v, b * h, n, d, qk_kind, pv_kind, granularity, smooth_k, sm_scale_log2e, p + w.qc, qs,
+                         p + w.kc, ks, p + w.vop, vs, p + w.kmean, p + w.quant, w.attn - w.quant, stream);
+  if (st) return st;
+  return attn_fwd_impl(p + w.qc, qs, p + w.kc, ks, p + w.vop, vs, b, h, n, d, qk_kind, pv_kind, granularity, tile_mask,
+                       mask_stride_z, mask_nq, mask_nkv, doc_ids, p + w.attn, w.bytes - w.attn, out, out_layout, lse,
+                       nullptr, "sage_forward", stream);
 }
 
 int sage_attn_qk_accumulators(const void* q_codes, const float* q_scale, const void* k_codes, const float* k_scale,

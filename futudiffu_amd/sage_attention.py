@@ -14,10 +14,10 @@ argument meaning and error behaviour) on top of the gfx950 HIP library
 * ``sage_attn_op`` (``futudiffu::sage_attn``) and ``sage_attn_masked_op``
   (``futudiffu::sage_attn_masked``), with autograd -> :664-690, :740-769
 
-Each call runs two kernels on the current stream: ``sage_quantize_qkv``
-(K smoothing + Q/K/V quantization) and ``sage_attn_fwd``.  All outputs and
-temporaries are allocated through the PyTorch caching allocator; nothing
-synchronizes the host.  Variant choice (qk int8/fp8, pv bf16/fp8, scale
+Each forward runs two kernels on the current stream, those of
+``sage_quantize_qkv`` (K smoothing + Q/K/V quantization) and ``sage_attn_fwd``,
+in one library call.  All outputs and temporaries are allocated through the
+PyTorch caching allocator; nothing synchronizes the host.  Variant choice (qk int8/fp8, pv bf16/fp8, scale
 granularity, smoothing, exact doc-id masking) is also available as explicit
 keyword arguments of :func:`sage_forward`, which the module-level
 configuration only supplies defaults for.
@@ -32,6 +32,7 @@ Differences from the reference, all deliberate:
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
@@ -68,7 +69,9 @@ def configure_sage(*, smooth_k: bool = True, qk_quant: str = "fp8", pv_quant: st
 
 
 def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle of torch.cuda.current_stream(device), without the Stream object
+    # (1.9 -> 0.3 us of a 43 us call)
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: Tensor | None) -> int | None:
@@ -134,7 +137,7 @@ def _quant_outputs(BH: int, N: int, D: int, qk: str, pv: str, granularity: str, 
 
 def _fold(sm_scale: float) -> float:
     """``sm_scale*log2(e)`` as the fp32 the kernels receive (sage_attention.py:493-495)."""
-    return float(torch.tensor(sm_scale * _LOG2E, dtype=torch.float32))
+    return ctypes.c_float(sm_scale * _LOG2E).value
 
 
 def quantize_qkv(q: Tensor, k: Tensor, v: Tensor, sm_scale: float | None = None, *,
@@ -262,6 +265,14 @@ def _norm_mask(block_mask: Tensor | None, BH: int, N: int, device) -> tuple[Tens
     return bm, stride_z, nq, nkv
 
 
+def _norm_doc_ids(doc_ids: Tensor | None, B: int, N: int, device) -> Tensor | None:
+    if doc_ids is None:
+        return None
+    if doc_ids.shape != (B, N):
+        raise ValueError(f"doc_ids must be [B, N] = [{B}, {N}], got {tuple(doc_ids.shape)}")
+    return doc_ids.to(device=device, dtype=torch.int32).contiguous()
+
+
 def attn_from_quantized(qz: SageQuantized, B: int, H: int, *, block_mask: Tensor | None = None,
                         doc_ids: Tensor | None = None, out: Tensor | None = None,
                         lse: Tensor | None = None, out_layout: str = "bhnd") -> tuple[Tensor, Tensor]:
@@ -277,10 +288,7 @@ def attn_from_quantized(qz: SageQuantized, B: int, H: int, *, block_mask: Tensor
     dev = qz.q_codes.device
     out_shape = (B, H, N, D) if out_layout == "bhnd" else (B, N, H * D)
     bm, stride_z, nq, nkv = _norm_mask(block_mask, BH, N, dev)
-    if doc_ids is not None:
-        if doc_ids.shape != (B, N):
-            raise ValueError(f"doc_ids must be [B, N] = [{B}, {N}], got {tuple(doc_ids.shape)}")
-        doc_ids = doc_ids.to(device=dev, dtype=torch.int32).contiguous()
+    doc_ids = _norm_doc_ids(doc_ids, B, N, dev)
     if doc_ids is None:  # with a tile mask too: room for the split tail items
         wsb = int(lib.sage_attn_workspace_bytes(B, H, N, D))
     else:
@@ -324,8 +332,26 @@ def sage_forward(q: Tensor, k: Tensor, v: Tensor, sm_scale: float | None = None,
         sm_scale = 1.0 / math.sqrt(D)
     if out_layout not in _LAYOUT:
         raise ValueError(f"out_layout must be one of {sorted(_LAYOUT)}, got {out_layout!r}")
-    qz = quantize_qkv(q, k, v, sm_scale, qk=qk, pv=pv, granularity=granularity, smooth_k=smooth_k)
-    return attn_from_quantized(qz, B, H, block_mask=block_mask, doc_ids=doc_ids, out_layout=out_layout)
+    if granularity not in _GRAN:
+        raise ValueError(f"bad variant qk={qk!r} pv={pv!r} granularity={granularity!r}")
+    # quantize_qkv and attn_from_quantized in one library call over one
+    # workspace: the quantized operands are not returned, and their eight
+    # tensors and the second call were half of the host time of a small call
+    # (1x4x256x64: 43 us of Python and launches around 15 us of kernels)
+    dev = q.device
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    bm, stride_z, nq, nkv = _norm_mask(block_mask, B * H, N, dev)
+    doc_ids = _norm_doc_ids(doc_ids, B, N, dev)
+    lib = _lib.load()
+    wsb = lib.sage_forward_workspace_bytes(B, H, N, D, _PV[pv], doc_ids is not None)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    out = torch.empty((B, H, N, D) if out_layout == "bhnd" else (B, N, H * D), dtype=torch.bfloat16, device=dev)
+    lse = torch.empty((B * H, N), dtype=torch.float32, device=dev)
+    _lib.check(lib.sage_forward(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), B, H, N, D, _QK[qk], _PV[pv], _GRAN[granularity],
+        int(bool(smooth_k)), _fold(sm_scale), _ptr(bm), stride_z, nq, nkv, _ptr(doc_ids), ws.data_ptr(), wsb,
+        out.data_ptr(), _LAYOUT[out_layout], lse.data_ptr(), _stream_handle(dev)))
+    return out, lse
 
 
 def sage_forward_from_qkv(qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: Tensor, freqs_cis: Tensor,
@@ -419,10 +445,7 @@ def sage_backward(q: Tensor, k: Tensor, v: Tensor, out: Tensor, lse: Tensor, dou
     lib = _lib.load()
     BH = B * H
     bm, stride_z, nq, nkv = _norm_mask(block_mask, BH, N, dev)
-    if doc_ids is not None:
-        if doc_ids.shape != (B, N):
-            raise ValueError(f"doc_ids must be [B, N] = [{B}, {N}], got {tuple(doc_ids.shape)}")
-        doc_ids = doc_ids.to(device=dev, dtype=torch.int32).contiguous()
+    doc_ids = _norm_doc_ids(doc_ids, B, N, dev)
     wsb = int(lib.sage_attn_bwd_workspace_bytes(B, H, N, D))
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
     dq, dk, dv = (torch.empty_like(q) for _ in range(3))
@@ -504,6 +527,7 @@ def _sage_attn_op_fake(q, k, v, sm_scale):
 def _legacy_setup_context(ctx, inputs, output):
     q, k, v, sm_scale = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)  # no zeros for the unused LSE gradient
     ctx.save_for_backward(q, k, v, out, lse)
     ctx.sm_scale = sm_scale
     ctx.qk = _SAGE_QK_QUANT
@@ -512,6 +536,7 @@ def _legacy_setup_context(ctx, inputs, output):
 
 def _legacy_backward(ctx, grad_out, grad_lse):
     q, k, v, out, lse = ctx.saved_tensors
+    grad_out = torch.zeros_like(out) if grad_out is None else grad_out
     dq, dk, dv = sage_backward(q, k, v, out, lse, grad_out.contiguous(), ctx.sm_scale, qk=ctx.qk,
                                smooth_k=ctx.smooth_k)
     return dq, dk, dv, None
@@ -536,6 +561,7 @@ def _sage_attn_masked_op_fake(q, k, v, block_mask, sm_scale):
 def _legacy_masked_setup_context(ctx, inputs, output):
     q, k, v, block_mask, sm_scale = inputs
     out, lse = output
+    ctx.set_materialize_grads(False)  # no zeros for the unused LSE gradient
     ctx.save_for_backward(q, k, v, out, lse, block_mask)
     ctx.sm_scale = sm_scale
     ctx.smooth_k = _SAGE_SMOOTH_K
@@ -543,6 +569,7 @@ def _legacy_masked_setup_context(ctx, inputs, output):
 
 def _legacy_masked_backward(ctx, grad_out, grad_lse):
     q, k, v, out, lse, block_mask = ctx.saved_tensors
+    grad_out = torch.zeros_like(out) if grad_out is None else grad_out
     dq, dk, dv = sage_backward(q, k, v, out, lse, grad_out.contiguous(), ctx.sm_scale, block_mask=block_mask,
                                qk="int8", smooth_k=ctx.smooth_k)
     return dq, dk, dv, None, None

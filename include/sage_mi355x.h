@@ -330,6 +330,24 @@ int sage_attn_bwd(const void* q, const void* k, const void* v,
                   void* dq, void* dk, void* dv,
                   hipStream_t stream);
 
+/* sage_quantize_qkv and sage_attn_fwd in one call, the quantized operands kept
+ * in the workspace: the whole forward of the attention op
+ * (sage_attention.py:461-531) from bf16 q, k, v [B, H, N, D] contiguous.
+ * Arguments as in those two; the same kernels, results and status codes.
+ * For callers that do not keep the operands: one allocation and one call where
+ * the pair takes eleven and two. */
+int sage_forward(const void* q, const void* k, const void* v,
+                 int64_t b, int64_t h, int64_t n, int64_t d,
+                 int qk_kind, int pv_kind, int granularity, int smooth_k, float sm_scale_log2e,
+                 const uint8_t* tile_mask, int64_t mask_stride_z, int64_t mask_nq, int64_t mask_nkv,
+                 const int32_t* doc_ids, void* workspace, size_t workspace_bytes,
+                 void* out, int out_layout, float* lse, hipStream_t stream);
+
+/* Bytes of the workspace sage_forward needs (codes, scales, K mean, the V
+ * operand and the workspaces of its two parts). */
+size_t sage_forward_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d,
+                                    int pv_kind, int with_doc_ids);
+
 /* Parity: sage_attn_fwd with per-token scales, no mask and the [B, H, N, D]
  * output, which also stores the QK^T accumulators its own loop consumes, tile
  * by tile, as that loop forms them (the split tail pieces included): s_out

@@ -128,3 +128,37 @@ def test_legacy_masked_op_matches_oracle(cuda, sa):
     torch.cuda.synchronize()
     for name, a, b in zip(("dq", "dk", "dv"), (dq, dk, dv), want):
         assert torch.equal(a.contiguous().view(torch.int16), b.view(torch.int16)), f"{name} differs"
+
+
+@pytest.mark.parametrize("B,H,N,D", [(1, 1, 1, 64), (2, 3, 200, 128), (1, 2, 257, 64)])
+@pytest.mark.parametrize("qk,pv,gran,mask", [("int8", "fp8", "token", None), ("fp8", "bf16", "block64", None),
+                                             ("int8", "bf16", "token", "tile"), ("int8", "fp8", "token", "doc")])
+def test_one_call_forward_equals_the_pair(cuda, B, H, N, D, qk, pv, gran, mask):
+    """sage_forward (one library call over one workspace) gives the bits of
+    quantize_qkv followed by attn_from_quantized, in both output layouts, from
+    non-contiguous inputs too."""
+    from futudiffu_amd import sage_attention as SA
+    q, k, v = (t.to(cuda) for t in O.make_inputs(B, H, N, D, seed=N + D))
+    bm = O.build_block_mask([N - N // 3, N // 3], N).to(cuda) if mask == "tile" else None
+    doc = (torch.arange(N) >= N - N // 3).to(torch.int32).expand(B, N).to(cuda) if mask == "doc" else None
+    print(f"one call {B}x{H}x{N}x{D} {qk}/{pv} {gran} {mask}", flush=True)
+    for smooth in (True, False):
+        qz = SA.quantize_qkv(q, k, v, qk=qk, pv=pv, granularity=gran, smooth_k=smooth)
+        for layout in ("bhnd", "bnhd"):
+            want, wl = SA.attn_from_quantized(qz, B, H, block_mask=bm, doc_ids=doc, out_layout=layout)
+            strided = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+            for args in ((q, k, v), strided):
+                out, lse = SA.sage_forward(*args, qk=qk, pv=pv, granularity=gran, smooth_k=smooth, block_mask=bm,
+                                           doc_ids=doc, out_layout=layout)
+                assert torch.equal(out, want) and torch.equal(lse, wl)
+
+
+def test_gradient_through_the_lse_only(cuda):
+    """No gradient reaches out: the formulas (which ask for no materialized
+    gradients) treat it as zeros, so q, k and v get zeros, not None."""
+    import futudiffu_amd  # noqa: F401
+    q, k, v = (t.to(cuda).requires_grad_(True) for t in O.make_inputs(1, 2, 130, 64, seed=5))
+    _, lse = torch.ops.futudiffu_ii.sage_attn_ext(q, k, v, None, None, 0.125, "int8", "bf16", "token", True)
+    lse.sum().backward()
+    for t in (q, k, v):
+        assert t.grad is not None and not t.grad.float().any()
