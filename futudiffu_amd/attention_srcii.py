@@ -74,9 +74,10 @@ def _grad_of(grad: Tensor | None, out: Tensor) -> Tensor:
 
 
 def _to_bhnd(x: Tensor, shape) -> Tensor:
-    """[B, N, H*D] -> contiguous [B, H, N, D]."""
+    """[B, N, H*D] as a [B, H, N, D] view, which the backward reads in place
+    (the two transposed copies took 41 of 440 us of a 1x30x3071 training step)."""
     B, H, N, D = shape
-    return x.view(B, N, H, D).transpose(1, 2).contiguous()
+    return x.reshape(B, N, H, D).transpose(1, 2)
 
 
 # ---- backward ops (attention_srcii.py:36-48, :91-103) -------------------------------

@@ -133,10 +133,11 @@ struct Rows {
   static constexpr int bytes32 = blocks32 * stride;  // a 32-row block
 
   static __device__ __forceinline__ int swap(int row_in_block) { return (row_in_block >> 2) * 2; }
-  // byte offset in its source block of the chunk that lane `lane` of the load moves
-  static __device__ __forceinline__ int src_off(int lane) {
+  // byte offset in its source block (rows `row_bytes` apart) of the chunk that
+  // lane `lane` of the load moves
+  static __device__ __forceinline__ int src_off(int lane, int row_bytes) {
     const int t = (lane >> 2) % RPB, run = (lane >> 2) / RPB;
-    return t * (2 * D) + run * 64 + ((lane & 3) ^ swap(t)) * 16;
+    return t * row_bytes + run * 64 + ((lane & 3) ^ swap(t)) * 16;
   }
   // row operand: lane (h, r) reads row r, channels [16 c2 + 8h, +8) at
   // row_off(lane, c2 % 2) + row_imm(c2)
@@ -160,19 +161,23 @@ __device__ __forceinline__ void dma_16(uint8_t* lds, __amdgpu_buffer_rsrc_t rs, 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, lds, 16, off, 0, 0, 0);
 }
 
-// Rows [0, 32) of `rows` (row-major, contiguous; rows past `left` read as
-// zeros) into the LDS block at `lds`, by waves `wave`, wave + WAVES, ...  The
-// whole offset sits in the range-checked vector operand.
+// Rows [0, 32) of `rows` (row_bytes apart; rows past `left` read as zeros)
+// into the LDS block at `lds`, by waves `wave`, wave + WAVES, ...  Each load has
+// a resource over its own rows, so the lane offset (src_off) is the same for all.
 template <int D, int WAVES>
-__device__ __forceinline__ void dma_rows32(uint8_t* lds, int wave, int src_off, const uint16_t* rows, int64_t left) {
+__device__ __forceinline__ void dma_rows32(uint8_t* lds, int wave, int src_off, const uint16_t* rows, int row_bytes,
+                                           int64_t left) {
   using R = Rows<D>;
-  const int valid = (int)(left < 0 ? 0 : left > 32 ? 32 : left);
-  const __amdgpu_buffer_rsrc_t rs = raw_rsrc(rows, (uint32_t)(valid * D * 2));
+  const int valid = (int)(left > 32 ? 32 : left);
 #pragma unroll
   for (int j0 = 0; j0 < R::blocks32; j0 += WAVES) {
     const int j = j0 + wave;
-    if (R::blocks32 % WAVES == 0 || j < R::blocks32)
-      dma_16(lds + j * R::stride, rs, src_off + j * 1024);
+    if (R::blocks32 % WAVES == 0 || j < R::blocks32) {
+      const int v = min(valid - j * R::RPB, R::RPB);  // rows of this block
+      const __amdgpu_buffer_rsrc_t rs = raw_rsrc(reinterpret_cast<const uint8_t*>(rows) + (int64_t)j * R::RPB * row_bytes,
+                                                 v > 0 ? (uint32_t)((v - 1) * row_bytes + 2 * D) : 0u);
+      dma_16(lds + j * R::stride, rs, src_off);
+    }
   }
 }
 
@@ -199,6 +204,12 @@ __device__ __forceinline__ bf16x8 tr_frag(const uint8_t* __restrict__ base, int 
   const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(base + Rows<D>::tr_imm(c, tt, 0)));
   const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsPtr)(base + Rows<D>::tr_imm(c, tt, 1)));
   return __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+}
+
+// The first row of dO of head bh (rows dout_rs elements apart).
+__device__ __forceinline__ const uint16_t* dout_head(const BwdParams& p, int bh) {
+  const int b = bh / p.h;
+  return p.dout + b * p.dout_bs + (bh - b * p.h) * p.dout_hs;
 }
 
 // Activity of up to 64 steps: bit i of each mask is step base + i.
@@ -229,9 +240,10 @@ __device__ __forceinline__ int xcd_item(int b, int total) {
 // key in the forward): 2^(s - inf) = 0 needs no per-element test.  Lane
 // (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps; the products are
 // fp32, summed per lane then over the token's lanes.  One 64-token block (bx)
-// of head bh.
+// of head bh, whose first rows dout and out point at.
 template <int D>
-__device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, const uint16_t* __restrict__ out,
+__device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, int64_t dout_rs,
+                                            const uint16_t* __restrict__ out, int64_t out_rs,
                                             const float* __restrict__ lse, int bh, int64_t bx, int64_t n, int64_t np,
                                             float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
   constexpr int LPR = D / 8, RPP = 256 / LPR, PASSES = 64 / RPP;
@@ -240,9 +252,9 @@ __device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, c
 #pragma unroll
   for (int ps = 0; ps < PASSES; ++ps) {
     const int64_t t = tok0 + rr + ps * RPP;
-    const int64_t row = ((int64_t)bh * n + min(t, n - 1)) * D + c8 * 8;
-    const uint4 a = *reinterpret_cast<const uint4*>(dout + row);
-    const uint4 o = *reinterpret_cast<const uint4*>(out + row);
+    const int64_t row = min(t, n - 1);
+    const uint4 a = *reinterpret_cast<const uint4*>(dout + row * dout_rs + c8 * 8);
+    const uint4 o = *reinterpret_cast<const uint4*>(out + row * out_rs + c8 * 8);
     float s = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -337,7 +349,7 @@ __device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int i
   }
   bf16x8 dof[2 * NC];  // dO[qrow][16c2 + 8h, +8)
   {
-    const uint16_t* dr = p.dout + ((int64_t)bh * n + min(qrow, n - 1)) * D + 8 * h;
+    const uint16_t* dr = dout_head(p, bh) + min(qrow, n - 1) * p.dout_rs + 8 * h;
 #pragma unroll
     for (int c2 = 0; c2 < 2 * NC; ++c2) dof[c2] = *reinterpret_cast<const bf16x8*>(dr + 16 * c2);
   }
@@ -391,13 +403,13 @@ __device__ __forceinline__ void dq_item(const BwdParams& p, uint8_t* smem, int i
   };
 
   // ---- staging -------------------------------------------------------------------
-  const int src_off = R::src_off(lane);
+  const int src_off = R::src_off(lane, 2 * D);
   auto load_step = [&](int s, int stage) __attribute__((always_inline)) {
     const int64_t key0 = (int64_t)s * 32;
     uint8_t* sb = smem + stage * St::bytes;
     dma_chunks_buf<2 * D, kBwdWaves>(sb, wave, lane, raw_rsrc(p.kc + ((int64_t)bh * np + key0) * D, 32 * D), 0);
-    dma_rows32<D, kBwdWaves>(sb + St::offV, wave, src_off, p.v + ((int64_t)bh * n + key0) * D, n - key0);
-    dma_rows32<D, kBwdWaves>(sb + St::offT, wave, src_off, p.kt + ((int64_t)bh * n + key0) * D, n - key0);
+    dma_rows32<D, kBwdWaves>(sb + St::offV, wave, src_off, p.v + ((int64_t)bh * n + key0) * D, 2 * D, n - key0);
+    dma_rows32<D, kBwdWaves>(sb + St::offT, wave, src_off, p.kt + ((int64_t)bh * n + key0) * D, 2 * D, n - key0);
     if (wave == 2) dma_words32(sb + St::offKd, lane, p.ks + (int64_t)bh * np + key0);
     if constexpr (MASK & 2) {
       if (wave == 3) dma_words32_unaligned(sb + St::offDoc, lane, p.doc + (int64_t)bidx * n + key0, n - key0);
@@ -593,7 +605,9 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
 #pragma unroll
     for (int c = 0; c < NC; ++c) kf[c] = *reinterpret_cast<const i32x4*>(kbp + (c * 64 + lane) * 16);
   }
-  const int src_off = R::src_off(lane), tr_off = R::tr_off(lane);
+  const int src_off = R::src_off(lane, 2 * D), do_off = R::src_off(lane, (int)(2 * p.dout_rs));
+  const int tr_off = R::tr_off(lane);
+  const uint16_t* dout = dout_head(p, bh);
   const int row_off[2] = {R::row_off(lane, 0), R::row_off(lane, 1)};
   bf16x8 vf[2 * NC];                                         // V[krow][16c2 + 8h, +8)
   uint8_t* vlds = smem + 2 * St::bytes + wave * R::bytes32;  // or the wave's V rows
@@ -602,7 +616,7 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
 #pragma unroll
     for (int c2 = 0; c2 < 2 * NC; ++c2) vf[c2] = *reinterpret_cast<const bf16x8*>(vr + 16 * c2);
   } else if (wave_live) {
-    dma_rows32<D, 1>(vlds, 0, src_off, p.v + ((int64_t)bh * n + k0) * D, n - k0);
+    dma_rows32<D, 1>(vlds, 0, src_off, p.v + ((int64_t)bh * n + k0) * D, 2 * D, n - k0);
   }
   const float kd = p.ks[(int64_t)bh * np + krow];
   const int dk_doc = (MASK & 2) ? (krow < n ? p.doc[(int64_t)bidx * n + krow] : -1) : 0;
@@ -659,8 +673,8 @@ __device__ __forceinline__ void dkdv_item(const BwdParams& p, uint8_t* smem, int
     const int64_t m0 = (int64_t)s * 32;
     uint8_t* sb = smem + stage * St::bytes;
     dma_chunks_buf<2 * D, kBwdWaves>(sb, wave, lane, raw_rsrc(p.qc + ((int64_t)bh * np + m0) * D, 32 * D), 0);
-    dma_rows32<D, kBwdWaves>(sb + St::offDo, wave, src_off, p.dout + ((int64_t)bh * n + m0) * D, n - m0);
-    dma_rows32<D, kBwdWaves>(sb + St::offQ, wave, src_off, p.q + ((int64_t)bh * n + m0) * D, n - m0);
+    dma_rows32<D, kBwdWaves>(sb + St::offDo, wave, do_off, dout + m0 * p.dout_rs, (int)(2 * p.dout_rs), n - m0);
+    dma_rows32<D, kBwdWaves>(sb + St::offQ, wave, src_off, p.q + ((int64_t)bh * n + m0) * D, 2 * D, n - m0);
     if (wave < 3) {
       const float* src = wave == 0 ? p.qs : wave == 1 ? p.lse_pad : p.neg_delta;
       dma_words32(sb + St::offQd + wave * 128, lane, src + (int64_t)bh * np + m0);
@@ -828,30 +842,25 @@ __global__ void __launch_bounds__(kBwdThreads, 2) bwd_kernel(BwdParams p, int it
 // The preparation in one launch, grid (np / 64, BH, 1 or 2): z = 0 the
 // per-query values, z = 1 the smoothed K rows.
 template <int D>
-__global__ void __launch_bounds__(256) bwd_prep_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ mu,
-                                                       uint16_t* __restrict__ kt, const uint16_t* __restrict__ dout,
-                                                       const uint16_t* __restrict__ out,
-                                                       const float* __restrict__ lse, int64_t n, int64_t np,
-                                                       float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
+__global__ void __launch_bounds__(256) bwd_prep_kernel(BwdPrep a, int64_t n, int64_t np) {
   const int bh = blockIdx.y;
   const int64_t bx = blockIdx.x;
-  if (blockIdx.z == 0)
-    delta_block<D>(dout, out, lse, bh, bx, n, np, neg_delta, lse_pad);
-  else if (bx * 64 < n)
-    smooth_block<D>(k, mu, bh, bx, n, kt);
+  if (blockIdx.z == 0) {
+    const int b = bh / a.h, h = bh - b * a.h;
+    delta_block<D>(a.dout + b * a.dout_bs + h * a.dout_hs, a.dout_rs, a.out + b * a.out_bs + h * a.out_hs, a.out_rs,
+                   a.lse, bh, bx, n, np, a.neg_delta, a.lse_pad);
+  } else if (bx * 64 < n) {
+    smooth_block<D>(a.k, a.mu, bh, bx, n, a.kt);
+  }
 }
 
-hipError_t launch_bwd_prep(const uint16_t* k, const uint16_t* mu, uint16_t* kt, const uint16_t* dout,
-                           const uint16_t* out, const float* lse, int64_t bh, int64_t n, int64_t d, float* neg_delta,
-                           float* lse_pad, hipStream_t st) {
+hipError_t launch_bwd_prep(const BwdPrep& a, int64_t bh, int64_t n, int64_t d, hipStream_t st) {
   const int64_t np = padded_len(n);
-  const dim3 grid((unsigned)(np / 64), (unsigned)bh, mu ? 2u : 1u);
+  const dim3 grid((unsigned)(np / 64), (unsigned)bh, a.mu ? 2u : 1u);
   if (d == 128)
-    hipLaunchKernelGGL(bwd_prep_kernel<128>, grid, dim3(256), 0, st, k, mu, kt, dout, out, lse, n, np, neg_delta,
-                       lse_pad);
+    hipLaunchKernelGGL(bwd_prep_kernel<128>, grid, dim3(256), 0, st, a, n, np);
   else if (d == 64)
-    hipLaunchKernelGGL(bwd_prep_kernel<64>, grid, dim3(256), 0, st, k, mu, kt, dout, out, lse, n, np, neg_delta,
-                       lse_pad);
+    hipLaunchKernelGGL(bwd_prep_kernel<64>, grid, dim3(256), 0, st, a, n, np);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

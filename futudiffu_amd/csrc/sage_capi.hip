@@ -536,6 +536,17 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
                   float sm_scale_log2e, const uint8_t* tile_mask, int64_t mask_stride_z, int64_t mask_nq, int64_t mask_nkv,
                   const int32_t* doc_ids, void* workspace, size_t workspace_bytes, void* dq, void* dk, void* dv,
                   hipStream_t stream) {
+  return sage_attn_bwd_layout(q, k, v, out, SAGE_OUT_BHND, lse, dout, SAGE_OUT_BHND, b, h, n, d, qk_kind, smooth_k,
+                              sm_scale, sm_scale_log2e, tile_mask, mask_stride_z, mask_nq, mask_nkv, doc_ids,
+                              workspace, workspace_bytes, dq, dk, dv, stream);
+}
+
+int sage_attn_bwd_layout(const void* q, const void* k, const void* v, const void* out, int out_layout,
+                         const float* lse, const void* dout, int dout_layout, int64_t b, int64_t h, int64_t n,
+                         int64_t d, int qk_kind, int smooth_k, float sm_scale, float sm_scale_log2e,
+                         const uint8_t* tile_mask, int64_t mask_stride_z, int64_t mask_nq, int64_t mask_nkv,
+                         const int32_t* doc_ids, void* workspace, size_t workspace_bytes, void* dq, void* dk, void* dv,
+                         hipStream_t stream) {
   if (b <= 0 || h <= 0) return fail(SAGE_ERR_ARG, "b=%lld and h=%lld must be positive", (long long)b, (long long)h);
   int st = check_common(b * h, n, d, qk_kind, SAGE_PV_BF16, SAGE_GRAN_TOKEN);
   if (st) return st;
@@ -545,6 +556,9 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
     if (!aligned16(p)) return fail(SAGE_ERR_ALIGN, "tensor pointers must be 16-byte aligned");
   if (!(sm_scale > 0.0f) || !(sm_scale_log2e > 0.0f))
     return fail(SAGE_ERR_ARG, "sm_scale and sm_scale_log2e must be positive");
+  for (const int layout : {out_layout, dout_layout})
+    if (layout != SAGE_OUT_BHND && layout != SAGE_OUT_BNHD)
+      return fail(SAGE_ERR_ARG, "out and dout layouts must be 0 ([B,H,N,D]) or 1 ([B,N,H,D]), got %d", layout);
   const int64_t nq = (n + 127) / 128, nkv = (n + 63) / 64;
   int mask = 0;
   if (tile_mask) {
@@ -579,9 +593,25 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
       reinterpret_cast<uint16_t*>(w + ws.kmean), sage::ProdArgs{}, stream);
   if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (quantize)");
   const uint16_t* mean = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kmean) : nullptr;
-  e = sage::launch_bwd_prep(k16, mean, reinterpret_cast<uint16_t*>(w + ws.kt), do16, static_cast<const uint16_t*>(out),
-                            lse, bh, n, d, reinterpret_cast<float*>(w + ws.neg_delta),
-                            reinterpret_cast<float*>(w + ws.lse_pad), stream);
+  // element strides per batch, head and row of a layout
+  auto strides = [&](int layout, int64_t& bs, int64_t& hs, int64_t& rs) {
+    bs = h * n * d;
+    hs = layout == SAGE_OUT_BNHD ? d : n * d;
+    rs = layout == SAGE_OUT_BNHD ? h * d : d;
+  };
+  sage::BwdPrep prep{};
+  prep.k = k16;
+  prep.mu = mean;
+  prep.kt = reinterpret_cast<uint16_t*>(w + ws.kt);
+  prep.dout = do16;
+  strides(dout_layout, prep.dout_bs, prep.dout_hs, prep.dout_rs);
+  prep.out = static_cast<const uint16_t*>(out);
+  strides(out_layout, prep.out_bs, prep.out_hs, prep.out_rs);
+  prep.lse = lse;
+  prep.neg_delta = reinterpret_cast<float*>(w + ws.neg_delta);
+  prep.lse_pad = reinterpret_cast<float*>(w + ws.lse_pad);
+  prep.h = (int)h;
+  e = sage::launch_bwd_prep(prep, bh, n, d, stream);
   if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (prep)");
   const int4* sums = reinterpret_cast<const int4*>(w + ws.sums);
   const int64_t np = sage::padded_len(n);
@@ -600,6 +630,9 @@ int sage_attn_bwd(const void* q, const void* k, const void* v, const void* out, 
   p.kt = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kt) : k16;
   p.v = static_cast<const uint16_t*>(v);
   p.dout = do16;
+  p.dout_bs = prep.dout_bs;
+  p.dout_hs = prep.dout_hs;
+  p.dout_rs = prep.dout_rs;
   p.lse_pad = reinterpret_cast<const float*>(w + ws.lse_pad);
   p.neg_delta = reinterpret_cast<const float*>(w + ws.neg_delta);
   p.tile_mask = tile_mask;

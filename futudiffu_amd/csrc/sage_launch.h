@@ -185,9 +185,9 @@ hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t p
 
 // Backward (sage_kernels.py:321-349, :805-1030, :1491-1722).  Codes and
 // scales are the quantization's per-token outputs ([BH, Np] layout, Q scale
-// with sm_scale*log2(e)); q, v, dout, kt (K~, the smoothed K: k itself without
-// smoothing) and the gradients are plain rows [BH, N, D]; lse_pad and
-// neg_delta are [BH, Np] (launch_bwd_prep).
+// with sm_scale*log2(e)); q, v, kt (K~, the smoothed K: k itself without
+// smoothing) and the gradients are plain rows [BH, N, D], dout rows of D at the
+// given strides; lse_pad and neg_delta are [BH, Np] (launch_bwd_prep).
 struct BwdParams {
   const uint8_t* qc;
   const float* qs;
@@ -197,6 +197,7 @@ struct BwdParams {
   const uint16_t* kt;
   const uint16_t* v;
   const uint16_t* dout;
+  int64_t dout_bs, dout_hs, dout_rs;  // element strides per batch, head and row (AttnParams::out_bs)
   const float* lse_pad;
   const float* neg_delta;
   const uint8_t* tile_mask;
@@ -228,10 +229,21 @@ constexpr int kBwdDqSplit = 64;
 
 // The backward's own operands: kt = bf16(k - mu) rows [BH, N, D] (not written
 // when mu is null), neg_delta = -rowsum(dout * out) and the LSE with +inf for
-// rows without gradient, both [BH, Np].
-hipError_t launch_bwd_prep(const uint16_t* k, const uint16_t* mu, uint16_t* kt, const uint16_t* dout,
-                           const uint16_t* out, const float* lse, int64_t bh, int64_t n, int64_t d, float* neg_delta,
-                           float* lse_pad, hipStream_t st);
+// rows without gradient, both [BH, Np]; dout and out at their strides.
+struct BwdPrep {
+  const uint16_t* k;
+  const uint16_t* mu;
+  uint16_t* kt;
+  const uint16_t* dout;
+  int64_t dout_bs, dout_hs, dout_rs;
+  const uint16_t* out;
+  int64_t out_bs, out_hs, out_rs;
+  const float* lse;
+  float* neg_delta;
+  float* lse_pad;
+  int h;
+};
+hipError_t launch_bwd_prep(const BwdPrep& a, int64_t bh, int64_t n, int64_t d, hipStream_t st);
 hipError_t launch_bwd(int qk, int mask, const BwdParams& p, int64_t d, int64_t bh, hipStream_t st);
 hipError_t launch_doc_from_cu(const int32_t* cu, int64_t nb, int64_t nseg, int64_t n, int32_t* doc,
                               hipStream_t st);

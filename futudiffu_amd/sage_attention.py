@@ -416,6 +416,14 @@ def sage_attn_forward_masked_merged_heads(q: Tensor, k: Tensor, v: Tensor, block
                         granularity=granularity, out_layout="bnhd")
 
 
+def _rows_layout(t: Tensor) -> tuple[Tensor, int]:
+    """A [B, H, N, D] tensor the backward can read in place, with its memory
+    layout: [B, H, N, D], or [B, N, H, D] (a transposed view); a copy else."""
+    if not t.is_contiguous() and t.transpose(1, 2).is_contiguous():
+        return t, _LAYOUT["bnhd"]
+    return t.contiguous(), _LAYOUT["bhnd"]
+
+
 def sage_backward(q: Tensor, k: Tensor, v: Tensor, out: Tensor, lse: Tensor, dout: Tensor,
                   sm_scale: float | None = None, *, block_mask: Tensor | None = None,
                   doc_ids: Tensor | None = None, qk: str | None = None,
@@ -441,7 +449,8 @@ def sage_backward(q: Tensor, k: Tensor, v: Tensor, out: Tensor, lse: Tensor, dou
             raise ValueError(f"{name} must be a bf16 [{B}, {H}, {N}, {D}] tensor on {dev}")
     if tuple(lse.shape) != (B * H, N) or lse.dtype != torch.float32 or lse.device != dev:
         raise ValueError(f"lse must be an fp32 [{B * H}, {N}] tensor on {dev}")
-    q, k, v, out, dout, lse = (t.contiguous() for t in (q, k, v, out, dout, lse))
+    q, k, v, lse = (t.contiguous() for t in (q, k, v, lse))
+    (out, out_layout), (dout, dout_layout) = _rows_layout(out), _rows_layout(dout)
     lib = _lib.load()
     BH = B * H
     bm, stride_z, nq, nkv = _norm_mask(block_mask, BH, N, dev)
@@ -449,9 +458,9 @@ def sage_backward(q: Tensor, k: Tensor, v: Tensor, out: Tensor, lse: Tensor, dou
     wsb = int(lib.sage_attn_bwd_workspace_bytes(B, H, N, D))
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
     dq, dk, dv = (torch.empty_like(q) for _ in range(3))
-    _lib.check(lib.sage_attn_bwd(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), dout.data_ptr(),
-        B, H, N, D, _QK[qk], int(bool(smooth_k)), float(sm_scale), _fold(sm_scale), _ptr(bm), stride_z, nq, nkv,
+    _lib.check(lib.sage_attn_bwd_layout(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), out_layout, lse.data_ptr(), dout.data_ptr(),
+        dout_layout, B, H, N, D, _QK[qk], int(bool(smooth_k)), float(sm_scale), _fold(sm_scale), _ptr(bm), stride_z, nq, nkv,
         _ptr(doc_ids), ws.data_ptr(), wsb, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), _stream_handle(dev)))
     return dq, dk, dv
 

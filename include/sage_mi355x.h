@@ -330,6 +330,23 @@ int sage_attn_bwd(const void* q, const void* k, const void* v,
                   void* dq, void* dk, void* dv,
                   hipStream_t stream);
 
+/* sage_attn_bwd with out and dout each in [B, H, N, D] (SAGE_OUT_BHND) or in
+ * the out-projection's [B, N, H, D] (SAGE_OUT_BNHD), in which a forward with
+ * out_layout SAGE_OUT_BNHD and its consumer's gradient have them: the kernels
+ * read the rows where they are.  The same results; dq, dk, dv are
+ * [B, H, N, D] always. */
+int sage_attn_bwd_layout(const void* q, const void* k, const void* v,
+                         const void* out, int out_layout, const float* lse,
+                         const void* dout, int dout_layout,
+                         int64_t b, int64_t h, int64_t n, int64_t d,
+                         int qk_kind, int smooth_k, float sm_scale, float sm_scale_log2e,
+                         const uint8_t* tile_mask, int64_t mask_stride_z,
+                         int64_t mask_nq, int64_t mask_nkv,
+                         const int32_t* doc_ids,
+                         void* workspace, size_t workspace_bytes,
+                         void* dq, void* dk, void* dv,
+                         hipStream_t stream);
+
 /* sage_quantize_qkv and sage_attn_fwd in one call, the quantized operands kept
  * in the workspace: the whole forward of the attention op
  * (sage_attention.py:461-531) from bf16 q, k, v [B, H, N, D] contiguous.

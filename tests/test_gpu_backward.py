@@ -261,3 +261,23 @@ def test_backward_step_edges(cuda, N, kind):
     if N > 1:  # one key: softmax is constant, dQ and dK are rounding only
         _close(dq, rq, "dq")
         _close(dk, rk, "dk")
+
+
+@pytest.mark.parametrize("B,H,N,D", [(1, 3, 200, 128), (2, 4, 65, 64), (2, 1, 130, 128), (1, 2, 1, 64)])
+def test_backward_reads_merged_heads_in_place(cuda, B, H, N, D):
+    """out and dout as views of [B, N, H*D] tensors (each alone and both) give
+    the bits of their contiguous copies; other strides are copied."""
+    from futudiffu_amd import sage_attention as SA
+    q, k, v, dout = _inputs(B, H, N, D, seed=17 + N)
+    sm = 1.0 / math.sqrt(D)
+    qg, kg, vg, dog = (t.to(cuda) for t in (q, k, v, dout))
+    out, lse = SA.sage_forward(qg, kg, vg, sm, qk="int8", pv="bf16", smooth_k=True)
+    merged = lambda t: t.transpose(1, 2).reshape(B, N, H * D).contiguous().view(B, N, H, D).transpose(1, 2)  # noqa: E731
+    wide = torch.empty(B, H, N, 2 * D, dtype=torch.bfloat16, device=cuda)
+    wide[..., :D] = dog
+    print(f"bwd merged heads {B}x{H}x{N}x{D}", flush=True)
+    want = SA.sage_backward(qg, kg, vg, out, lse, dog, sm, qk="int8", smooth_k=True)
+    for o, g in ((merged(out), dog), (out, merged(dog)), (merged(out), merged(dog)), (out, wide[..., :D])):
+        got = SA.sage_backward(qg, kg, vg, o, lse, g, sm, qk="int8", smooth_k=True)
+        for name, a, b_ in zip(("dq", "dk", "dv"), got, want):
+            assert a.is_contiguous() and torch.equal(a, b_), name
