@@ -8,11 +8,10 @@
 //
 // Operands.  P is recomputed from the forward's per-token codes exactly as the
 // forward scores them, s = acc * qd * kd (qd carrying sm_scale*log2(e)),
-// p = 2^(s - lse) with the forward's base-2 LSE.  The quantization kernel
-// supplies the Q and smoothed-K codes and scales; one preparation launch
-// (bwd_prep_kernel) writes the rows K~ = bf16(k - mean), -D = -rowsum(dO * O)
-// and the LSE padded to whole blocks.  Q, dO, V and K~ are read as the plain
-// bf16 rows they are.
+// p = 2^(s - lse) with the forward's base-2 LSE.  The quantization launch, in
+// its backward form, supplies the Q and smoothed-K codes and scales, the rows
+// K~ = bf16(k - mean), -D = -rowsum(dO * O) and the LSE padded to whole blocks.
+// Q, dO, V and K~ are read as the plain bf16 rows they are.
 //
 // Rows in LDS.  One copy of a 32-row block serves both as the row operand of
 // v_mfma_f32_32x32x16_bf16 (contraction over channels: lane (h, r) reads the
@@ -33,7 +32,8 @@
 // waves all ran the same phase between two barriers, with separate row and
 // transposed images of each operand, the kernel takes 1056 -> 862 us at
 // 1x30x4416x128 and 1808 -> 1127 us on the packed 1x30x6912 batch with document
-// ids, and the preparation 51 -> 23 us.  What bounds it now is the power limit:
+// ids, and the preparation that wrote those
+// images (51 us) is gone.  What bounds it now is the power limit:
 // 27.4 M MFMAs of random data run at 18.2 ns each per SIMD alone (1.79 GHz,
 // 489 us), 20.4 ns beside six vector instructions each (546 us).
 // Work items are dealt to XCDs in contiguous ranges.  One launch (bwd_kernel)
@@ -68,10 +68,6 @@
 namespace sage {
 
 namespace {
-
-__device__ __forceinline__ uint32_t word_at(const uint4& w, int i) {
-  return i == 0 ? w.x : i == 1 ? w.y : i == 2 ? w.z : w.w;
-}
 
 // 16-byte unit as a native vector: its copies are plain loads and stores.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -221,10 +217,6 @@ struct StepMasks {
 
 }  // namespace
 
-// ---------------------------------------------------------------------------
-// Preparation
-// ---------------------------------------------------------------------------
-
 // Item of workgroup b of a 1D grid of `total` items: the hardware hands
 // workgroup b to XCD b % 8, and each XCD has its own L2, so every XCD takes a
 // contiguous range of items (head-major order) and its resident workgroups
@@ -233,71 +225,6 @@ __device__ __forceinline__ int xcd_item(int b, int total) {
   constexpr int kXcd = 8;
   const int x = b % kXcd, local = b / kXcd, per = total / kXcd, rem = total % kXcd;
   return x * per + min(x, rem) + local;
-}
-
-// -D = -rowsum(dO * O) per token in fp32 (sage_kernels.py:321-349), zero past
-// N, and the LSE with +inf for rows without a gradient (past N, or no visible
-// key in the forward): 2^(s - inf) = 0 needs no per-element test.  Lane
-// (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps; the products are
-// fp32, summed per lane then over the token's lanes.  One 64-token block (bx)
-// of head bh, whose first rows dout and out point at.
-template <int D>
-__device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, int64_t dout_rs,
-                                            const uint16_t* __restrict__ out, int64_t out_rs,
-                                            const float* __restrict__ lse, int bh, int64_t bx, int64_t n, int64_t np,
-                                            float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
-  constexpr int LPR = D / 8, RPP = 256 / LPR, PASSES = 64 / RPP;
-  const int tid = threadIdx.x, c8 = tid % LPR, rr = tid / LPR;
-  const int64_t tok0 = bx * 64;
-#pragma unroll
-  for (int ps = 0; ps < PASSES; ++ps) {
-    const int64_t t = tok0 + rr + ps * RPP;
-    const int64_t row = min(t, n - 1);
-    const uint4 a = *reinterpret_cast<const uint4*>(dout + row * dout_rs + c8 * 8);
-    const uint4 o = *reinterpret_cast<const uint4*>(out + row * out_rs + c8 * 8);
-    float s = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int sh = (e & 1) * 16;
-      s += bf16_to_f32((uint16_t)(word_at(a, e >> 1) >> sh)) * bf16_to_f32((uint16_t)(word_at(o, e >> 1) >> sh));
-    }
-#pragma unroll
-    for (int off = 1; off < LPR; off <<= 1) s += __shfl_xor(s, off);
-    if (c8 == 0) {
-      const float l = lse[(int64_t)bh * n + min(t, n - 1)];
-      neg_delta[(int64_t)bh * np + t] = t < n ? -s : 0.0f;
-      lse_pad[(int64_t)bh * np + t] = t < n && l > -INFINITY ? l : INFINITY;
-    }
-  }
-}
-
-// K~ = bf16(k - mean) of one 64-token block (the quantization's smoothed K,
-// sage_attention.py:63-71), one thread per 16-byte chunk.
-template <int D>
-__device__ __forceinline__ void smooth_block(const uint16_t* __restrict__ k, const uint16_t* __restrict__ mu, int bh,
-                                             int64_t bx, int64_t n, uint16_t* __restrict__ kt) {
-  constexpr int CPR = D / 8;
-  const int64_t rows = min((int64_t)64, n - bx * 64);
-  const int64_t at = ((int64_t)bh * n + bx * 64) * D;
-  const uint4* src = reinterpret_cast<const uint4*>(k + at);
-  uint4* dst = reinterpret_cast<uint4*>(kt + at);
-  const uint4 m = reinterpret_cast<const uint4*>(mu + (int64_t)bh * D)[threadIdx.x % CPR];
-#pragma unroll
-  for (int c0 = 0; c0 < 64 * CPR; c0 += 256) {
-    const int c = c0 + (int)threadIdx.x;
-    if (c < rows * CPR) {
-      const uint4 x = src[c];
-      uint32_t o[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t w = word_at(x, i), mw = word_at(m, i);
-        const uint16_t lo = f32_to_bf16_rne(bf16_to_f32((uint16_t)w) - bf16_to_f32((uint16_t)mw));
-        const uint16_t hi = f32_to_bf16_rne(bf16_to_f32((uint16_t)(w >> 16)) - bf16_to_f32((uint16_t)(mw >> 16)));
-        o[i] = lo | ((uint32_t)hi << 16);
-      }
-      dst[c] = make_uint4(o[0], o[1], o[2], o[3]);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -838,33 +765,6 @@ __global__ void __launch_bounds__(kBwdThreads, 2) bwd_kernel(BwdParams p, int it
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-
-// The preparation in one launch, grid (np / 64, BH, 1 or 2): z = 0 the
-// per-query values, z = 1 the smoothed K rows.
-template <int D>
-__global__ void __launch_bounds__(256) bwd_prep_kernel(BwdPrep a, int64_t n, int64_t np) {
-  const int bh = blockIdx.y;
-  const int64_t bx = blockIdx.x;
-  if (blockIdx.z == 0) {
-    const int b = bh / a.h, h = bh - b * a.h;
-    delta_block<D>(a.dout + b * a.dout_bs + h * a.dout_hs, a.dout_rs, a.out + b * a.out_bs + h * a.out_hs, a.out_rs,
-                   a.lse, bh, bx, n, np, a.neg_delta, a.lse_pad);
-  } else if (bx * 64 < n) {
-    smooth_block<D>(a.k, a.mu, bh, bx, n, a.kt);
-  }
-}
-
-hipError_t launch_bwd_prep(const BwdPrep& a, int64_t bh, int64_t n, int64_t d, hipStream_t st) {
-  const int64_t np = padded_len(n);
-  const dim3 grid((unsigned)(np / 64), (unsigned)bh, a.mu ? 2u : 1u);
-  if (d == 128)
-    hipLaunchKernelGGL(bwd_prep_kernel<128>, grid, dim3(256), 0, st, a, n, np);
-  else if (d == 64)
-    hipLaunchKernelGGL(bwd_prep_kernel<64>, grid, dim3(256), 0, st, a, n, np);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
 
 template <int D, int QK, int MASK>
 hipError_t launch_bwd_t(const BwdParams& p, int64_t bh, hipStream_t st) {

@@ -130,10 +130,10 @@ int check_producer(const void* qkv, const float* q_norm_w, const float* k_norm_w
 }
 
 // Backward workspace: byte offsets of the quantization's outputs (codes,
-// scales, K mean, column-sum partials, the V operand), the smoothed K rows,
-// -D and the padded LSE.
+// scales, K mean, column-sum partials), the smoothed K rows, -D and the padded
+// LSE.
 struct BwdWorkspace {
-  size_t qc, qs, kc, ks, kmean, quant, vop, kt, neg_delta, lse_pad, sums, dq_part, dq_ctr, bytes;
+  size_t qc, qs, kc, ks, kmean, quant, kt, neg_delta, lse_pad, sums, dq_part, dq_ctr, bytes;
 };
 
 BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
@@ -152,13 +152,11 @@ BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
   w.kmean = take((size_t)bh * d * 2);
   w.quant = take(sage::quant_workspace_bytes(bh, n, d));
   // Five regions of one bf16 image each: the size is part of the interface
-  // (callers keep workspaces of it), the last three are not used in full
-  // since the passes read dO, Q and V as they are.
-  w.vop = take(rows * d * 2);
+  // (callers keep workspaces of it), the last three are spare since the passes
+  // read dO, Q and V as they are.
   w.kt = take(rows * d * 2);
   w.lse_pad = take(rows * d * 2);
-  take(rows * d * 2);
-  take(rows * d * 2);
+  for (int i = 0; i < 3; ++i) take(rows * d * 2);
   w.neg_delta = take(rows * 4);
   // document-id summaries (used with doc_ids): key tiles, 32- and 128-row blocks
   w.sums = take((size_t)b * ((n + 63) / 64 + np / 32 + np / 128) * sizeof(int4));
@@ -585,23 +583,14 @@ int sage_attn_bwd_layout(const void* q, const void* k, const void* v, const void
   const auto* q16 = static_cast<const uint16_t*>(q);
   const auto* k16 = static_cast<const uint16_t*>(k);
   const auto* do16 = static_cast<const uint16_t*>(dout);
-  // codes, scales and the K mean of the forward's per-token quantization
-  hipError_t e = sage::launch_quantize(
-      qk_kind, SAGE_PV_BF16, SAGE_GRAN_TOKEN, smooth_k != 0, q16, k16, do16, bh, n, d,
-      sm_scale_log2e, reinterpret_cast<double*>(w + ws.quant), w + ws.qc,
-      reinterpret_cast<float*>(w + ws.qs), w + ws.kc, reinterpret_cast<float*>(w + ws.ks), w + ws.vop, nullptr,
-      reinterpret_cast<uint16_t*>(w + ws.kmean), sage::ProdArgs{}, stream);
-  if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (quantize)");
-  const uint16_t* mean = smooth_k ? reinterpret_cast<const uint16_t*>(w + ws.kmean) : nullptr;
-  // element strides per batch, head and row of a layout
+  // codes, scales and the K mean of the forward's per-token quantization, and
+  // the backward's own operands, in one launch
   auto strides = [&](int layout, int64_t& bs, int64_t& hs, int64_t& rs) {
     bs = h * n * d;
     hs = layout == SAGE_OUT_BNHD ? d : n * d;
     rs = layout == SAGE_OUT_BNHD ? h * d : d;
   };
   sage::BwdPrep prep{};
-  prep.k = k16;
-  prep.mu = mean;
   prep.kt = reinterpret_cast<uint16_t*>(w + ws.kt);
   prep.dout = do16;
   strides(dout_layout, prep.dout_bs, prep.dout_hs, prep.dout_rs);
@@ -611,8 +600,11 @@ int sage_attn_bwd_layout(const void* q, const void* k, const void* v, const void
   prep.neg_delta = reinterpret_cast<float*>(w + ws.neg_delta);
   prep.lse_pad = reinterpret_cast<float*>(w + ws.lse_pad);
   prep.h = (int)h;
-  e = sage::launch_bwd_prep(prep, bh, n, d, stream);
-  if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (prep)");
+  hipError_t e = sage::launch_quantize_bwd(
+      qk_kind, smooth_k != 0, q16, k16, bh, n, d, sm_scale_log2e, reinterpret_cast<double*>(w + ws.quant), w + ws.qc,
+      reinterpret_cast<float*>(w + ws.qs), w + ws.kc, reinterpret_cast<float*>(w + ws.ks),
+      reinterpret_cast<uint16_t*>(w + ws.kmean), prep, stream);
+  if (e != hipSuccess) return launch_status(e, "sage_attn_bwd (quantize)");
   const int4* sums = reinterpret_cast<const int4*>(w + ws.sums);
   const int64_t np = sage::padded_len(n);
   if (doc_ids) {

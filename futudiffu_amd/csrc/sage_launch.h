@@ -146,6 +146,24 @@ hipError_t launch_quantize(int qk, int pv, int gran, bool smooth, const uint16_t
                            const uint16_t* v, int64_t bh, int64_t n, int64_t d, float fold, double* ws,
                            uint8_t* qc, float* qs, uint8_t* kc, float* ks, uint8_t* vout, float* vs,
                            uint16_t* kmean, const ProdArgs& prod, hipStream_t st);
+// The quantization in its backward form: per-token codes and scales of Q and K
+// and the K mean, and the backward's own operands: the rows kt = bf16(k - mean)
+// [BH, N, D] (with smoothing), neg_delta = -rowsum(dout * out) and the LSE with
+// +inf for rows without gradient, both [BH, Np].
+struct BwdPrep {
+  uint16_t* kt;
+  const uint16_t* dout;
+  int64_t dout_bs, dout_hs, dout_rs;  // element strides per batch, head and row
+  const uint16_t* out;
+  int64_t out_bs, out_hs, out_rs;
+  const float* lse;
+  float* neg_delta;
+  float* lse_pad;
+  int h;  // heads per batch
+};
+hipError_t launch_quantize_bwd(int qk, bool smooth, const uint16_t* q, const uint16_t* k, int64_t bh, int64_t n,
+                               int64_t d, float fold, double* ws, uint8_t* qc, float* qs, uint8_t* kc, float* ks,
+                               uint16_t* kmean, const BwdPrep& prep, hipStream_t st);
 hipError_t launch_qkv_postprocess(const ProdArgs& prod, int64_t bh, int64_t n, int64_t d, uint16_t* q_out,
                                   uint16_t* k_out, uint16_t* v_out, hipStream_t st);
 // Gradient of the producer with respect to its input (fused_kernels.py:711-783):
@@ -187,7 +205,7 @@ hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t p
 // scales are the quantization's per-token outputs ([BH, Np] layout, Q scale
 // with sm_scale*log2(e)); q, v, kt (K~, the smoothed K: k itself without
 // smoothing) and the gradients are plain rows [BH, N, D], dout rows of D at the
-// given strides; lse_pad and neg_delta are [BH, Np] (launch_bwd_prep).
+// given strides; lse_pad and neg_delta are [BH, Np] (launch_quantize_bwd).
 struct BwdParams {
   const uint8_t* qc;
   const float* qs;
@@ -227,23 +245,6 @@ struct BwdParams {
 // multiple of 8, so both halves of an item run on one XCD).
 constexpr int kBwdDqSplit = 64;
 
-// The backward's own operands: kt = bf16(k - mu) rows [BH, N, D] (not written
-// when mu is null), neg_delta = -rowsum(dout * out) and the LSE with +inf for
-// rows without gradient, both [BH, Np]; dout and out at their strides.
-struct BwdPrep {
-  const uint16_t* k;
-  const uint16_t* mu;
-  uint16_t* kt;
-  const uint16_t* dout;
-  int64_t dout_bs, dout_hs, dout_rs;
-  const uint16_t* out;
-  int64_t out_bs, out_hs, out_rs;
-  const float* lse;
-  float* neg_delta;
-  float* lse_pad;
-  int h;
-};
-hipError_t launch_bwd_prep(const BwdPrep& a, int64_t bh, int64_t n, int64_t d, hipStream_t st);
 hipError_t launch_bwd(int qk, int mask, const BwdParams& p, int64_t d, int64_t bh, hipStream_t st);
 hipError_t launch_doc_from_cu(const int32_t* cu, int64_t nb, int64_t nseg, int64_t n, int32_t* doc,
                               hipStream_t st);

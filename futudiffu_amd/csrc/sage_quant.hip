@@ -27,6 +27,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 namespace sage {
 
@@ -522,6 +523,18 @@ __device__ __forceinline__ void rows_load(const uint16_t* src, int64_t stride, i
   for (int ps = 0; ps < PASSES; ++ps) w[ps] = load16(rs, (uint32_t)(((rr + ps * RPP) * stride + c8 * 8) * 2));
 }
 
+// The launch's backward form (sage_attn_bwd): kPV_BWD in place of a V kind.  The
+// V units form -D and the padded LSE, the K units also write the smoothed rows.
+// As a launch of its own after a quantization that wrote an unused V operand
+// that work took 23 of 58 us at 1x30x4416x128 (memory-bound: 308 MB together,
+// 239 MB now); the backward 864 -> 849 us, the packed batch 1179 -> 1158 us.
+constexpr int kPV_BWD = 2;
+struct BwdQuantArgs : ProdArgs {
+  BwdPrep prep;
+};
+template <int PV>
+using QuantExtra = std::conditional_t<PV == kPV_BWD, BwdQuantArgs, ProdArgs>;
+
 // The producer's inputs for the rows of one head: the norm weights and the
 // rotation rows from `row0` (the flattened (batch, token) index of token 0).
 struct ProdRows {
@@ -535,11 +548,11 @@ struct ProdRows {
 // block from the loads of rows_load.  PROD: rows of the projection output
 // through RMSNorm + rotary (pr: the block's weights and rotations).  TAIL: the
 // block reaches past N.
-template <int D, int QK, int GRAN, bool PROD, bool TAIL>
+template <int D, int QK, int GRAN, bool PROD, bool TAIL, bool KT = false>
 __device__ __forceinline__ void rows_quant(uint4 (&w)[64 / (256 / (D / 8))], const ProdRows& pr,
                                            int64_t tok0, int64_t n, float fold,
                                            const float* mu, uint8_t* __restrict__ codes, float* __restrict__ scale,
-                                           unsigned* blk_amax, int tid) {
+                                           unsigned* blk_amax, int tid, uint16_t* __restrict__ kt = nullptr) {
   constexpr int LPR = D / 8;
   constexpr int RPP = 256 / LPR;
   constexpr int PASSES = 64 / RPP;
@@ -573,15 +586,22 @@ __device__ __forceinline__ void rows_quant(uint4 (&w)[64 / (256 / (D / 8))], con
     if (mu != nullptr) {
       // bf16(k - mean); rows past N (loaded as zeros) stay zero
       const float keep = (!TAIL || tok0 + rr + ps * RPP < n) ? 1.0f : 0.0f;
+      uint32_t row[4];
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
         const uint32_t p2 = pack_bf16x2(x[ps][e] - m[e], x[ps][e + 1] - m[e + 1]);  // round to nearest even
+        row[e / 2] = p2;
         x[ps][e] = __uint_as_float(p2 << 16);
         x[ps][e + 1] = __uint_as_float(p2 & 0xffff0000u);
         if constexpr (TAIL) {
           x[ps][e] *= keep;
           x[ps][e + 1] *= keep;
         }
+      }
+      if constexpr (KT) {
+        const int64_t tok = tok0 + rr + ps * RPP;
+        if (!TAIL || tok < n)
+          *reinterpret_cast<uint4*>(kt + tok * D + c8 * 8) = make_uint4(row[0], row[1], row[2], row[3]);
       }
     }
   }
@@ -598,6 +618,43 @@ __device__ __forceinline__ void rows_block(const uint16_t* src, int64_t stride, 
   rows_load<D>(src, stride, tok0, n, tid, w);
   rows_quant<D, QK, GRAN, PROD, false>(w, ProdRows{&prod, nw, row0}, tok0, n, fold, nullptr, codes, scale, blk_amax,
                                        tid);
+}
+
+// The backward's per-query values, in place of V in its form of the launch:
+// -D = -rowsum(dO * O) per token in fp32 (sage_kernels.py:321-349), zero past
+// N, and the LSE with +inf for rows without a gradient (past N, or no visible
+// key in the forward): 2^(s - inf) = 0 needs no per-element test.  Lane
+// (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps; the products are
+// fp32, summed per lane then over the token's lanes.  One 64-token block (bx)
+// of head bh, whose first rows dout and out point at.
+template <int D>
+__device__ __forceinline__ void delta_block(const uint16_t* __restrict__ dout, int64_t dout_rs,
+                                            const uint16_t* __restrict__ out, int64_t out_rs,
+                                            const float* __restrict__ lse, int bh, int64_t bx, int64_t n, int64_t np,
+                                            float* __restrict__ neg_delta, float* __restrict__ lse_pad) {
+  constexpr int LPR = D / 8, RPP = 256 / LPR, PASSES = 64 / RPP;
+  const int tid = threadIdx.x, c8 = tid % LPR, rr = tid / LPR;
+  const int64_t tok0 = bx * 64;
+#pragma unroll
+  for (int ps = 0; ps < PASSES; ++ps) {
+    const int64_t t = tok0 + rr + ps * RPP;
+    const int64_t row = min(t, n - 1);
+    const uint4 a = *reinterpret_cast<const uint4*>(dout + row * dout_rs + c8 * 8);
+    const uint4 o = *reinterpret_cast<const uint4*>(out + row * out_rs + c8 * 8);
+    float s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int sh = (e & 1) * 16;
+      s += bf16_to_f32((uint16_t)(word_of(a, e >> 1) >> sh)) * bf16_to_f32((uint16_t)(word_of(o, e >> 1) >> sh));
+    }
+#pragma unroll
+    for (int off = 1; off < LPR; off <<= 1) s += __shfl_xor(s, off);
+    if (c8 == 0) {
+      const float l = lse[(int64_t)bh * n + min(t, n - 1)];
+      neg_delta[(int64_t)bh * np + t] = t < n ? -s : 0.0f;
+      lse_pad[(int64_t)bh * np + t] = t < n && l > -INFINITY ? l : INFINITY;
+    }
+  }
 }
 
 // V of one 64-token block: per-channel fp8 scales and codes, or bf16, in the
@@ -709,6 +766,30 @@ __device__ __forceinline__ void v_block(const uint16_t* src, int64_t stride, int
 #pragma unroll
   for (int i = tid; i < VBYTES / 16; i += 256)
     reinterpret_cast<uint4*>(vo)[i] = reinterpret_cast<const uint4*>(vimg)[i];
+}
+
+// The unit of a launch's V role: V of one block, or the backward's per-query values.
+template <int D, int PV>
+__device__ __forceinline__ void v_unit(const QuantExtra<PV>& extra, const uint16_t* src, int64_t stride, int64_t tok0,
+                                       int64_t n, int64_t blk, int bh, int64_t np, uint8_t* __restrict__ vout,
+                                       float* __restrict__ vs, uint8_t* lds, int tid) {
+  if constexpr (PV == kPV_BWD) {
+    const BwdPrep& a = extra.prep;
+    const int b = bh / a.h, h = bh - b * a.h;
+    delta_block<D>(a.dout + b * a.dout_bs + h * a.dout_hs, a.dout_rs, a.out + b * a.out_bs + h * a.out_hs, a.out_rs,
+                   a.lse, bh, blk, n, np, a.neg_delta, a.lse_pad);
+  } else {
+    v_block<D, PV>(src, stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
+  }
+}
+
+// The smoothed rows of head bh that the backward's K units write.
+template <int D, int PV>
+__device__ __forceinline__ uint16_t* kt_rows(const QuantExtra<PV>& extra, int bh, int64_t n) {
+  if constexpr (PV == kPV_BWD)
+    return extra.prep.kt + (int64_t)bh * n * D;
+  else
+    return nullptr;
 }
 
 // fp64 column sums of K over one chunk (k_sum_tokens tokens) of one head.
@@ -830,7 +911,7 @@ __global__ void __launch_bounds__(256) quantize_qv_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t bhn,
     int64_t n, int64_t np, float fold, double* __restrict__ ksum_part, uint8_t* __restrict__ qc,
     float* __restrict__ qs, uint8_t* __restrict__ kc, float* __restrict__ ks, uint8_t* __restrict__ vout,
-    float* __restrict__ vs, ProdArgs prod) {
+    float* __restrict__ vs, QuantExtra<PV> prod) {
   using L = QuantLds<D, PV>;
   constexpr int ROLES = SMOOTH ? 2 : 3;
   __shared__ __attribute__((aligned(16))) uint8_t lds[L::kTotal];
@@ -859,7 +940,7 @@ __global__ void __launch_bounds__(256) quantize_qv_kernel(
   const int64_t co = (int64_t)bh * np * D;
   const int64_t sco = (GRAN == kGRAN_TOKEN) ? (int64_t)bh * np : (int64_t)bh * (np / 64);
   if (role == 1) {
-    v_block<D, PV>(src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
+    v_unit<D, PV>(prod, src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
     return;
   }
   if (GRAN == kGRAN_BLOCK64) {
@@ -878,11 +959,11 @@ __global__ void __launch_bounds__(256) quantize_qv_kernel(
 // 64-token blocks of one head (the padded length is a multiple of 128),
 // shifted by the head's mean; 1D grid, unit y * BH + head.  The chunk sums
 // are loaded first (needed first), then the K rows.
-template <int D, int QK, int GRAN, bool PROD>
+template <int D, int QK, int PV, int GRAN, bool PROD>
 __global__ void __launch_bounds__(256) quantize_k_kernel(const uint16_t* __restrict__ k, int64_t bhn, int64_t n,
                                                          int64_t np, const double* __restrict__ ksum_part,
                                                          uint8_t* __restrict__ kc, float* __restrict__ ks,
-                                                         uint16_t* __restrict__ kmean, ProdArgs prod) {
+                                                         uint16_t* __restrict__ kmean, QuantExtra<PV> prod) {
   constexpr int TPC = 256 / D;
   constexpr int PASSES = 64 / (256 / (D / 8));
   __shared__ double msum[TPC][D];
@@ -904,12 +985,14 @@ __global__ void __launch_bounds__(256) quantize_k_kernel(const uint16_t* __restr
   const int64_t co = (int64_t)bh * np * D;
   const int64_t sco = (GRAN == kGRAN_TOKEN) ? (int64_t)bh * np : (int64_t)bh * (np / 64);
   const ProdRows pr{&prod, prod.kw, src.row0};
+  constexpr bool KT = PV == kPV_BWD;
+  uint16_t* kt = kt_rows<D, PV>(prod, bh, n);
   if (tok0 + 128 <= n) {
-    rows_quant<D, QK, GRAN, PROD, false>(w0, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[0], tid);
-    rows_quant<D, QK, GRAN, PROD, false>(w1, pr, tok0 + 64, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[1], tid);
+    rows_quant<D, QK, GRAN, PROD, false, KT>(w0, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[0], tid, kt);
+    rows_quant<D, QK, GRAN, PROD, false, KT>(w1, pr, tok0 + 64, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[1], tid, kt);
   } else {
-    rows_quant<D, QK, GRAN, PROD, true>(w0, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[0], tid);
-    rows_quant<D, QK, GRAN, PROD, true>(w1, pr, tok0 + 64, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[1], tid);
+    rows_quant<D, QK, GRAN, PROD, true, KT>(w0, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[0], tid, kt);
+    rows_quant<D, QK, GRAN, PROD, true, KT>(w1, pr, tok0 + 64, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[1], tid, kt);
   }
 }
 
@@ -962,6 +1045,12 @@ __device__ __forceinline__ double head_sum_part(bool ready, const HeadRows<D, PR
 // and the kernel runs in 51.5 instead of 58 us at 1x4416x30x128 (6 waves:
 // spills, slower).
 constexpr int kProdWaves = 5;
+
+// Waves per SIMD quantize_one_kernel is compiled for (1: no bound).  The
+// backward form would take 102 VGPRs left to itself and 69 at 7 waves; 5, 7
+// and 8 waves measured the same (849.3-849.9 us for the 1x30x4416 backward).
+template <int PV, bool PROD>
+constexpr int kOneWaves = PROD ? kProdWaves : PV == kPV_BWD ? 7 : 1;
 
 // Slab units of the producer form with per-token scales: a Q or K unit takes
 // the RPP tokens of one pass (lane (rr, c8): token s0 + rr, channels
@@ -1086,12 +1175,12 @@ struct SlabLds {
 // of block r - lag.  A K slab unit waits for its heads' mean flags (bounded,
 // with the chunk-sum fallback).
 template <int D, int QK, int PV, int GRAN, bool PROD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PROD ? kProdWaves : 1))) quantize_one_kernel(
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kOneWaves<PV, PROD>))) quantize_one_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t bhn,
     int64_t n, int64_t np, float fold, double* __restrict__ ksum_part, uint64_t* __restrict__ flags,
     uint64_t epoch, int spin_limit, int64_t lag, uint8_t* __restrict__ qc, float* __restrict__ qs,
     uint8_t* __restrict__ kc, float* __restrict__ ks, uint8_t* __restrict__ vout, float* __restrict__ vs,
-    uint16_t* __restrict__ kmean, ProdArgs prod) {
+    uint16_t* __restrict__ kmean, QuantExtra<PV> prod) {
   using L = QuantLds<D, PV>;
   constexpr bool SLAB = PROD && GRAN == kGRAN_TOKEN;
   constexpr int TPC = 256 / D;
@@ -1262,7 +1351,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PROD ?
       const HeadRows<D, PROD> src(q, k, v, prod, bh, n);
       const int64_t tok0 = blk * 64;
       if (role == 1) {
-        v_block<D, PV>(src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
+        v_unit<D, PV>(prod, src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
         return;
       }
       if (GRAN == kGRAN_BLOCK64) {
@@ -1313,10 +1402,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PROD ?
     const int64_t co = (int64_t)bh * np * D;
     const int64_t sco = (GRAN == kGRAN_TOKEN) ? (int64_t)bh * np : (int64_t)bh * (np / 64);
     const ProdRows pr{&prod, prod.kw, src.row0};
+    constexpr bool KT = PV == kPV_BWD;
+    uint16_t* kt = kt_rows<D, PV>(prod, bh, n);
     if (tok0 + 64 <= n)
-      rows_quant<D, QK, GRAN, PROD, false>(w, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, blk_amax, tid);
+      rows_quant<D, QK, GRAN, PROD, false, KT>(w, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, blk_amax, tid, kt);
     else
-      rows_quant<D, QK, GRAN, PROD, true>(w, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, blk_amax, tid);
+      rows_quant<D, QK, GRAN, PROD, true, KT>(w, pr, tok0, n, 1.0f, mu, kc + co, ks + sco, blk_amax, tid, kt);
   }
 }
 
@@ -1339,7 +1430,7 @@ __global__ void __launch_bounds__(256) quantize_fused_kernel(
     int64_t n, int64_t np, float fold, double* __restrict__ ksum_part, uint64_t* __restrict__ flags,
     uint64_t epoch, int spin_limit, uint8_t* __restrict__ qc, float* __restrict__ qs, uint8_t* __restrict__ kc,
     float* __restrict__ ks, uint8_t* __restrict__ vout, float* __restrict__ vs, uint16_t* __restrict__ kmean,
-    ProdArgs prod) {
+    QuantExtra<PV> prod) {
   using L = QuantLds<D, PV>;
   constexpr int LPR = D / 8;
   constexpr int RPP = 256 / LPR;
@@ -1360,7 +1451,7 @@ __global__ void __launch_bounds__(256) quantize_fused_kernel(
     const int64_t blk = (u - nch) >> 1;
     const int64_t tok0 = blk * 64;
     if (role == 1) {
-      v_block<D, PV>(src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
+      v_unit<D, PV>(prod, src.v, src.stride, tok0, n, blk, bh, np, vout, vs, lds, tid);
       return;
     }
     if (GRAN == kGRAN_BLOCK64) {
@@ -1427,15 +1518,19 @@ __global__ void __launch_bounds__(256) quantize_fused_kernel(
   const float* mu = reinterpret_cast<const float*>(lds + TPC * D * 8);
   const int64_t co = (int64_t)bh * np * D;
   const int64_t sco = (GRAN == kGRAN_TOKEN) ? (int64_t)bh * np : (int64_t)bh * (np / 64);
+  constexpr bool KT = PV == kPV_BWD;
+  uint16_t* kt = kt_rows<D, PV>(prod, bh, n);
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     const int64_t t0 = tok0 + 64 * b;
     __builtin_amdgcn_sched_barrier(0);  // one block at a time
     if (t0 >= np) break;  // uniform: blocks past the padded length hold no codes
     if (t0 + 64 <= n)
-      rows_quant<D, QK, GRAN, false, false>(w[b], ProdRows{}, t0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[b], tid);
+      rows_quant<D, QK, GRAN, false, false, KT>(w[b], ProdRows{}, t0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[b], tid,
+                                                kt);
     else
-      rows_quant<D, QK, GRAN, false, true>(w[b], ProdRows{}, t0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[b], tid);
+      rows_quant<D, QK, GRAN, false, true, KT>(w[b], ProdRows{}, t0, n, 1.0f, mu, kc + co, ks + sco, &blk_amax[b], tid,
+                                               kt);
   }
 }
 
@@ -1471,6 +1566,7 @@ struct QuantCall {
   float* vs;
   uint16_t* kmean;
   ProdArgs prod;
+  const BwdPrep* prep;  // the backward form's operands (kPV_BWD)
   int path;  // kQuantAuto, kQuantTwoKernels, kQuantOneFallback, kQuantLagged
 };
 
@@ -1490,6 +1586,11 @@ template <int D, int QK, int PV, int GRAN, bool SMOOTH, bool PROD>
 hipError_t launch_quantize_t(const QuantCall& a, hipStream_t st) {
   const int64_t np = padded_len(a.n);
   const int64_t nblk = np / 64;
+  QuantExtra<PV> extra{};
+  if constexpr (PV == kPV_BWD)
+    extra.prep = *a.prep;
+  else
+    extra = a.prod;
   if constexpr (SMOOTH) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     const hipError_t ce = hipStreamIsCapturing(st, &cap);
@@ -1509,7 +1610,7 @@ hipError_t launch_quantize_t(const QuantCall& a, hipStream_t st) {
           const int64_t grid = a.bh * (nch + 2 * nblk);
           hipLaunchKernelGGL((quantize_fused_kernel<D, QK, PV, GRAN>), dim3((unsigned)grid), dim3(256), 0, st,
                              a.q, a.k, a.v, a.bh, a.n, np, a.fold, a.ws, flags, next_epoch(), spin, a.qc, a.qs,
-                             a.kc, a.ks, a.vout, a.vs, a.kmean, a.prod);
+                             a.kc, a.ks, a.vout, a.vs, a.kmean, extra);
           return hipGetLastError();
         }
       }
@@ -1521,7 +1622,7 @@ hipError_t launch_quantize_t(const QuantCall& a, hipStream_t st) {
       const int64_t lag = min(nblk, (kLagUnits + 2 * a.bh - 1) / (2 * a.bh));
       hipLaunchKernelGGL((quantize_one_kernel<D, QK, PV, GRAN, PROD>), dim3((unsigned)grid), dim3(256), 0, st, a.q,
                          a.k, a.v, a.bh, a.n, np, a.fold, a.ws, flags, next_epoch(), spin, lag, a.qc, a.qs, a.kc,
-                         a.ks, a.vout, a.vs, a.kmean, a.prod);
+                         a.ks, a.vout, a.vs, a.kmean, extra);
       return hipGetLastError();
     }
   }
@@ -1529,10 +1630,10 @@ hipError_t launch_quantize_t(const QuantCall& a, hipStream_t st) {
   const int64_t nsum = SMOOTH ? k_sum_chunks(a.n, D) * a.bh : 0;
   hipLaunchKernelGGL((quantize_qv_kernel<D, QK, PV, GRAN, SMOOTH, PROD>), dim3((unsigned)(nsum + ROLES * nblk * a.bh)),
                      dim3(256), 0, st, a.q, a.k, a.v, a.bh, a.n, np, a.fold, a.ws, a.qc, a.qs, a.kc, a.ks, a.vout,
-                     a.vs, a.prod);
+                     a.vs, extra);
   if (SMOOTH) {
-    hipLaunchKernelGGL((quantize_k_kernel<D, QK, GRAN, PROD>), dim3((unsigned)(nblk / 2 * a.bh)), dim3(256), 0, st,
-                       a.k, a.bh, a.n, np, a.ws, a.kc, a.ks, a.kmean, a.prod);
+    hipLaunchKernelGGL((quantize_k_kernel<D, QK, PV, GRAN, PROD>), dim3((unsigned)(nblk / 2 * a.bh)), dim3(256), 0,
+                       st, a.k, a.bh, a.n, np, a.ws, a.kc, a.ks, a.kmean, extra);
   }
   return hipGetLastError();
 }
@@ -1561,9 +1662,30 @@ hipError_t launch_quantize(int qk, int pv, int gran, bool smooth, const uint16_t
                            const uint16_t* v, int64_t bh, int64_t n, int64_t d, float fold, double* ws,
                            uint8_t* qc, float* qs, uint8_t* kc, float* ks, uint8_t* vout, float* vs,
                            uint16_t* kmean, const ProdArgs& prod, hipStream_t st) {
-  const QuantCall a{q, k, v, bh, n, fold, ws, qc, qs, kc, ks, vout, vs, kmean, prod, quant_path()};
+  const QuantCall a{q, k, v, bh, n, fold, ws, qc, qs, kc, ks, vout, vs, kmean, prod, nullptr, quant_path()};
   if (d == 128) return launch_quantize_d<128>(qk, pv, gran, smooth, a, st);
   if (d == 64) return launch_quantize_d<64>(qk, pv, gran, smooth, a, st);
+  return hipErrorInvalidValue;
+}
+
+template <int D>
+hipError_t launch_quantize_bwd_d(int qk, bool smooth, const QuantCall& a, hipStream_t st) {
+  constexpr int T = kGRAN_TOKEN;
+  if (qk == kQK_INT8)
+    return smooth ? launch_quantize_t<D, kQK_INT8, kPV_BWD, T, true, false>(a, st)
+                  : launch_quantize_t<D, kQK_INT8, kPV_BWD, T, false, false>(a, st);
+  return smooth ? launch_quantize_t<D, kQK_FP8, kPV_BWD, T, true, false>(a, st)
+                : launch_quantize_t<D, kQK_FP8, kPV_BWD, T, false, false>(a, st);
+}
+
+hipError_t launch_quantize_bwd(int qk, bool smooth, const uint16_t* q, const uint16_t* k, int64_t bh, int64_t n,
+                               int64_t d, float fold, double* ws, uint8_t* qc, float* qs, uint8_t* kc, float* ks,
+                               uint16_t* kmean, const BwdPrep& prep, hipStream_t st) {
+  // no unit reads the V pointer: k stands in for it
+  const QuantCall a{q,  k,  k,       bh,      n,     fold,       ws,    qc,          qs,
+                    kc, ks, nullptr, nullptr, kmean, ProdArgs{}, &prep, quant_path()};
+  if (d == 128) return launch_quantize_bwd_d<128>(qk, smooth, a, st);
+  if (d == 64) return launch_quantize_bwd_d<64>(qk, smooth, a, st);
   return hipErrorInvalidValue;
 }
 

@@ -281,3 +281,23 @@ def test_backward_reads_merged_heads_in_place(cuda, B, H, N, D):
         got = SA.sage_backward(qg, kg, vg, o, lse, g, sm, qk="int8", smooth_k=True)
         for name, a, b_ in zip(("dq", "dk", "dv"), got, want):
             assert a.is_contiguous() and torch.equal(a, b_), name
+
+
+@pytest.mark.parametrize("B,H,N,D", [(1, 2, 1, 64), (2, 3, 257, 128), (1, 2, 700, 64)])
+@pytest.mark.parametrize("smooth", [True, False])
+def test_backward_forms_of_the_quantization_agree(cuda, monkeypatch, B, H, N, D, smooth):
+    """The quantization's backward form (smoothed K rows, -D, padded LSE) gives
+    the same gradients, bit for bit, through every form of the launch: two
+    kernels (as under capture), lagged, single-read, and the fallback sums."""
+    from futudiffu_amd import sage_attention as SA
+    q, k, v, dout = _inputs(B, H, N, D, seed=31 + N)
+    sm = 1.0 / math.sqrt(D)
+    qg, kg, vg, dog = (t.to(cuda) for t in (q, k, v, dout))
+    print(f"bwd quantization forms {B}x{H}x{N}x{D} smooth={smooth}", flush=True)
+    out, lse = SA.sage_forward(qg, kg, vg, sm, qk="int8", pv="bf16", smooth_k=smooth)
+    want = SA.sage_backward(qg, kg, vg, out, lse, dog, sm, qk="int8", smooth_k=smooth)
+    for form in ("two", "lagged", "fused", "fallback"):
+        monkeypatch.setenv("SAGE_QUANT_PATH", form)
+        got = SA.sage_backward(qg, kg, vg, out, lse, dog, sm, qk="int8", smooth_k=smooth)
+        for name, a, b_ in zip(("dq", "dk", "dv"), got, want):
+            assert torch.equal(a, b_), f"{form} {name}"
