@@ -113,10 +113,10 @@ int check_producer(const void* qkv, const float* q_norm_w, const float* k_norm_w
   for (const void* p : ptrs)
     if (!aligned16(p)) return fail(SAGE_ERR_ALIGN, "tensor pointers must be 16-byte aligned");
   if (!(norm_eps >= 0.0f)) return fail(SAGE_ERR_ARG, "norm_eps must be >= 0");
-  // the producer's backward: one workgroup per (64-token block, head) in a 1D grid
+  // at most one launch's workgroups of one per (64-token block, head)
   if (b * h * ((n + 63) / 64) > kMaxGridUnits)
     return fail(SAGE_ERR_ARG, "b*h*ceil(n/64) = %lld exceeds the grid limit", (long long)(b * h * ((n + 63) / 64)));
-  // the standalone producer: one per (pass of 256/(d/8) tokens, group of kSlabHeads heads)
+  // the standalone producer and its backward: one per (pass of 256/(d/8) tokens, group of kSlabHeads heads)
   const int64_t rpp = 256 / (d / 8);
   const int64_t slabs = b * ((n + rpp - 1) / rpp) * ((h + sage::kSlabHeads - 1) / sage::kSlabHeads);
   if (slabs > kMaxGridUnits)

@@ -188,6 +188,35 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// The sums over a token's LPR lanes of G per-token values (the tree of
+// tokens_rrms, reduce-scattered): lane p of a quad gets token p % G's, valid
+// in quads 1 and 3 of each 16-lane row (from_odd_quads hands them on).
+template <int LPR, int G>
+__device__ __forceinline__ double scatter_sums(const double (&ss)[G], int tid) {
+  const bool b0 = tid & 1, b1 = tid & 2;
+  double s;
+  if constexpr (G == 4) {
+    // lanes l, l^1: keep tokens b0 and b0 + 2, hand over b0^1 and (b0^1) + 2
+    const double a0 = (b0 ? ss[1] : ss[0]) + dpp_f64<0xB1>(b0 ? ss[0] : ss[1]);
+    const double a2 = (b0 ? ss[3] : ss[2]) + dpp_f64<0xB1>(b0 ? ss[2] : ss[3]);
+    // lanes l, l^2: keep token b0 + 2*b1
+    s = (b1 ? a2 : a0) + dpp_f64<0x4E>(b1 ? a0 : a2);
+  } else {
+    s = (b0 ? ss[1] : ss[0]) + dpp_f64<0xB1>(b0 ? ss[0] : ss[1]);  // keep token b0
+    s += dpp_f64<0x4E>(s);
+  }
+  // quads q and q^1 of the token: quad r reads quad r - 1 (row_ror:4), valid
+  // in quads 1 and 3; LPR 16: half-rows (row_ror:8), valid in quads 1 and 3
+  s += dpp_f64<0x124>(s);
+  if constexpr (LPR == 16) s += dpp_f64<0x128>(s);
+  return s;
+}
+
+// Quads 0 and 2 of a 16-lane row (banks 0 and 2) take the next quad's values (row_shl:4).
+__device__ __forceinline__ float from_odd_quads(float r) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(r), __float_as_int(r), 0x104, 0xf, 0x5, false));
+}
+
 // Reciprocal RMS of the G tokens (G = 2 or 4) of which a lane holds channels
 // [8*c8, +8) (w[g]: token g), rrms = 1 / sqrt(mean(x^2) + eps) over each
 // token's D channels (fused_kernels.py:316-320), returned in every lane of a
@@ -218,27 +247,10 @@ __device__ __forceinline__ float tokens_rrms(const uint4 (&w)[G], float eps, int
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss[g] = __builtin_fma((double)x[e], (double)x[e], ss[g]);
   }
-  const bool b0 = tid & 1, b1 = tid & 2;
-  double s;
-  if constexpr (G == 4) {
-    // lanes l, l^1: keep tokens b0 and b0 + 2, hand over b0^1 and (b0^1) + 2
-    const double a0 = (b0 ? ss[1] : ss[0]) + dpp_f64<0xB1>(b0 ? ss[0] : ss[1]);
-    const double a2 = (b0 ? ss[3] : ss[2]) + dpp_f64<0xB1>(b0 ? ss[2] : ss[3]);
-    // lanes l, l^2: keep token b0 + 2*b1
-    s = (b1 ? a2 : a0) + dpp_f64<0x4E>(b1 ? a0 : a2);
-  } else {
-    s = (b0 ? ss[1] : ss[0]) + dpp_f64<0xB1>(b0 ? ss[0] : ss[1]);  // keep token b0
-    s += dpp_f64<0x4E>(s);
-  }
-  // quads q and q^1 of the token: quad r reads quad r - 1 (row_ror:4), valid
-  // in quads 1 and 3; LPR 16: half-rows (row_ror:8), valid in quads 1 and 3
-  s += dpp_f64<0x124>(s);
-  if constexpr (LPR == 16) s += dpp_f64<0x128>(s);
+  const double s = scatter_sums<LPR, G>(ss, tid);
   const float ms = (float)(s / (double)D);
-  float r = 1.0f / sqrtf(ms + eps);  // correctly rounded sqrt and division
-  // quads 0 and 2 (banks 0 and 2) take the next quad's (row_shl:4)
-  r = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(r), __float_as_int(r), 0x104, 0xf, 0x5, false));
-  return r;
+  const float r = 1.0f / sqrtf(ms + eps);  // correctly rounded sqrt and division
+  return from_odd_quads(r);
 }
 
 // RMSNorm + rotary embedding of the 8 channels [8*c8, +8) of one token held
@@ -287,22 +299,6 @@ __device__ __forceinline__ void load_w8(const float* w, int c8, float (&out)[8])
   for (int i = 0; i < 4; ++i) {
     out[i] = a[i];
     out[4 + i] = b[i];
-  }
-}
-
-// Block coordinates (unit, bh).  Reading bf16 q, k, v [BH, N, D], the 2D grid
-// (units, BH) walks one head's units.  The projection output [B, N, 3*H*D]
-// holds every head in each token row, so producer launches use a 1D grid with
-// the head fastest: consecutive workgroups read all heads of the same rows.
-template <bool PROD>
-__device__ __forceinline__ void block_coords(const ProdArgs& prod, int64_t& unit, int& bh) {
-  if constexpr (PROD) {
-    const int64_t b = blockIdx.x;
-    unit = b / prod.bh;
-    bh = (int)(b - unit * prod.bh);
-  } else {
-    unit = blockIdx.x;
-    bh = (int)blockIdx.y;
   }
 }
 
@@ -392,8 +388,12 @@ __global__ void __launch_bounds__(256) qkv_postprocess_kernel(ProdArgs prod, int
 // and k; v's gradient passes through; all written in the [B, N, 3*H*D]
 // layout (:778-783).  fp32 arithmetic with fp64 row sums (8 channels per lane,
 // then the token's lanes); the norm weights and rotations get no gradient, as
-// in the reference.  One workgroup per (64-token block, head), head fastest;
-// lane (rr, c8) holds channels [8*c8, +8) of tokens rr + RPP*ps.
+// in the reference.  Memory-bound (275 MB at 1x30x4416x128): the units are
+// those of qkv_postprocess_kernel, so a token's rotations (as many bytes as one
+// head's q and its gradient) are read once for eight heads, four heads' loads are in
+// flight together, and each lane forms the sqrt and divisions of one head of
+// the four instead of all.  One workgroup per (64-token block, head) before:
+// 66.2 -> 53.9 us at that size, 5.1 TB/s, the rate of a large copy.
 template <int D>
 __global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod, int64_t n,
                                                                   const uint16_t* __restrict__ gq,
@@ -402,64 +402,76 @@ __global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod,
                                                                   uint16_t* __restrict__ dqkv) {
   constexpr int LPR = D / 8;
   constexpr int RPP = 256 / LPR;
-  constexpr int PASSES = 64 / RPP;
-  int64_t unit;
-  int bh;
-  block_coords<true>(prod, unit, bh);
   const int tid = threadIdx.x;
   const int c8 = tid % LPR, rr = tid / LPR;
-  const int64_t tok0 = unit * 64;
-  const HeadRows<D, true> src(nullptr, nullptr, nullptr, prod, bh, n);
-  const int64_t head_off = (int64_t)(bh % prod.h) * D;  // the head's column offset in each third
-  const int64_t third = (int64_t)prod.h * D;
-  float qn[8], kn[8];
-  load_w8(prod.qw, c8, qn);
-  load_w8(prod.kw, c8, kn);
-  auto one = [&](uint4 xw, uint4 gw, const float (&w)[8], const f32x4 (&fr)[4]) __attribute__((always_inline)) {
-    float x[8], g[8], gp[8];
-    unpack8(xw, x);
-    unpack8(gw, g);
+  const int64_t ngb = (prod.h + kSlabHeads - 1) / kSlabHeads, nsl = (n + RPP - 1) / RPP;
+  const int64_t unit = blockIdx.x;
+  const int64_t bs = unit / ngb;  // b * nsl + slab
+  const int b = (int)(bs / nsl);
+  const int64_t s0 = (bs - (int64_t)b * nsl) * RPP;
+  const int h0 = (int)(unit - bs * ngb) * kSlabHeads, h1 = min(h0 + kSlabHeads, prod.h);
+  const int64_t t = s0 + rr;
+  const bool valid = t < n;
+  const int64_t tc = valid ? t : n - 1;  // clamped: the lanes of a token reduce together
+  f32x4 fr[4];
+  load_freqs<D>(prod.freqs, (int64_t)b * n + tc, c8, fr);
+  const int64_t hd = (int64_t)prod.h * D;
+  const int64_t row = ((int64_t)b * n + tc) * 3 * hd + c8 * 8;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {  // transpose of [[cos, -sin], [sin, cos]]
-      const float c = fr[p][0], sn = fr[p][2];
-      gp[2 * p] = (c * g[2 * p] + sn * g[2 * p + 1]) * w[2 * p];
-      gp[2 * p + 1] = (c * g[2 * p + 1] - sn * g[2 * p]) * w[2 * p + 1];
-    }
-    double ss = 0.0, gx = 0.0;
+  for (int it = 0; it < kSlabHeads / 4; ++it) {
+    const int hb = h0 + 4 * it;
+    if (hb >= h1) break;  // uniform
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      ss = __builtin_fma((double)x[e], (double)x[e], ss);
-      gx = __builtin_fma((double)gp[e], (double)x[e], gx);
-    }
-    ss = token_sum<LPR>(ss);
-    gx = token_sum<LPR>(gx);
-    const float rrms = 1.0f / sqrtf((float)(ss / (double)D) + prod.eps);
-    const float cr = (float)(gx / (double)D) * rrms * rrms;
-    uint32_t o[4];
+    for (int m = 0; m < 3; ++m) {
+      const uint16_t* grad = m == 0 ? gq : m == 1 ? gk : gv;
+      uint4 gw[4], xw[4];
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-      o[p] = pack_bf16x2(rrms * (gp[2 * p] - x[2 * p] * cr), rrms * (gp[2 * p + 1] - x[2 * p + 1] * cr));
-    return make_uint4(o[0], o[1], o[2], o[3]);
-  };
+      for (int j = 0; j < 4; ++j) {
+        const int64_t hh = min(hb + j, h1 - 1);
+        gw[j] = *reinterpret_cast<const uint4*>(grad + (((int64_t)b * prod.h + hh) * n + tc) * D + c8 * 8);
+        if (m < 2) xw[j] = *reinterpret_cast<const uint4*>(prod.qkv + row + m * hd + hh * D);
+      }
+      if (m < 2) {
+        float w[8], gp[4][8];
+        load_w8(m == 0 ? prod.qw : prod.kw, c8, w);
+        double ss[4], gx[4];
 #pragma unroll
-  for (int ps = 0; ps < PASSES; ++ps) {
-    const int64_t t = tok0 + rr + ps * RPP;
-    const int64_t tok = min(t, n - 1);  // clamped: the lanes of a token reduce together
-    const int64_t gofs = ((int64_t)bh * n + tok) * D + c8 * 8;
-    const uint4 xq = *reinterpret_cast<const uint4*>(src.q + tok * src.stride + c8 * 8);
-    const uint4 xk = *reinterpret_cast<const uint4*>(src.k + tok * src.stride + c8 * 8);
-    const uint4 g_q = *reinterpret_cast<const uint4*>(gq + gofs);
-    const uint4 g_k = *reinterpret_cast<const uint4*>(gk + gofs);
-    const uint4 g_v = *reinterpret_cast<const uint4*>(gv + gofs);
-    f32x4 fr[4];
-    load_freqs<D>(prod.freqs, src.row0 + tok, c8, fr);
-    const uint4 dq = one(xq, g_q, qn, fr);
-    const uint4 dk = one(xk, g_k, kn, fr);
-    if (t < n) {
-      uint16_t* row = dqkv + (src.row0 + t) * 3 * third + head_off + c8 * 8;
-      *reinterpret_cast<uint4*>(row) = dq;
-      *reinterpret_cast<uint4*>(row + third) = dk;
-      *reinterpret_cast<uint4*>(row + 2 * third) = g_v;
+        for (int j = 0; j < 4; ++j) {
+          float x[8], g[8];
+          unpack8(xw[j], x);
+          unpack8(gw[j], g);
+          ss[j] = 0.0;
+          gx[j] = 0.0;
+#pragma unroll
+          for (int p = 0; p < 4; ++p) {  // transpose of [[cos, -sin], [sin, cos]]
+            const float c = fr[p][0], sn = fr[p][2];
+            gp[j][2 * p] = (c * g[2 * p] + sn * g[2 * p + 1]) * w[2 * p];
+            gp[j][2 * p + 1] = (c * g[2 * p + 1] - sn * g[2 * p]) * w[2 * p + 1];
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            ss[j] = __builtin_fma((double)x[e], (double)x[e], ss[j]);
+            gx[j] = __builtin_fma((double)gp[j][e], (double)x[e], gx[j]);
+          }
+        }
+        const float r1 = 1.0f / sqrtf((float)(scatter_sums<LPR, 4>(ss, tid) / (double)D) + prod.eps);
+        const float c1 = (float)(scatter_sums<LPR, 4>(gx, tid) / (double)D) * r1 * r1;
+        const float rq = from_odd_quads(r1), cq = from_odd_quads(c1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float rrms = quad_lane(rq, j), cr = quad_lane(cq, j);
+          float x[8];
+          unpack8(xw[j], x);
+          uint32_t o[4];
+#pragma unroll
+          for (int p = 0; p < 4; ++p)
+            o[p] = pack_bf16x2(rrms * (gp[j][2 * p] - x[2 * p] * cr), rrms * (gp[j][2 * p + 1] - x[2 * p + 1] * cr));
+          gw[j] = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (valid && hb + j < h1) *reinterpret_cast<uint4*>(dqkv + row + m * hd + (int64_t)(hb + j) * D) = gw[j];
     }
   }
 }
@@ -1705,7 +1717,9 @@ hipError_t launch_qkv_postprocess(const ProdArgs& prod, int64_t bh, int64_t n, i
 
 hipError_t launch_qkv_postprocess_bwd(const ProdArgs& prod, int64_t bh, int64_t n, int64_t d, const uint16_t* gq,
                                       const uint16_t* gk, const uint16_t* gv, uint16_t* dqkv, hipStream_t st) {
-  const dim3 grid((unsigned)((n + 63) / 64 * bh));  // head fastest (block_coords)
+  const int64_t rpp = 256 / (d / 8);  // tokens per slab
+  const int64_t groups = (prod.h + kSlabHeads - 1) / kSlabHeads;
+  const dim3 grid((unsigned)((bh / prod.h) * ((n + rpp - 1) / rpp) * groups));
   if (d == 128)
     hipLaunchKernelGGL(qkv_postprocess_bwd_kernel<128>, grid, dim3(256), 0, st, prod, n, gq, gk, gv, dqkv);
   else if (d == 64)

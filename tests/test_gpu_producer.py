@@ -141,6 +141,13 @@ def test_producer_backward_matches_oracle(cuda, B, N, H, D):
     assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} beyond one bf16 step, worst {err.max().item():.3e}"
 
 
+# head counts around the units' four and eight heads, tokens around their 16 or
+# 32, over several batches
+@pytest.mark.parametrize("B,N,H,D", [(3, 1, 1, 64), (2, 17, 5, 128), (2, 33, 8, 64), (2, 300, 9, 128), (3, 129, 12, 64)])
+def test_producer_backward_head_groups(cuda, B, N, H, D):
+    test_producer_backward_matches_oracle(cuda, B, N, H, D)
+
+
 def test_autograd_through_fused_qkv_postprocess(cuda):
     import futudiffu_amd.fused_kernels  # noqa: F401  (registers futudiffu::fused_qkv_postprocess)
     B, N, H, D = 1, 200, 2, 128
