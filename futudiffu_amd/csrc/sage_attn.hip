@@ -1480,9 +1480,9 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
     // the split items and leave partials; the last piece of an item to arrive
     // merges them (merge_pieces), or merge_split_kernel does after the launch
     // (unmasked launches only).  A tile-masked item's pieces are equal shares
-    // of its active tiles, kMinPiece at least: it uses only as many of its
+    // of its active tiles, at least 4 of them beside a full round and at least
+    // 12 where every item is cut (tail_split): it uses only as many of its
     // workgroups as that gives, the others exit.
-    constexpr int kMinPiece = 4;
     const int64_t b = blockIdx.x;
     if (b >= p.n_whole) {
       const int64_t c = b - p.n_whole;
@@ -1495,7 +1495,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
       if constexpr (MASK == 1) {
         const uint8_t* row = mask_row(p, bh, qt);
         const int count = active_count(row, p.nt);
-        parts = max(1, min(parts, count / kMinPiece));
+        parts = max(1, min(parts, p.n_whole == 0 ? count / 12 : count / 4));
         if (part >= parts) return;
         t0 = nth_active(row, p.nt, (int)((int64_t)part * count / parts));
         t1 = part + 1 < parts ? nth_active(row, p.nt, (int)((int64_t)(part + 1) * count / parts)) : p.nt;
@@ -1786,7 +1786,7 @@ AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool ma
   const int64_t nt = (n + 63) / 64;
   const int64_t items = b * h * (np / kRowsPerWG);
   AttnWorkspace w;
-  w.split = tail_split(items, nt);
+  w.split = tail_split(items, nt, d);
   w.doc_off = 0;
   // summaries (int4), the per-query-tile scheduled ranges (int4), then the
   // list of split query tiles (a count and kHeavyMax entries)

@@ -70,7 +70,7 @@ constexpr int kResidentWGs = 512;
 template <int D>
 constexpr int64_t kPartFloats = 128 * D + 2 * 256;
 
-// Tail split of an unmasked launch of n_items 128-row items of nt key tiles:
+// Split of an unmasked launch of n_items 128-row items of nt key tiles:
 // whole items fill complete rounds of the resident workgroups; the items of
 // the last, partial round are cut into `parts` ranges of key tiles (at most
 // 4), chosen to minimize (rounds the pieces take) x (tiles per piece + 2
@@ -91,14 +91,39 @@ constexpr int64_t kPartFloats = 128 * D + 2 * 256;
 // items: 54.3 / 57.7 / 59.6 us in 2 / 3 / 4 pieces).  With the merge inside
 // the attention kernel, 300 items: 34.4 us in 2 pieces, 31.7 / 31.6 in 3 / 4,
 // 33.1 in 5.
+//
+// Launches of no more items than CUs: each item walks all its tiles alone (1.05
+// us a tile) while CUs idle, so every item is cut, from 24 tiles on.  At most
+// 128 items: pieces of 10 tiles or more, as many as there are CUs for (3x3000,
+// 72 items of 47 tiles: 53.6 us whole, 30.6 in 3 pieces, 36.8 / 38.7 in 4 / 6
+// that share CUs), since a piece's start, partial and share of the merge cost
+// some 7 us (16x1024, 16 tiles: 21.3 -> 23.5 in 2; 2x2048, 32 tiles: 37.4 ->
+// 24.0 in 3 of 10, 27.4 in 2 of 16, 26.3 in 5 of 6).  More items: the pieces
+// must share CUs, which pays from 48 tiles (D=64: 140 items of 69 tiles 61.5 ->
+// 42.4 us, 240 of 60 tiles 54.3 -> 50.2, 192 of 32 tiles 30.6 -> 31.6).  The
+// partials stay within the allocation-free entry point's scratch (small_slots),
+// so that it takes every such launch: at D=128 up to 123 items.
 struct TailSplit {
   int64_t whole;
   int parts;
 };
 
-inline TailSplit tail_split(int64_t n_items, int64_t nt) {
+// Partial slots (128 x D + 512 floats) in 16 MiB less 64 KiB for the rest of
+// the workspace, whose summaries take under 32 KiB at 256 items.
+inline constexpr int64_t small_slots(int64_t d) { return ((16 << 20) - (64 << 10)) / ((128 * d + 512) * 4); }
+
+inline TailSplit tail_split(int64_t n_items, int64_t nt, int64_t d) {
   TailSplit t{n_items, 1};
   constexpr int64_t kCUs = kResidentWGs / 2;
+  if (n_items <= kCUs) {
+    const bool share = n_items > kCUs / 2;
+    if (nt < (share ? 48 : 24)) return t;
+    const int64_t room = share ? (int64_t)kResidentWGs : kCUs, slots = small_slots(d);
+    int64_t parts = (room < slots ? room : slots) / n_items;
+    parts = parts < 8 ? parts : 8;
+    parts = parts < nt / 10 ? parts : nt / 10;
+    return parts > 1 ? TailSplit{0, (int)parts} : t;
+  }
   if (n_items > kCUs && n_items < kResidentWGs) {
     const int64_t spill = n_items - kCUs;
     if (spill <= 128 && nt >= 2) {

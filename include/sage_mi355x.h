@@ -172,8 +172,9 @@ int sage_quantize_from_qkv(const void* qkv, const float* q_norm_w, const float* 
  * key-tile range of every 128-row query block (written and used when doc_ids
  * is given), then the fp32 partial results of the key-tile pieces of
  * the 128-row items that an unmasked launch splits (the items past the last
- * whole round of 512 resident workgroups) and an 8-byte arrival counter per
- * split item (the last piece to finish merges the item's partials; the
+ * whole round of 512 resident workgroups; below one round the items past one
+ * per CU; every item of a launch of fewer items than CUs and enough key tiles)
+ * and an 8-byte arrival counter per split item (the last piece to finish merges the item's partials; the
  * counters need no clearing, each call tags them with a value no earlier
  * call used).  Enough for every launch of that shape.  No reference
  * counterpart (the Triton launch needs no workspace). */
@@ -182,7 +183,7 @@ size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 /* Bytes of device workspace a sage_attn_fwd launch with a tile_mask or
  * doc_ids needs: the summaries only (a few KB; 7 KB for the packed 1x30x6912
  * batch).  A tile-masked launch without doc_ids that is given room for them
- * (sage_attn_workspace_bytes) splits its last items like an unmasked one: as
+ * (sage_attn_workspace_bytes) splits its items like an unmasked one: as
  * many of them as keep the partials within SAGE_NOALLOC_SCRATCH_BYTES, so
  * sage_attn_fwd_noalloc cuts the same ones.  No reference counterpart. */
 size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);

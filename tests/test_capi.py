@@ -85,6 +85,27 @@ def test_sizes_and_padding():
         assert lib.sage_attn_masked_workspace_bytes(b, h, n, d) == doc
 
 
+def test_few_items_workspace_fits_the_allocation_free_entry():
+    """A launch of at most 256 items cuts them all from 24 key tiles on (48 past
+    128 items); its partials stay within the allocation-free entry point's
+    scratch, which took every such launch before."""
+    from futudiffu_amd import _lib
+    lib = _lib.load()
+    cut = 0
+    for b, h, d in ((1, 1, 128), (1, 1, 64), (2, 1, 128), (1, 3, 128), (1, 4, 64), (4, 8, 128), (240, 1, 64)):
+        for n in range(64, 32768 // (b * h) + 1, 64):
+            need = lib.sage_attn_workspace_bytes(b, h, n, d)
+            assert need <= 16 << 20, (b, h, n, d)
+            items, nt = b * h * ((n + 127) // 128), n // 64
+            has = need > lib.sage_attn_masked_workspace_bytes(b, h, n, d)
+            cut += has
+            if nt < (24 if items <= 128 else 48):
+                assert not has, (b, h, n, d)
+            elif items <= 120:
+                assert has, (b, h, n, d)
+    assert cut > 100
+
+
 def _quant_call(lib, **over):
     a = dict(q=16, k=32, v=48, bh=2, n=100, d=128, qk=0, pv=1, gran=0, smooth=1, fold=0.18,
              qc=64, qs=80, kc=96, ks=112, vo=128, vs=144, km=160, ws=None, wsb=0, stream=None)

@@ -208,3 +208,42 @@ def test_tile_masked_tail_split(cuda, pv, D):
         assert (got - want.float()[:, :, see]).abs().max().item() <= 2e-2
         assert O.cosine(got, want[:, :, see]) >= 0.999
         assert (lse[hh].cpu()[see] - wl[0][see]).abs().max().item() <= 2e-3
+
+
+def test_tile_masked_few_items_cut(cuda):
+    """Two heads of 1921 tokens are 32 items of 31 key tiles, cut into up to
+    three shares of at least 12 active tiles: a 3D mask gives the items 0 to 31
+    active tiles, scattered ones, on both sides of 24.  Against the uncut launch
+    (a workspace of the masked size), to the rounding of P in another frame."""
+    from futudiffu_amd import _lib
+    from futudiffu_amd import sage_attention as SA
+    B, H, N, D, nq, nkv = 1, 2, 1921, 128, 16, 31
+    lib = _lib.load()
+    q, k, v = (t.to(cuda) for t in O.make_inputs(B, H, N, D, seed=95))
+    g = torch.Generator().manual_seed(96)
+    mask = torch.zeros(H, nq, nkv, dtype=torch.uint8)
+    for i in range(H * nq):
+        mask[i // nq, i % nq, torch.randperm(nkv, generator=g)[:i]] = 1
+    mask[0, 0] = 1
+    mask[1, 3] = 0
+    mg = mask.to(cuda)
+    live = mask.sum(2).repeat_interleave(128, 1)[:, :N] > 0
+    for pv in ("bf16", "fp8"):
+        print(f"masked few items int8/{pv}", flush=True)
+        qz = SA.quantize_qkv(q, k, v, qk="int8", pv=pv)
+        out, lse = SA.attn_from_quantized(qz, B, H, block_mask=mg)
+        wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))
+        assert wsb < int(lib.sage_attn_workspace_bytes(B, H, N, D))
+        ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+        o1, l1 = torch.empty_like(out), torch.empty_like(lse)
+        _lib.check(lib.sage_attn_fwd(
+            qz.q_codes.data_ptr(), qz.q_scale.data_ptr(), qz.k_codes.data_ptr(), qz.k_scale.data_ptr(),
+            qz.v_op.data_ptr(), SA._ptr(qz.v_scale), B, H, N, D, 0, SA._PV[pv], 0, mg.data_ptr(), nq * nkv, nq, nkv,
+            None, ws.data_ptr(), wsb, o1.data_ptr(), 0, l1.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(torch.isfinite(lse).cpu(), live) and torch.equal(torch.isfinite(l1).cpu(), live)
+        assert not out[0][~live.to(cuda)].float().any()
+        # the bound of test_tile_masked_tail_split: one bf16 step of an output up to 2
+        assert (out.float() - o1.float()).abs().max().item() <= 8e-3
+        fin = live.to(cuda)
+        assert (lse[fin] - l1[fin]).abs().max().item() <= 1e-4

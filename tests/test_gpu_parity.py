@@ -453,6 +453,34 @@ def test_split_items_merged_in_kernel_as_by_merge_kernel(cuda, monkeypatch, B, H
         _assert_bits_equal(lse, want_lse, f"lse, call {i}")
 
 
+@pytest.mark.parametrize("B,H,N,D,qk,pv", [(1, 1, 1472, 128, "int8", "bf16"), (1, 2, 1473, 128, "int8", "fp8"),
+                                           (2, 1, 1857, 64, "fp8", "bf16"), (1, 1, 5121, 128, "int8", "bf16"),
+                                           (1, 6, 3073, 64, "int8", "fp8")])
+def test_few_items_cut_over_the_chip(cuda, monkeypatch, B, H, N, D, qk, pv):
+    """Launches of at most 256 items cut every item from 24 key tiles on: 23
+    tiles (whole), 24 with a ragged last one (2 pieces), 30 over two batches
+    (3), 81 (8, the cap), and 150 items of 49 tiles whose pieces share CUs (3).
+    The merge by the last piece gives the merge kernel's bits, and the result
+    agrees with the oracle."""
+    SA = _sa()
+    q, k, v = O.make_inputs(B, H, N, D, seed=71 + N)
+    print(f"few items {B}x{H}x{N}x{D} {qk}/{pv}", flush=True)
+    qz = SA.quantize_qkv(q.to(cuda), k.to(cuda), v.to(cuda), qk=qk, pv=pv)
+    monkeypatch.setenv("SAGE_MERGE", "kernel")
+    want, want_lse = SA.attn_from_quantized(qz, B, H)
+    torch.cuda.synchronize()
+    monkeypatch.delenv("SAGE_MERGE")
+    for i in range(2):
+        out, lse = SA.attn_from_quantized(qz, B, H)
+        torch.cuda.synchronize()
+        _assert_bits_equal(out, want, f"out, call {i}")
+        _assert_bits_equal(lse, want_lse, f"lse, call {i}")
+    if N <= 2048:  # every head
+        _compare(out, lse, q, k, v, qk, pv, "token")
+    else:  # one head: the oracle's N x N scores
+        _compare(out[:, -1:], lse.view(B, H, N)[:, -1], q[:, -1:], k[:, -1:], v[:, -1:], qk, pv, "token")
+
+
 @pytest.mark.parametrize("qk", ["int8", "fp8"])
 @pytest.mark.parametrize("N", [64, 65, 128, 192, 250, 320, 500])
 def test_bf16_loop_without_row_max(cuda, N, qk):
