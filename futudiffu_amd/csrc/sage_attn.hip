@@ -1786,13 +1786,13 @@ AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool ma
   const int64_t nt = (n + 63) / 64;
   const int64_t items = b * h * (np / kRowsPerWG);
   AttnWorkspace w;
-  w.split = tail_split(items, nt, d);
+  w.split = masked ? TailSplit{items, 1} : tail_split(items, nt, d);
   w.doc_off = 0;
   // summaries (int4), the per-query-tile scheduled ranges (int4), then the
   // list of split query tiles (a count and kHeavyMax entries)
   w.heavy_off = (size_t)(b * (nt + np / 32 + np / 128 + np / 128)) * sizeof(int4);
   w.part_off = (w.heavy_off + (size_t)(1 + kHeavyMax) * sizeof(int4) + 255) & ~(size_t)255;
-  int64_t split_items = !masked && w.split.parts > 1 ? items - w.split.whole : 0;
+  int64_t split_items = items - w.split.whole;
   if (limit != 0 && split_items > 0) {
     const int64_t item_bytes = w.split.parts * (128 * d + 512) * (int64_t)sizeof(float) + (int64_t)sizeof(uint64_t);
     const int64_t room = (int64_t)limit - (int64_t)w.part_off;

@@ -342,11 +342,14 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   memset(&p, 0, sizeof(p));
   // Masked launches need no partial slots.  With a tile mask alone and a
   // workspace that has room for them all the same (sage_attn_workspace_bytes,
-  // or the scratch of the allocation-free entry point), the last items are
+  // or the scratch of the allocation-free entry point), items are
   // split as in an unmasked launch: the production op is always masked, and at
   // 1x30x4416 its 1050 items leave a third round of 26.  The pieces' slots stay
   // within that scratch, so every entry point cuts the same items.
   sage::AttnWorkspace ws = sage::attn_workspace(b, h, n, d, mask != 0);
+  // a launch whose every item is cut runs whole in a workspace of the summaries
+  // alone, the size it needs without the cut
+  if (mask == 0 && ws.split.whole == 0 && workspace_bytes < ws.bytes) ws = sage::attn_workspace(b, h, n, d, true);
   bool masked_split = false;
   if (mask == 1 && merge_in_kernel()) {
     const sage::AttnWorkspace split = sage::attn_workspace(b, h, n, d, false, SAGE_NOALLOC_SCRATCH_BYTES);

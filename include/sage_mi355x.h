@@ -176,8 +176,10 @@ int sage_quantize_from_qkv(const void* qkv, const float* q_norm_w, const float* 
  * per CU; every item of a launch of fewer items than CUs and enough key tiles)
  * and an 8-byte arrival counter per split item (the last piece to finish merges the item's partials; the
  * counters need no clearing, each call tags them with a value no earlier
- * call used).  Enough for every launch of that shape.  No reference
- * counterpart (the Triton launch needs no workspace). */
+ * call used).  Enough for every launch of that shape; a launch of fewer items
+ * than CUs also takes a workspace of the summaries alone, and runs its items
+ * whole then.  No reference counterpart (the Triton launch needs no
+ * workspace). */
 size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
 /* Bytes of device workspace a sage_attn_fwd launch with a tile_mask or

@@ -475,6 +475,19 @@ def test_few_items_cut_over_the_chip(cuda, monkeypatch, B, H, N, D, qk, pv):
         torch.cuda.synchronize()
         _assert_bits_equal(out, want, f"out, call {i}")
         _assert_bits_equal(lse, want_lse, f"lse, call {i}")
+    # a workspace of the summaries alone runs the items whole
+    from futudiffu_amd import _lib
+    lib = _lib.load()
+    wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+    o1, l1 = torch.empty_like(out), torch.empty_like(lse)
+    _lib.check(lib.sage_attn_fwd(
+        qz.q_codes.data_ptr(), qz.q_scale.data_ptr(), qz.k_codes.data_ptr(), qz.k_scale.data_ptr(),
+        qz.v_op.data_ptr(), SA._ptr(qz.v_scale), B, H, N, D, SA._QK[qk], SA._PV[pv], 0, None, 0, 0, 0, None,
+        ws.data_ptr(), wsb, o1.data_ptr(), 0, l1.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert (out.float() - o1.float()).abs().max().item() <= 8e-3  # one bf16 step of an output up to 2
+    assert (lse - l1).abs().max().item() <= 1e-4
     if N <= 2048:  # every head
         _compare(out, lse, q, k, v, qk, pv, "token")
     else:  # one head: the oracle's N x N scores
