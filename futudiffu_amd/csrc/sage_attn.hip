@@ -31,7 +31,7 @@
 // O and l are kept in a lazily moved frame: they hold sums of 2^(s - m_ref),
 // where the per-row reference point m_ref only moves when a block max exceeds
 // it by more than kTau (then O and l are rescaled, which is rare after the
-// first tiles).  The LSE is m_ref + log2(l), the reference's m + log2(l).
+// first tiles; the pipelined bf16 loop finds such a block by its sum of P).  The LSE is m_ref + log2(l), the reference's m + log2(l).
 // fp8 P follows the reference per (row, 64-key block) scaling
 // (sage_kernels.py:1137-1141): with bm the block's row max, the code argument
 // is e = 2^(s - bm) * 448 (= p * 448 / max(p)), and the block's PV product is

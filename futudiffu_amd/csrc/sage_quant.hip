@@ -19,7 +19,9 @@
 // through flags tagged with a per-call epoch.  Under stream capture the
 // launch uses two kernels instead (quantize_qv_kernel, quantize_k_kernel):
 // a captured epoch would repeat on every replay.  Both forms write the same
-// bits.
+// bits.  In the backward's form (kPV_BWD) the V role forms -rowsum(dO * O) and
+// the padded LSE of a block instead of V codes, and the K role also writes the
+// smoothed rows bf16(k - mean) that the dQ pass multiplies by.
 #include "sage_common.h"
 #include "sage_launch.h"
 
