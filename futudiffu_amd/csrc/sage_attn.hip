@@ -10,10 +10,11 @@
 // query rows.  Keys stream in 64-key tiles (the reference KV tile, which is
 // also the V-scale block) through a ring of LDS stages filled by direct
 // global -> LDS loads: tile i+2 is issued while tile i is consumed and tile
-// i+1 already feeds the next S^T; one barrier per tile.  Without document
-// ids (and with them for fp8 P.V) the loop is software-pipelined: the P.V of
-// tile i-1 is formed in iteration i, its MFMAs under tile i's score
-// conversion and softmax.
+// i+1 already feeds the next S^T; one barrier per tile.  The loop is
+// software-pipelined: the P.V of tile i-1 is formed in iteration i, its MFMAs
+// under tile i's score conversion and softmax.  With document ids the tiles up
+// to the last that some wave does not see whole go through a general loop
+// first, one tile after the other with a per-element visibility test.
 //
 // Per wave and tile:
 //   S^T[key][query] = K . Q^T with v_mfma_i32_32x32x32_i8 (int8) or
@@ -134,8 +135,7 @@ __global__ void __launch_bounds__(256) doc_summary_kernel(const int32_t* __restr
 
 // LDS stage layout (bytes): K codes, V operand, then a contiguous region of
 // per-key K scales (token granularity) and per-channel V scales (fp8 P.V),
-// then per-key document ids.  Every part except the document ids arrives by
-// direct global -> LDS loads.
+// then per-key document ids.  Every part arrives by direct global -> LDS loads.
 template <int D, int PV>
 struct Stage {
   static constexpr int kBytes = 64 * D;
@@ -210,6 +210,10 @@ constexpr int32_t kC0Bits = 0x3E22F983;
 constexpr float kC0 = 0.15915494309189535f;
 static_assert(__builtin_bit_cast(int32_t, kC0) == kC0Bits, "c0 must be the inline constant 1/(2 pi)");
 constexpr float kC0Scale = 67108864.0f;  // 2^26, the accumulator's ulp inverted
+// fp8 P.V with document ids gains more from the subtraction than from the
+// registers; every other loop starts from 0.
+template <int PV, int MASK>
+constexpr bool kFromC0 = PV == kPV_FP8 && (MASK & 2) != 0;
 template <bool C0>
 __device__ __forceinline__ i32x16 i8_start() {
   if constexpr (C0)
@@ -748,7 +752,7 @@ __device__ __forceinline__ void tile_body(const uint8_t* sb, const uint8_t* sb_n
   using St = Stage<D, PV>;
   constexpr int NC = D / 32;
   const int h = lane >> 5, r = lane & 31;
-  constexpr bool C0 = (MASK & 2) != 0;  // the int8 chains' start (i8_start)
+  constexpr bool C0 = kFromC0<PV, MASK>;  // the int8 chains' start (i8_start)
   float u[2][16];
   half_scores<D, QK, PV, GRAN, MASKED, C0>(sb, s0, 0, h, kd_blk, kvalid, true, dq, u[0]);
   half_scores<D, QK, PV, GRAN, MASKED, C0>(sb, s1, 1, h, kd_blk, kvalid, true, dq, u[1]);
@@ -801,6 +805,7 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
   using SM = Smem<D, PV>;
   using SAcc = typename SAccT<QK>::type;
   constexpr int NC = D / 32;  // 32-channel chunks
+  constexpr bool DOC = (MASK & 2) != 0;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int h = lane >> 5, r = lane & 31;
   const int nq = (int)(p.np / kRowsPerWG);
@@ -826,8 +831,7 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     qd = p.qs[(int64_t)bh * p.np + q0 + r];
   else
     qd = p.qs[(int64_t)bh * (p.np / 64) + (q0 >> 6)];
-  // the int8 chains' start (i8_start): from c0 with document ids
-  constexpr bool kC0Start = (MASK & 2) != 0;
+  constexpr bool kC0Start = kFromC0<PV, MASK>;  // the int8 chains' start (i8_start)
   // log2-domain multiplier of the (K-scaled) accumulators; int8 QK scores
   // started from c0 carry 2^-26, which the multiplier takes back exactly
   const float w = fmaxf(qd, 1e-30f) * (QK == kQK_INT8 && kC0Start ? kC0Scale : 1.0f);
@@ -863,12 +867,10 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
 
   // ---- loads: global -> LDS stage --------------------------------------------
   // The K and V parts in 64-chunk blocks spread over the four waves, the K and
-  // V scales by lanes of wave 0, all as direct global -> LDS loads; the key
-  // document ids (bounds-checked: -1 past N) through registers of threads
-  // 48..63.  The caller waits for vmcnt(0) before the barrier that publishes
+  // V scales by lanes of wave 0, the key document ids by lanes of wave 1, all
+  // as direct global -> LDS loads.  The caller waits for vmcnt(0) before the barrier that publishes
   // the stage.
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  int4 pre_doc = make_int4(-1, -1, -1, -1);
   // buffer resources over this head's K and V operands and scales: the stage
   // copies take a scalar tile offset and a loop-invariant lane offset
   const __amdgpu_buffer_rsrc_t rs_k = raw_rsrc(kg, (uint32_t)(p.np * D));
@@ -876,14 +878,13 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
   const __amdgpu_buffer_rsrc_t rs_ks = raw_rsrc(p.ks + (int64_t)bh * p.np, (uint32_t)(p.np * 4));
   const __amdgpu_buffer_rsrc_t rs_vs =
       raw_rsrc(PV == kPV_FP8 ? p.vs + (int64_t)bh * (p.np / 64) * D : p.ks, (uint32_t)(p.np / 64 * D * 4));
-  // document ids of the keys, copied like the scales (fp8 P.V).  The whole
+  // document ids of the keys, copied like the scales.  The whole
   // offset goes in the vector operand, the part the buffer range check
   // covers (per dword for a 16-byte load), so ids past N read as 0 and no
   // byte past the caller's [B, N] array is fetched; no score sees those ids,
   // since keys past N are masked by count
-  constexpr bool kDocDma = (MASK & 2) && PV == kPV_FP8;
   const __amdgpu_buffer_rsrc_t rs_doc =
-      raw_rsrc(kDocDma ? static_cast<const void*>(docb) : static_cast<const void*>(p.ks), (uint32_t)(p.n * 4));
+      raw_rsrc(DOC ? static_cast<const void*>(docb) : static_cast<const void*>(p.ks), (uint32_t)(p.n * 4));
   auto load_k = [&](int tt, uint8_t* sbw) __attribute__((always_inline)) {
     dma_chunks_buf<St::cK, 4>(sbw, wave_u, lane, rs_k, tt * 64 * D);
   };
@@ -898,22 +899,12 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
       if (PV == kPV_FP8 && lane >= 16 && lane < 16 + D / 4)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_vs, sbw + St::offKd, 16, (lane - 16) * 16, tt * D * 4, 0, 0);
     }
-    if (kDocDma && wave_u == 1 && lane < 16)
+    if (DOC && wave_u == 1 && lane < 16)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_doc, sbw + St::offDoc, 16, tt * 256 + lane * 16, 0, 0, 0);
-    if (!kDocDma && (MASK & 2) && tid >= 48 && tid < 64) {
-      const int64_t base = (int64_t)tt * 64 + (tid - 48) * 4;
-      pre_doc.x = base + 0 < p.n ? docb[base + 0] : -1;
-      pre_doc.y = base + 1 < p.n ? docb[base + 1] : -1;
-      pre_doc.z = base + 2 < p.n ? docb[base + 2] : -1;
-      pre_doc.w = base + 3 < p.n ? docb[base + 3] : -1;
-    }
   };
   auto load_tile = [&](int tt, uint8_t* sbw) __attribute__((always_inline)) {
     load_k(tt, sbw);
     load_v(tt, sbw);
-  };
-  auto store_doc = [&](uint8_t* sbw) __attribute__((always_inline)) {
-    if (!kDocDma && (MASK & 2) && tid >= 48 && tid < 64) reinterpret_cast<int4*>(sbw + St::offDoc)[tid - 48] = pre_doc;
   };
   auto kd_block = [&](int tt) -> float {
     return GRAN == kGRAN_TOKEN ? 0.0f : load_uniform(p.ks, (int64_t)bh * (p.np / 64) + tt);
@@ -940,20 +931,19 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     }
   };
 
-  constexpr bool DOC = (MASK & 2) != 0;
-  // the software-pipelined loop: every fp8 P.V variant, and bf16 P.V without
-  // document ids
-  constexpr bool kFast = PV == kPV_FP8 || !DOC;
   // bf16 P.V on the pipelined loop keeps three stages: a tile's K part is
   // loaded two tiles ahead and its V part (with the scales) one tile ahead,
   // so the K of tile i+2 goes into the stage whose V (tile i-1) the pending
   // product still reads
-  constexpr bool kSplit = kFast && PV == kPV_BF16;
+  constexpr bool kSplit = PV == kPV_BF16;
   // Document ids: the item's scheduled tiles lie in [range.x, range.z), and
-  // with fp8 P.V the tiles before prefix_end (one past the last that some
+  // the tiles before prefix_end (one past the last that some
   // live wave does not see whole, from doc_prefix_kernel) go through the
   // general tile body with its per-element visibility test; the pipelined
-  // loop computes every scheduled tile in every live wave with no test.
+  // loop computes every scheduled tile in every live wave with no test.  bf16
+  // P.V all in the general loop took 427 us on the packed 1x30x6912 batch and
+  // 1146 us on 4x30x4352 with padded keys; so it takes 352 and 977 us (int8 QK;
+  // fp8 QK 390 -> 332, 1049 -> 911).
   int prefix_end = t_begin;
   if constexpr (DOC) {
     const int4 range = load_uniform(p.doc_range, (int64_t)bidx * nq + qt);
@@ -965,7 +955,7 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     t_begin = listed ? t_end : t_begin;
     t_begin = max(t_begin, range.x);
     t_end = min(t_end, range.z);
-    if constexpr (kFast) prefix_end = range.y;
+    prefix_end = range.y;
   }
   // ---- prologue: tiles 0 and 1 of the schedule in stages 0 and 1 --------------
   int t = next_active(t_begin);
@@ -973,15 +963,12 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
   int t2 = t1 < t_end ? next_active(t1 + 1) : t_end;
   if (t < t_end) {
     load_tile(t, smem);
-    store_doc(smem);
   }
   if (t1 < t_end) {
-    if constexpr (kSplit) {
+    if constexpr (kSplit && !DOC)
       load_k(t1, smem + St::bytes);
-    } else {
-      load_tile(t1, smem + St::bytes);
-      store_doc(smem + St::bytes);
-    }
+    else
+      load_tile(t1, smem + St::bytes);  // the general loop takes whole tiles
   }
   wait_vmem();
   __syncthreads();
@@ -1019,7 +1006,6 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
       qk_both<D, QK, kC0Start>(sb_next, qf, lane, s0, s1);
 
     // ---- publish tile t2 ---------------------------------------------------------
-    if (t2 < t_end) store_doc(smem + stage2 * St::bytes);
     wait_vmem();
     __syncthreads();
     stage = stage1;
@@ -1027,225 +1013,217 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
     t1 = t2;
     t2 = t2 < t_end ? next_active(t2 + 1) : t_end;
   };
-  if constexpr (kFast) {
-    // ---- every scheduled tile is computed by every live wave, so the product
-    // of tile i-1 is always pending in iteration i.  The first and the last
-    // tile are peeled off the loop, which leaves its body one straight basic
-    // block for the scheduler: the pending P.V in two chunk-pair halves, each
-    // under half of this tile's score conversion, then the next tile's S^T
-    // under this tile's softmax.  fp8: the pending product's MFMAs and their
-    // dequantization into O; bf16: its MFMAs accumulate into O, after the
-    // frame move the previous softmax decided (deferred to here, so the
-    // softmax never waits for the product in flight).  With document ids
-    // (fp8) the tiles before prefix_end, which some live wave does not see
-    // whole, go through the general body first; every later scheduled tile
-    // is seen whole by every live wave.
-    constexpr int NP = NC / 2;
-    int stage = 0;
-    if constexpr (DOC) {
-      while (t < t_end && t < prefix_end) general_step(stage);
+  // ---- every scheduled tile is computed by every live wave, so the product
+  // of tile i-1 is always pending in iteration i.  The first and the last
+  // tile are peeled off the loop, which leaves its body one straight basic
+  // block for the scheduler: the pending P.V in two chunk-pair halves, each
+  // under half of this tile's score conversion, then the next tile's S^T
+  // under this tile's softmax.  fp8: the pending product's MFMAs and their
+  // dequantization into O; bf16: its MFMAs accumulate into O, after the
+  // frame move the previous softmax decided (deferred to here, so the
+  // softmax never waits for the product in flight).  With document ids
+  // (fp8) the tiles before prefix_end, which some live wave does not see
+  // whole, go through the general body first; every later scheduled tile
+  // is seen whole by every live wave.
+  constexpr int NP = NC / 2;
+  int stage = 0;
+  if constexpr (DOC) {
+    while (t < t_end && t < prefix_end) general_step(stage);
+  }
+  auto sp = [&](int s_) { return smem + s_ * St::bytes; };
+  auto next_stage = [&](int s_, int k_) { return (s_ + k_) % kSt; };
+  auto advance = [&]() __attribute__((always_inline)) {
+    stage = next_stage(stage, 1);
+    t = t1;
+    t1 = t2;
+    t2 = t2 < t_end ? next_active(t2 + 1) : t_end;
+  };
+  auto issue_loads = [&]() __attribute__((always_inline)) {
+    if constexpr (kSplit) {
+      if (t2 < t_end) load_k(t2, sp(next_stage(stage, 2)));
+      if (t1 < t_end) load_v(t1, sp(next_stage(stage, 1)));
+    } else {
+      if (t2 < t_end) load_tile(t2, sp(next_stage(stage, 2)));
     }
-    auto sp = [&](int s_) { return smem + s_ * St::bytes; };
-    auto next_stage = [&](int s_, int k_) { return (s_ + k_) % kSt; };
-    auto advance = [&]() __attribute__((always_inline)) {
-      stage = next_stage(stage, 1);
-      t = t1;
-      t1 = t2;
-      t2 = t2 < t_end ? next_active(t2 + 1) : t_end;
-    };
-    auto issue_loads = [&]() __attribute__((always_inline)) {
-      if constexpr (kSplit) {
-        if (t2 < t_end) load_k(t2, sp(next_stage(stage, 2)));
-        if (t1 < t_end) load_v(t1, sp(next_stage(stage, 1)));
-      } else {
-        if (t2 < t_end) load_tile(t2, sp(next_stage(stage, 2)));
-      }
-    };
-    auto publish = [&]() __attribute__((always_inline)) {
-      if (t2 < t_end) store_doc(sp(next_stage(stage, 2)));
-      wait_vmem();
-      __syncthreads();
-    };
-    if (!wave_live) {
-      // rows past N: the same loads and barriers, nothing computed
-      while (t < t_end) {
-        issue_loads();
-        publish();
-        advance();
-      }
-      __syncthreads();
-      return !listed;
-    }
-    const bool any = t < t_end;
-#ifdef SAGE_PHASE_TIMING
-    uint64_t ph_acc[kPhases] = {0, 0, 0, 0, 0, 0};
-    uint64_t ph_last = __builtin_amdgcn_s_memtime();
-    const uint64_t ph_start = ph_last;
-    int ph_n = 0;
-#endif
-    // the pending product: fp8 P codes and their row factor, or bf16 P and
-    // the frame move that precedes its accumulation
-    i32x8 pa_p = {0, 0, 0, 0, 0, 0, 0, 0};
-    float rsc_p = 0.0f;
-    bf16x8 pb_p[2][2];
-    float alpha_p = 1.0f;
-    bool move_p = false;
-    int stage_p = 0;
-    // fp8: the first chunk pair's stage operands of the pending product, read
-    // in the iteration that forms its P codes, before its softmax, whose
-    // vector work covers their LDS latency (the barrier waits for every LDS
-    // access in flight)
-    PvFrags pf0;
-    bf16x8 vf_p[kVAhead];  // bf16: its first V fragments
-    auto prefetch_pending = [&]() __attribute__((always_inline)) {
-      // the tile about to become pending
-      if constexpr (PV == kPV_FP8) {
-        pf0 = pv_load<D>(sp(stage), lane, 0);
-      } else {
-#pragma unroll
-        for (int i = 0; i < kVAhead; ++i) vf_p[i] = v_frag<D>(sp(stage), lane, i);
-      }
-    };
-    float u[2][16];
-    auto softmax_p = [&]() __attribute__((always_inline)) {
-      if constexpr (PV == kPV_FP8)
-        softmax_fp8<D>(u, w, m_ref, l_acc, o, xrow, h, r, pa_p, rsc_p);
-      else
-        move_p = softmax_bf16(u, w, m_ref, l_acc, pb_p, alpha_p);
-    };
-    // the pending product, chunk pair c2 (its frame move first, for bf16)
-    auto pending_pair = [&](const uint8_t* sbp, int c2) __attribute__((always_inline)) {
-      if constexpr (PV == kPV_FP8) {
-        f32x16 p0, p1;
-        f32x32 rv;
-        pv_issue<D>(sbp, pa_p, rsc_p, lane, c2, p0, p1, rv);
-        pv_accum(o, c2, p0, p1, rv);
-      } else {
-        pv_bf16_pair<D>(sbp, pb_p, lane, c2, o);
-      }
-    };
-    auto pending_move = [&]() __attribute__((always_inline)) {
-      if constexpr (PV == kPV_BF16) {
-        if (move_p) frame_move_o<D>(o, xrow, alpha_p, h, r);
-      }
-    };
-    if (t < t_end) {  // first tile: nothing pending
+  };
+  auto publish = [&]() __attribute__((always_inline)) {
+    wait_vmem();
+    __syncthreads();
+  };
+  if (!wave_live) {
+    // rows past N: the same loads and barriers, nothing computed
+    while (t < t_end) {
       issue_loads();
-      dump(t, s0, s1);
-      const float kdb = kd_block(t);
-      const int kvalid = keys_valid(t);
-      half_scores<D, QK, PV, GRAN, false, kC0Start>(sp(stage), s0, 0, h, kdb, kvalid, false, dq, u[0]);
-      half_scores<D, QK, PV, GRAN, false, kC0Start>(sp(stage), s1, 1, h, kdb, kvalid, false, dq, u[1]);
-      if (t1 < t_end) qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
-      prefetch_pending();
-      softmax_p();
-      stage_p = stage;
       publish();
       advance();
     }
-    // one iteration for a whole tile t with a successor
-    auto iteration = [&]() __attribute__((always_inline)) {
-      SAGE_PHASE(0);  // loop overhead since the last iteration's end
-      issue_loads();
-      if constexpr (PV == kPV_BF16) {
-        dump(t, s0, s1);
-        pending_move();
-        move_p = tile_bf16<D, QK, GRAN>(sp(stage), sp(stage_p), sp(next_stage(stage, 1)), qf, lane, kd_block(t), s0,
-                                        s1, o, vf_p, pb_p, w, m_ref, l_acc, alpha_p);
-        prefetch_pending();
-      } else {
-        const uint8_t* sb = sp(stage);
-        const uint8_t* sbp = sp(stage_p);
-        const float kdb = kd_block(t);
-        dump(t, s0, s1);
-        auto scores = [&](int b_, float (&u_)[16]) __attribute__((always_inline)) {
-          half_scores<D, QK, PV, GRAN, false, kC0Start>(sb, b_ ? s1 : s0, b_, h, kdb, 64, false, dq, u_);
-        };
-        f32x16 p0, p1;
-        f32x32 rv;
-        pv_issue_f<D>(pf0, pa_p, rsc_p, p0, p1, rv);
-        scores(0, u[0]);
-        if constexpr (NP == 1) scores(1, u[1]);
-        pv_accum(o, 0, p0, p1, rv);
-        if constexpr (NP == 2) {
-          // fp8 QK: the second pair's products and factors only once the
-          // first pair's are consumed (with the next S^T formed later, both
-          // at once would not fit the registers)
-          if constexpr (QK == kQK_FP8) __builtin_amdgcn_sched_barrier(0);
-          pv_issue<D>(sbp, pa_p, rsc_p, lane, 2, p0, p1, rv);
-          scores(1, u[1]);
-          pv_accum(o, 2, p0, p1, rv);
-        }
-        if constexpr (QK == kQK_FP8 && D == 128) {
-          // fp8 QK, D = 128: the frame decision ends a scheduling region (its
-          // rare O rescale is a branch); the next tile's S^T goes after it,
-          // among the exp / pack work of this tile (A/B at 1x30x4416x128
-          // fp8/fp8: 234.7 -> 230.7 us and 240.3 -> 235.7 us; with int8 QK the
-          // same order measured 247.7 -> 250.8 us: the other wave of the SIMD
-          // already covers the QK^T burst)
-          prefetch_pending();
-          const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
-          softmax_fp8_exp_qk<D>(u, w, bm, m_ref, l_acc, pa_p, rsc_p, sp(next_stage(stage, 1)), qf, lane, s0, s1);
-        } else {
-          SAGE_PHASE(1);  // the pending product and this tile's score conversion
-          qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
-          SAGE_PHASE(2);  // the next tile's QK^T issue
-          prefetch_pending();
-          const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
-          SAGE_PHASE(3);  // row max and frame decision
-          softmax_fp8_exp(u, w, bm, m_ref, l_acc, pa_p, rsc_p);
-          SAGE_PHASE(4);  // exp, row sums, P packing
-        }
-      }
-      stage_p = stage;
-      publish();
-      SAGE_PHASE(5);  // stage loads complete, workgroup barrier
-      advance();
-#ifdef SAGE_PHASE_TIMING
-      ++ph_n;
-#endif
-    };
-    // the pending product, one chunk pair's products in flight at a time
-    auto flush = [&]() __attribute__((always_inline)) {
-      const uint8_t* sbp = sp(stage_p);
-      pending_move();
-#pragma unroll
-      for (int c2 = 0; c2 < NC; c2 += 2) {
-        pending_pair(sbp, c2);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    while (t1 < t_end) iteration();
-    if (t < t_end) {  // last tile: the pending product, then the tile with its P.V formed at once
-      flush();
-      const uint8_t* sb = sp(stage);
-      dump(t, s0, s1);
-      tile_body<D, QK, PV, GRAN, MASK, false>(sb, sb, qf, lane, s0, s1, o, m_ref, l_acc, w, xrow, dq, kd_block(t),
-                                              keys_valid(t));
-      publish();
-      advance();
-    } else if (any) {  // the single tile was also the first: its product is pending
-      flush();
-    }
-#ifdef SAGE_PHASE_TIMING
-    {
-      const uint64_t ph_end = __builtin_amdgcn_s_memtime();
-      const int slot = (int)blockIdx.x * 4 + wave;
-      if (lane == 0 && slot < kPhaseSlots) {
-#pragma unroll
-        for (int k = 0; k < kPhases; ++k) sage_phase_buf[slot][k] += ph_acc[k];
-        sage_phase_buf[slot][6] += (unsigned long long)ph_n;
-        sage_phase_buf[slot][7] += ph_end - ph_start;
-      }
-    }
-#endif
-    __syncthreads();  // the ring is reused after
+    __syncthreads();
     return !listed;
   }
-  if constexpr (!kFast) {
-    int stage = 0;
-    while (t < t_end) general_step(stage);
+  const bool any = t < t_end;
+#ifdef SAGE_PHASE_TIMING
+  uint64_t ph_acc[kPhases] = {0, 0, 0, 0, 0, 0};
+  uint64_t ph_last = __builtin_amdgcn_s_memtime();
+  const uint64_t ph_start = ph_last;
+  int ph_n = 0;
+#endif
+  // the pending product: fp8 P codes and their row factor, or bf16 P and
+  // the frame move that precedes its accumulation
+  i32x8 pa_p = {0, 0, 0, 0, 0, 0, 0, 0};
+  float rsc_p = 0.0f;
+  bf16x8 pb_p[2][2];
+  float alpha_p = 1.0f;
+  bool move_p = false;
+  int stage_p = 0;
+  // fp8: the first chunk pair's stage operands of the pending product, read
+  // in the iteration that forms its P codes, before its softmax, whose
+  // vector work covers their LDS latency (the barrier waits for every LDS
+  // access in flight)
+  PvFrags pf0;
+  bf16x8 vf_p[kVAhead];  // bf16: its first V fragments
+  auto prefetch_pending = [&]() __attribute__((always_inline)) {
+    // the tile about to become pending
+    if constexpr (PV == kPV_FP8) {
+      pf0 = pv_load<D>(sp(stage), lane, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kVAhead; ++i) vf_p[i] = v_frag<D>(sp(stage), lane, i);
+    }
+  };
+  float u[2][16];
+  auto softmax_p = [&]() __attribute__((always_inline)) {
+    if constexpr (PV == kPV_FP8)
+      softmax_fp8<D>(u, w, m_ref, l_acc, o, xrow, h, r, pa_p, rsc_p);
+    else
+      move_p = softmax_bf16(u, w, m_ref, l_acc, pb_p, alpha_p);
+  };
+  // the pending product, chunk pair c2 (its frame move first, for bf16)
+  auto pending_pair = [&](const uint8_t* sbp, int c2) __attribute__((always_inline)) {
+    if constexpr (PV == kPV_FP8) {
+      f32x16 p0, p1;
+      f32x32 rv;
+      pv_issue<D>(sbp, pa_p, rsc_p, lane, c2, p0, p1, rv);
+      pv_accum(o, c2, p0, p1, rv);
+    } else {
+      pv_bf16_pair<D>(sbp, pb_p, lane, c2, o);
+    }
+  };
+  auto pending_move = [&]() __attribute__((always_inline)) {
+    if constexpr (PV == kPV_BF16) {
+      if (move_p) frame_move_o<D>(o, xrow, alpha_p, h, r);
+    }
+  };
+  if (t < t_end) {  // first tile: nothing pending
+    issue_loads();
+    dump(t, s0, s1);
+    const float kdb = kd_block(t);
+    const int kvalid = keys_valid(t);
+    half_scores<D, QK, PV, GRAN, false, kC0Start>(sp(stage), s0, 0, h, kdb, kvalid, false, dq, u[0]);
+    half_scores<D, QK, PV, GRAN, false, kC0Start>(sp(stage), s1, 1, h, kdb, kvalid, false, dq, u[1]);
+    if (t1 < t_end) qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
+    prefetch_pending();
+    softmax_p();
+    stage_p = stage;
+    publish();
+    advance();
   }
+  // one iteration for a whole tile t with a successor
+  auto iteration = [&]() __attribute__((always_inline)) {
+    SAGE_PHASE(0);  // loop overhead since the last iteration's end
+    issue_loads();
+    if constexpr (PV == kPV_BF16) {
+      dump(t, s0, s1);
+      pending_move();
+      move_p = tile_bf16<D, QK, GRAN>(sp(stage), sp(stage_p), sp(next_stage(stage, 1)), qf, lane, kd_block(t), s0,
+                                      s1, o, vf_p, pb_p, w, m_ref, l_acc, alpha_p);
+      prefetch_pending();
+    } else {
+      const uint8_t* sb = sp(stage);
+      const uint8_t* sbp = sp(stage_p);
+      const float kdb = kd_block(t);
+      dump(t, s0, s1);
+      auto scores = [&](int b_, float (&u_)[16]) __attribute__((always_inline)) {
+        half_scores<D, QK, PV, GRAN, false, kC0Start>(sb, b_ ? s1 : s0, b_, h, kdb, 64, false, dq, u_);
+      };
+      f32x16 p0, p1;
+      f32x32 rv;
+      pv_issue_f<D>(pf0, pa_p, rsc_p, p0, p1, rv);
+      scores(0, u[0]);
+      if constexpr (NP == 1) scores(1, u[1]);
+      pv_accum(o, 0, p0, p1, rv);
+      if constexpr (NP == 2) {
+        // fp8 QK: the second pair's products and factors only once the
+        // first pair's are consumed (with the next S^T formed later, both
+        // at once would not fit the registers)
+        if constexpr (QK == kQK_FP8) __builtin_amdgcn_sched_barrier(0);
+        pv_issue<D>(sbp, pa_p, rsc_p, lane, 2, p0, p1, rv);
+        scores(1, u[1]);
+        pv_accum(o, 2, p0, p1, rv);
+      }
+      if constexpr (QK == kQK_FP8 && D == 128) {
+        // fp8 QK, D = 128: the frame decision ends a scheduling region (its
+        // rare O rescale is a branch); the next tile's S^T goes after it,
+        // among the exp / pack work of this tile (A/B at 1x30x4416x128
+        // fp8/fp8: 234.7 -> 230.7 us and 240.3 -> 235.7 us; with int8 QK the
+        // same order measured 247.7 -> 250.8 us: the other wave of the SIMD
+        // already covers the QK^T burst)
+        prefetch_pending();
+        const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
+        softmax_fp8_exp_qk<D>(u, w, bm, m_ref, l_acc, pa_p, rsc_p, sp(next_stage(stage, 1)), qf, lane, s0, s1);
+      } else {
+        SAGE_PHASE(1);  // the pending product and this tile's score conversion
+        qk_both<D, QK, kC0Start>(sp(next_stage(stage, 1)), qf, lane, s0, s1);
+        SAGE_PHASE(2);  // the next tile's QK^T issue
+        prefetch_pending();
+        const float bm = row_max_move<D>(u, w, m_ref, l_acc, o, xrow, h, r);
+        SAGE_PHASE(3);  // row max and frame decision
+        softmax_fp8_exp(u, w, bm, m_ref, l_acc, pa_p, rsc_p);
+        SAGE_PHASE(4);  // exp, row sums, P packing
+      }
+    }
+    stage_p = stage;
+    publish();
+    SAGE_PHASE(5);  // stage loads complete, workgroup barrier
+    advance();
+#ifdef SAGE_PHASE_TIMING
+    ++ph_n;
+#endif
+  };
+  // the pending product, one chunk pair's products in flight at a time
+  auto flush = [&]() __attribute__((always_inline)) {
+    const uint8_t* sbp = sp(stage_p);
+    pending_move();
+#pragma unroll
+    for (int c2 = 0; c2 < NC; c2 += 2) {
+      pending_pair(sbp, c2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  while (t1 < t_end) iteration();
+  if (t < t_end) {  // last tile: the pending product, then the tile with its P.V formed at once
+    flush();
+    const uint8_t* sb = sp(stage);
+    dump(t, s0, s1);
+    tile_body<D, QK, PV, GRAN, MASK, false>(sb, sb, qf, lane, s0, s1, o, m_ref, l_acc, w, xrow, dq, kd_block(t),
+                                            keys_valid(t));
+    publish();
+    advance();
+  } else if (any) {  // the single tile was also the first: its product is pending
+    flush();
+  }
+#ifdef SAGE_PHASE_TIMING
+  {
+    const uint64_t ph_end = __builtin_amdgcn_s_memtime();
+    const int slot = (int)blockIdx.x * 4 + wave;
+    if (lane == 0 && slot < kPhaseSlots) {
+#pragma unroll
+      for (int k = 0; k < kPhases; ++k) sage_phase_buf[slot][k] += ph_acc[k];
+      sage_phase_buf[slot][6] += (unsigned long long)ph_n;
+      sage_phase_buf[slot][7] += ph_end - ph_start;
+    }
+  }
+#endif
+  __syncthreads();  // the ring is reused after
   return !listed;
 }
 

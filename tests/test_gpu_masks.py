@@ -247,3 +247,28 @@ def test_tile_masked_few_items_cut(cuda):
         assert (out.float() - o1.float()).abs().max().item() <= 8e-3
         fin = live.to(cuda)
         assert (lse[fin] - l1[fin]).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("lens", [[64, 64], [40, 88], [40, 150], [100, 220], [130, 258], [70, 1, 400]])
+def test_bf16_document_ids_on_the_pipelined_loop(cuda, lens, D):
+    """bf16 P.V with document ids: the tiles some wave does not see whole go
+    through the general loop, the rest (here none to six, a ragged last one)
+    through the pipelined one; padding keys put mixed tiles before whole ones in
+    the second sample."""
+    from futudiffu_amd import sage_attention as SA
+    n = sum(lens)
+    doc = torch.cat([torch.full((s,), i, dtype=torch.int32) for i, s in enumerate(lens)])
+    pad = torch.zeros(n, dtype=torch.int32)
+    pad[lens[0] // 2: lens[0]] = -1
+    ids = torch.stack([doc, pad])
+    B, H = 2, 2
+    q, k, v = O.make_inputs(B, H, n, D, seed=300 + n)
+    print(f"bf16 document ids {lens} D={D}", flush=True)
+    out, lse = SA.sage_forward(q.to(cuda), k.to(cuda), v.to(cuda), qk="int8", pv="bf16", doc_ids=ids.to(cuda))
+    torch.cuda.synchronize()
+    want, wl, _ = O.sage_forward(q, k, v, None, "int8", "bf16", "token", True, None, ids)
+    # the output bounds of every variant against the reference scheme
+    assert (out.cpu().float() - want.float()).abs().max().item() <= 2e-2
+    assert O.cosine(out.cpu(), want) >= 0.999
+    assert (lse.cpu() - wl.view_as(lse.cpu())).abs().max().item() <= 2e-3
