@@ -395,9 +395,13 @@ __global__ void __launch_bounds__(256) qkv_postprocess_kernel(ProdArgs prod, int
 // head's q and its gradient) are read once for eight heads, four heads' loads are in
 // flight together, and each lane forms the sqrt and divisions of one head of
 // the four instead of all.  One workgroup per (64-token block, head) before:
-// 66.2 -> 53.9 us at that size, 5.1 TB/s, the rate of a large copy.
+// 66.2 -> 53.9 us at that size, 5.1 TB/s, the rate of a large copy.  Launches of
+// fewer such units than two a CU give each of q, k and v, and every four heads,
+// a unit of its own (heads 4, each 1): with eight heads a unit those were
+// slower than before (4x12x83x64 6.3 -> 8.7 us, 1x12x2453x64 10.5 -> 11.1), so
+// they take 4.6 and 9.1 us, 1x30x333x128 10.2 -> 7.0.
 template <int D>
-__global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod, int64_t n,
+__global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod, int64_t n, int heads, int each,
                                                                   const uint16_t* __restrict__ gq,
                                                                   const uint16_t* __restrict__ gk,
                                                                   const uint16_t* __restrict__ gv,
@@ -406,12 +410,13 @@ __global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod,
   constexpr int RPP = 256 / LPR;
   const int tid = threadIdx.x;
   const int c8 = tid % LPR, rr = tid / LPR;
-  const int64_t ngb = (prod.h + kSlabHeads - 1) / kSlabHeads, nsl = (n + RPP - 1) / RPP;
-  const int64_t unit = blockIdx.x;
+  const int64_t ngb = (prod.h + heads - 1) / heads, nsl = (n + RPP - 1) / RPP;
+  const int64_t unit = each ? blockIdx.x / 3 : blockIdx.x;
+  const int m0 = each ? (int)(blockIdx.x % 3) : 0, m1 = each ? m0 + 1 : 3;  // of q, k, v
   const int64_t bs = unit / ngb;  // b * nsl + slab
   const int b = (int)(bs / nsl);
   const int64_t s0 = (bs - (int64_t)b * nsl) * RPP;
-  const int h0 = (int)(unit - bs * ngb) * kSlabHeads, h1 = min(h0 + kSlabHeads, prod.h);
+  const int h0 = (int)(unit - bs * ngb) * heads, h1 = min(h0 + heads, prod.h);
   const int64_t t = s0 + rr;
   const bool valid = t < n;
   const int64_t tc = valid ? t : n - 1;  // clamped: the lanes of a token reduce together
@@ -425,6 +430,7 @@ __global__ void __launch_bounds__(256) qkv_postprocess_bwd_kernel(ProdArgs prod,
     if (hb >= h1) break;  // uniform
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
+      if (m < m0 || m >= m1) continue;  // uniform
       const uint16_t* grad = m == 0 ? gq : m == 1 ? gk : gv;
       uint4 gw[4], xw[4];
 #pragma unroll
@@ -1720,12 +1726,15 @@ hipError_t launch_qkv_postprocess(const ProdArgs& prod, int64_t bh, int64_t n, i
 hipError_t launch_qkv_postprocess_bwd(const ProdArgs& prod, int64_t bh, int64_t n, int64_t d, const uint16_t* gq,
                                       const uint16_t* gk, const uint16_t* gv, uint16_t* dqkv, hipStream_t st) {
   const int64_t rpp = 256 / (d / 8);  // tokens per slab
-  const int64_t groups = (prod.h + kSlabHeads - 1) / kSlabHeads;
-  const dim3 grid((unsigned)((bh / prod.h) * ((n + rpp - 1) / rpp) * groups));
+  const int64_t slabs = (bh / prod.h) * ((n + rpp - 1) / rpp);
+  // two units of eight heads a CU, or four heads of one of q, k, v a unit
+  const bool few = slabs * ((prod.h + kSlabHeads - 1) / kSlabHeads) < kResidentWGs;
+  const int heads = few ? 4 : kSlabHeads, each = few ? 1 : 0;
+  const dim3 grid((unsigned)(slabs * ((prod.h + heads - 1) / heads) * (few ? 3 : 1)));
   if (d == 128)
-    hipLaunchKernelGGL(qkv_postprocess_bwd_kernel<128>, grid, dim3(256), 0, st, prod, n, gq, gk, gv, dqkv);
+    hipLaunchKernelGGL(qkv_postprocess_bwd_kernel<128>, grid, dim3(256), 0, st, prod, n, heads, each, gq, gk, gv, dqkv);
   else if (d == 64)
-    hipLaunchKernelGGL(qkv_postprocess_bwd_kernel<64>, grid, dim3(256), 0, st, prod, n, gq, gk, gv, dqkv);
+    hipLaunchKernelGGL(qkv_postprocess_bwd_kernel<64>, grid, dim3(256), 0, st, prod, n, heads, each, gq, gk, gv, dqkv);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

@@ -142,8 +142,9 @@ def test_producer_backward_matches_oracle(cuda, B, N, H, D):
 
 
 # head counts around the units' four and eight heads, tokens around their 16 or
-# 32, over several batches
-@pytest.mark.parametrize("B,N,H,D", [(3, 1, 1, 64), (2, 17, 5, 128), (2, 33, 8, 64), (2, 300, 9, 128), (3, 129, 12, 64)])
+# 32, over several batches; the last two have two units of eight heads a CU
+@pytest.mark.parametrize("B,N,H,D", [(3, 1, 1, 64), (2, 17, 5, 128), (2, 33, 8, 64), (2, 300, 9, 128), (3, 129, 12, 64),
+                                     (16, 545, 9, 64), (2, 2100, 12, 128)])
 def test_producer_backward_head_groups(cuda, B, N, H, D):
     test_producer_backward_matches_oracle(cuda, B, N, H, D)
 
