@@ -492,6 +492,8 @@ int sage_attn_fwd_noalloc(const void* q_codes, const float* q_scale, const void*
 }
 
 size_t sage_forward_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d, int pv_kind, int with_doc_ids) {
+  // shapes sage_forward refuses: no size, and no division by a chunk count of zero
+  if (b <= 0 || h <= 0 || n <= 0 || (d != 64 && d != 128)) return 0;
   return forward_workspace(b, h, n, d, pv_kind, with_doc_ids != 0).bytes;
 }
 

@@ -115,6 +115,7 @@ inline constexpr int64_t small_slots(int64_t d) { return ((16 << 20) - (64 << 10
 inline TailSplit tail_split(int64_t n_items, int64_t nt, int64_t d) {
   TailSplit t{n_items, 1};
   constexpr int64_t kCUs = kResidentWGs / 2;
+  if (n_items <= 0) return t;  // a workspace size asked for an empty batch
   if (n_items <= kCUs) {
     const bool share = n_items > kCUs / 2;
     if (nt < (share ? 48 : 24)) return t;

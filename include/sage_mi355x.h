@@ -364,7 +364,8 @@ int sage_forward(const void* q, const void* k, const void* v,
                  void* out, int out_layout, float* lse, hipStream_t stream);
 
 /* Bytes of the workspace sage_forward needs (codes, scales, K mean, the V
- * operand and the workspaces of its two parts). */
+ * operand and the workspaces of its two parts); 0 for a shape it refuses (an
+ * empty batch, a head_dim other than 64 and 128). */
 size_t sage_forward_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d,
                                     int pv_kind, int with_doc_ids);
 

@@ -12,6 +12,8 @@
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -104,6 +106,31 @@ def test_few_items_workspace_fits_the_allocation_free_entry():
             elif items <= 120:
                 assert has, (b, h, n, d)
     assert cut > 100
+
+
+_EMPTY_SIZES = '''
+from futudiffu_amd import _lib
+lib = _lib.load()
+for n in (1, 1024, 1473, 4416):
+    for b, h in ((0, 30), (1, 0), (-1, 30)):
+        print(n, b, h, flush=True)
+        lib.sage_attn_workspace_bytes(b, h, n, 128), lib.sage_attn_masked_workspace_bytes(b, h, n, 128)
+        lib.sage_attn_bwd_workspace_bytes(b, h, n, 128)
+        for doc in (0, 1):
+            assert lib.sage_forward_workspace_bytes(b, h, n, 128, 0, doc) == 0
+    for d in (-4, 0, 96, 512):
+        assert lib.sage_forward_workspace_bytes(1, 2, n, d, 1, 0) == 0
+assert lib.sage_forward_workspace_bytes(1, 2, 0, 128, 1, 0) == 0
+assert lib.sage_attn_workspace_bytes(0, 30, 4416, 128) == lib.sage_attn_workspace_bytes(0, 30, 64, 128) == 256
+'''
+
+
+def test_workspace_sizes_of_empty_batches():
+    """The size functions take an empty batch (which the calls then refuse) at
+    every length; in a child process, since a division by its zero items would
+    end the process."""
+    r = subprocess.run([sys.executable, "-c", _EMPTY_SIZES], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-200:], r.stderr[-2000:])
 
 
 def _quant_call(lib, **over):

@@ -162,3 +162,13 @@ def test_gradient_through_the_lse_only(cuda):
     lse.sum().backward()
     for t in (q, k, v):
         assert t.grad is not None and not t.grad.float().any()
+
+
+@pytest.mark.parametrize("N", [100, 1473])
+def test_empty_batch_is_refused(cuda, N):
+    """An empty batch raises the library's error at every length (its workspace
+    size is asked for first)."""
+    from futudiffu_amd import sage_attention as SA
+    q = torch.empty(0, 4, N, 128, dtype=torch.bfloat16, device=cuda)
+    with pytest.raises(ValueError, match="positive"):
+        SA.sage_forward(q, q, q)
