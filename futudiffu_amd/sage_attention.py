@@ -418,8 +418,10 @@ def sage_attn_forward_masked_merged_heads(q: Tensor, k: Tensor, v: Tensor, block
 
 def _rows_layout(t: Tensor) -> tuple[Tensor, int]:
     """A [B, H, N, D] tensor the backward can read in place, with its memory
-    layout: [B, H, N, D], or [B, N, H, D] (a transposed view); a copy else."""
-    if not t.is_contiguous() and t.transpose(1, 2).is_contiguous():
+    layout: [B, H, N, D], or [B, N, H, D] (a transposed view); a copy else.
+    The kernels read 16 bytes at a time, so a transposed view that starts
+    elsewhere is copied too."""
+    if not t.is_contiguous() and t.transpose(1, 2).is_contiguous() and t.data_ptr() % 16 == 0:
         return t, _LAYOUT["bnhd"]
     return t.contiguous(), _LAYOUT["bhnd"]
 

@@ -317,6 +317,21 @@ def test_backward_python_glue_checks():
         SA.sage_backward(q.float(), q, q, q, lse, q)
 
 
+def test_backward_copies_misaligned_transposed_views():
+    """out and dO as [B, N, H, D] views are read in place only from a 16-byte
+    boundary (what the library takes); any other start is copied, as every
+    such view was."""
+    from futudiffu_amd import sage_attention as SA
+    B, H, N, D = 2, 3, 5, 64
+    buf = torch.randn(B * N * H * D + 8).bfloat16()
+    assert buf.data_ptr() % 16 == 0
+    for off in range(9):
+        t = buf[off:off + B * N * H * D].view(B, N, H, D).transpose(1, 2)
+        rows, layout = SA._rows_layout(t)
+        assert rows.data_ptr() % 16 == 0 and torch.equal(rows, t)
+        assert (rows.data_ptr() == t.data_ptr()) == (off % 8 == 0) and layout == (1 if off % 8 == 0 else 0)
+
+
 @fake_addresses
 def test_fused_quantize_entry_checks_outputs():
     from futudiffu_amd import _lib
