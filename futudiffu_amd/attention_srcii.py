@@ -223,9 +223,10 @@ def _ext_backward(ctx, grad_out, grad_lse):
     sm_scale, qk, smooth_k, layout = ctx.args
     grad_out = _grad_of(grad_out, out)
     if layout == "bnhd":
-        out, grad_out = _to_bhnd(out, q.shape), _to_bhnd(grad_out, q.shape)
-    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out.contiguous(), block_mask, doc_ids, sm_scale, qk,
-                                 smooth_k)
+        out, grad_out = _to_bhnd(out, q.shape), _to_bhnd(grad_out, q.shape)  # read in place
+    else:
+        grad_out = grad_out.contiguous()
+    dq, dk, dv = sage_bwd_ext_op(q, k, v, out, lse, grad_out, block_mask, doc_ids, sm_scale, qk, smooth_k)
     return dq, dk, dv, None, None, None, None, None, None, None, None
 
 

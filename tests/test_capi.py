@@ -432,6 +432,34 @@ def test_legacy_op_schemas_and_fake_shapes():
             assert lse.shape == (6, 40) and lse.dtype == torch.float32
 
 
+def test_merged_layout_backward_passes_views(monkeypatch):
+    """Every formula of a forward in the out-projection's layout hands the
+    backward views of out and dO, no transposed copies."""
+    from futudiffu_amd import attention_srcii as A
+    B, H, N, D = 2, 3, 5, 64
+    q = torch.zeros(B, H, N, D)
+    out, grad = torch.randn(B, N, H * D), torch.randn(B, N, H * D)
+    seen = []
+
+    def record(q_, k_, v_, out_, lse_, grad_, *rest):
+        seen.append((out_, grad_))
+        return q_, k_, v_
+
+    class Ctx:
+        granularity, sm_scale, smooth_k = "token", 0.1, True
+        args = (0.1, "int8", True, "bnhd")
+
+    monkeypatch.setattr(A, "sage_bwd_ext_op", record)
+    for formula, saved in ((A._ext_backward, (q, q, q, out, None, None, None)),
+                           (A._merged_backward, (q, q, q, out, None, None))):
+        Ctx.saved_tensors = saved
+        formula(Ctx(), grad, None)
+    assert len(seen) == 2
+    for pair in seen:
+        for x, rows in zip(pair, (out, grad)):
+            assert x.data_ptr() == rows.data_ptr() and torch.equal(x, rows.view(B, N, H, D).transpose(1, 2))
+
+
 def test_ext_backward_refuses_block_scales():
     """The backward recomputes P from per-token codes, so a forward run with
     per-64-token scales has no consistent gradient: refused before any work."""

@@ -304,16 +304,23 @@ def test_backward_forms_of_the_quantization_agree(cuda, monkeypatch, B, H, N, D,
 
 
 def test_merged_heads_autograd_takes_a_misaligned_gradient(cuda):
-    """The merged-heads forward's gradient may start anywhere in its storage."""
+    """The gradient of a forward in the out-projection's layout may start
+    anywhere in its storage, and the two ops with that layout agree."""
     import futudiffu_amd  # noqa: F401
+    ops = torch.ops.futudiffu_ii
     B, H, N, D = 1, 2, 200, 64
     q, k, v, dout = _inputs(B, H, N, D, seed=23)
     bm = O.build_block_mask([120, 80], N).to(cuda)
     args = [t.to(cuda).requires_grad_(True) for t in (q, k, v)]
-    out, _ = torch.ops.futudiffu_ii.sage_attn_masked_merged_heads(*args, bm, 1.0 / math.sqrt(D))
+    sm = 1.0 / math.sqrt(D)
     merged = dout.to(cuda).transpose(1, 2).reshape(B, N, H * D)
     odd = torch.empty(merged.numel() + 1, dtype=torch.bfloat16, device=cuda)[1:].view_as(merged).copy_(merged)
     print("bwd misaligned merged gradient", flush=True)
-    want = torch.autograd.grad(out, args, merged, retain_graph=True)
-    for a, b in zip(torch.autograd.grad(out, args, odd), want):
-        assert torch.equal(a, b)
+    want = None
+    for out, _ in (ops.sage_attn_masked_merged_heads(*args, bm, sm),
+                   ops.sage_attn_ext(*args, bm, None, sm, "int8", "bf16", "token", True, "bnhd")):
+        for grad in (merged, odd):
+            got = torch.autograd.grad(out, args, grad, retain_graph=True)
+            want = got if want is None else want
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
