@@ -35,6 +35,11 @@ def _declared():
     return sorted(set(re.findall(r"^\s*(?:const\s+)?[\w]+\s*\*?\s+(sage_\w+)\s*\(", text, re.M)))
 
 
+def test_include_folder_holds_the_header_alone():
+    """No link back to the folder, which tools that follow links would walk for ever."""
+    assert os.listdir(os.path.dirname(HEADER)) == ["sage_mi355x.h"]
+
+
 def test_header_declarations_found():
     names = _declared()
     assert {"sage_quantize_qkv", "sage_attn_fwd", "sage_abi_version", "sage_last_error"} <= set(names)
