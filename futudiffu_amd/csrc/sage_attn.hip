@@ -1408,22 +1408,19 @@ __device__ __forceinline__ uint64_t active_64(const uint8_t* row, int nt, int t)
   const int i = t + (int)(threadIdx.x & 63);
   return __ballot(i < nt && row[min(i, nt - 1)] != 0);
 }
-// (first active tile, one past the last); (nt, 0) with none
-__device__ __forceinline__ int2 active_ends(const uint8_t* row, int nt) {
+// (first active tile, one past the last), (nt, 0) with none; their number in count
+__device__ __forceinline__ int2 active_ends(const uint8_t* row, int nt, int& count) {
   int2 e = make_int2(nt, 0);
+  count = 0;
   for (int t = 0; t < nt; t += 64) {
     const uint64_t m = active_64(row, nt, t);
     if (m != 0) {
       e.x = min(e.x, t + __builtin_ctzll(m));
       e.y = t + 64 - __builtin_clzll(m);
+      count += __builtin_popcountll(m);
     }
   }
   return e;
-}
-__device__ __forceinline__ int active_count(const uint8_t* row, int nt) {
-  int n = 0;
-  for (int t = 0; t < nt; t += 64) n += __builtin_popcountll(active_64(row, nt, t));
-  return n;
 }
 // the active tile with k active ones before it; nt if there is none
 __device__ __forceinline__ int nth_active(const uint8_t* row, int nt, int k) {
@@ -1439,6 +1436,32 @@ __device__ __forceinline__ int nth_active(const uint8_t* row, int nt, int k) {
   return nt;
 }
 
+// Position i of a list of n that XCDs (workgroup i runs on XCD i % 8) take in
+// contiguous ranges.
+__device__ __forceinline__ int64_t xcd_range(int64_t i, int64_t n) {
+  const int x = (int)(i % 8);
+  const int64_t local = i / 8, per = n / 8, rem = n % 8;
+  return x * per + (x < rem ? x : rem) + local;
+}
+
+// The end of a piece of split item si: its partial into `slot`, and where it
+// is the last of the item's `parts` to arrive, the merge.
+template <int D>
+__device__ __forceinline__ void leave_piece(const AttnParams& p, uint8_t* smem, int64_t slot, int64_t si, int parts,
+                                            const f32x16 (&o)[D / 32], float m_ref, float l_acc) {
+  store_partial_coherent<D>(p.part + slot * kPartFloats<D>, o, m_ref, l_acc);
+  wait_vmem();  // this piece's partial is at the coherence point before it counts
+  __syncthreads();
+  int* last = reinterpret_cast<int*>(smem);
+  if (threadIdx.x == 0) *last = arrive_last(p.merge_ctr + si, p.merge_tag, parts) ? 1 : 0;
+  __syncthreads();
+  if (*last == 0) return;
+  __syncthreads();  // every wave has read the decision before the factors reuse the LDS
+  merge_pieces<D>(p, si, parts, reinterpret_cast<float*>(smem));
+  if (threadIdx.x == 0)
+    __hip_atomic_store(p.merge_ctr + si, p.merge_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <int D, int QK, int PV, int GRAN, int MASK, bool DUMP = false>
 __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
   using SM = Smem<D, PV>;
@@ -1450,17 +1473,14 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
 
   int bh, qt;
   bool skip_listed = false;  // document ids: this workgroup leaves a listed split query tile to the first ones
-  if constexpr ((MASK & 2) == 0) {
-    // Without document ids: items in head-major order.  Workgroups [0,
-    // n_whole) take whole items, dealt to XCDs (workgroup i runs on XCD i % 8)
-    // in contiguous ranges so that an XCD's resident workgroups share K/V
-    // tiles in its L2.  Later workgroups, dispatched last, take the pieces of
-    // the split items and leave partials; the last piece of an item to arrive
-    // merges them (merge_pieces), or merge_split_kernel does after the launch
-    // (unmasked launches only).  A tile-masked item's pieces are equal shares
-    // of its active tiles, at least 4 of them beside a full round and at least
-    // 12 where every item is cut (tail_split): it uses only as many of its
-    // workgroups as that gives, the others exit.
+  // Without document ids: items in head-major order.  Workgroups [0, n_whole)
+  // take whole items, dealt to XCDs (workgroup i runs on XCD i % 8) in
+  // contiguous ranges so that an XCD's resident workgroups share K/V tiles in
+  // its L2.  Later workgroups, dispatched last, take the pieces of the split
+  // items and leave partials; the last piece of an item to arrive merges them
+  // (merge_pieces), or merge_split_kernel does after the launch (unmasked
+  // launches only).
+  if constexpr (MASK == 0) {
     const int64_t b = blockIdx.x;
     if (b >= p.n_whole) {
       const int64_t c = b - p.n_whole;
@@ -1469,58 +1489,93 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
       const int part = (int)(c % p.split_parts);
       bh = (int)(pos / nq);
       qt = (int)(pos % nq);
-      int t0, t1, parts = p.split_parts;
-      if constexpr (MASK == 1) {
-        const uint8_t* row = mask_row(p, bh, qt);
-        const int count = active_count(row, p.nt);
-        parts = max(1, min(parts, p.n_whole == 0 ? count / 12 : count / 4));
-        if (part >= parts) return;
-        t0 = nth_active(row, p.nt, (int)((int64_t)part * count / parts));
-        t1 = part + 1 < parts ? nth_active(row, p.nt, (int)((int64_t)(part + 1) * count / parts)) : p.nt;
-      } else {
-        t0 = (int)((int64_t)part * p.nt / p.split_parts);
-        t1 = (int)((int64_t)(part + 1) * p.nt / p.split_parts);
-      }
-      item_tiles<D, QK, PV, GRAN, MASK, DUMP>(p, smem, bh, qt, t0, t1, o, m_ref, l_acc);
-      if (MASK == 1 && parts == 1) {  // too few active tiles to share
-        store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
-        return;
-      }
-      if (MASK == 0 && p.merge_ctr == nullptr) {
+      const int t0 = (int)((int64_t)part * p.nt / p.split_parts);
+      const int t1 = (int)((int64_t)(part + 1) * p.nt / p.split_parts);
+      item_tiles<D, QK, PV, GRAN, 0, DUMP>(p, smem, bh, qt, t0, t1, o, m_ref, l_acc);
+      if (p.merge_ctr == nullptr) {
         store_partial<D>(p.part + c * kPartFloats<D>, o, m_ref, l_acc);
         return;
       }
-      store_partial_coherent<D>(p.part + c * kPartFloats<D>, o, m_ref, l_acc);
-      wait_vmem();  // this piece's partial is at the coherence point before it counts
-      __syncthreads();
-      int* last = reinterpret_cast<int*>(smem);
-      if (threadIdx.x == 0) *last = arrive_last(p.merge_ctr + si, p.merge_tag, parts) ? 1 : 0;
-      __syncthreads();
-      if (*last == 0) return;
-      __syncthreads();  // every wave has read the decision before the factors reuse the LDS
-      merge_pieces<D>(p, si, parts, reinterpret_cast<float*>(smem));
-      if (threadIdx.x == 0)
-        __hip_atomic_store(p.merge_ctr + si, p.merge_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      leave_piece<D>(p, smem, c, si, p.split_parts, o, m_ref, l_acc);
       return;
     }
-    if (MASK == 0 || p.split_parts > 1) {
-      const int x = (int)(b % 8);
-      const int64_t local = b / 8, per = p.n_whole / 8, rem = p.n_whole % 8;
-      const int64_t pos = x * per + (x < rem ? x : rem) + local;
+    const int64_t pos = xcd_range(b, p.n_whole);
+    bh = (int)(pos / nq);
+    qt = (int)(pos % nq);
+  } else if constexpr (MASK == 1) {
+    // A tile-masked item's pieces are equal shares of its active tiles, at
+    // least share_min of them, and none where it has fewer than share_from:
+    // it uses only as many of its workgroups as that gives, the others exit.
+    // The first pieces of all items come first, dealt to XCDs like a launch of
+    // their own: for the items that stay whole they are the launch's
+    // remaining items in their usual places, and the workgroups that exit come
+    // after (interleaved with the pieces of one item in a row, 1x30x1500x128
+    // in 2, 3 documents: 28.3, 25.3 us with bf16 P.V against 26.3, 20.0 uncut).
+    // The loop starts at the first active tile and ends after the last:
+    // walking the others one scalar load at a time took 10 us per short
+    // document of the packed 6912-token batch.
+    const int64_t b = blockIdx.x;
+    int64_t si = 0;
+    int part = 0, parts = 1, count;
+    int2 ends;
+    auto whole_item = [&]() __attribute__((always_inline)) {
+      if (p.split_parts > 1) {
+        const int64_t pos = xcd_range(b, p.n_whole);
+        bh = (int)(pos / nq);
+        qt = (int)(pos % nq);
+      } else {
+        item_of((int)b, (int)gridDim.x, p.bh, nq, p.light_last, bh, qt);
+      }
+      ends = active_ends(mask_row(p, bh, qt), p.nt, count);
+    };
+    auto share = [&]() __attribute__((always_inline)) -> bool {  // false: not used
+      const int64_t c = b - p.n_whole, n_cut = (int64_t)p.bh * nq - p.n_whole;
+      part = (int)(c / n_cut);
+      si = xcd_range(c - part * n_cut, n_cut);
+      const int64_t pos = p.n_whole + si;
       bh = (int)(pos / nq);
       qt = (int)(pos % nq);
-    } else {
-      item_of((int)b, (int)gridDim.x, p.bh, nq, p.light_last, bh, qt);
-    }
-    if constexpr (MASK == 1) {
-      // the loop starts at the first active tile and ends after the last:
-      // walking the others one scalar load at a time took 10 us per short
-      // document of the packed 6912-token batch
-      const int2 ends = active_ends(mask_row(p, bh, qt), p.nt);
+      const uint8_t* row = mask_row(p, bh, qt);
+      ends = active_ends(row, p.nt, count);
+      parts = count < p.share_from ? 1 : max(1, min(p.split_parts, count / p.share_min));
+      if (part >= parts) return false;
+      if (parts > 1) {
+        ends.x = nth_active(row, p.nt, (int)((int64_t)part * count / parts));
+        if (part + 1 < parts) ends.y = nth_active(row, p.nt, (int)((int64_t)(part + 1) * count / parts));
+      }
+      return true;
+    };
+    auto run = [&]() __attribute__((always_inline)) {
       item_tiles<D, QK, PV, GRAN, MASK, DUMP>(p, smem, bh, qt, ends.x, ends.y, o, m_ref, l_acc);
+    };
+    auto store = [&]() __attribute__((always_inline)) {
+      if (parts == 1)
+        store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
+      else
+        leave_piece<D>(p, smem, si * p.split_parts + part, si, parts, o, m_ref, l_acc);
+    };
+    if constexpr (PV == kPV_FP8) {
+      // a copy of the loop for each (sharing one, D = 64 runs 3 % slower:
+      // 2x30x5000 551 -> 567 us)
+      if (b >= p.n_whole) {
+        if (!share()) return;
+        run();
+        store();
+        return;
+      }
+      whole_item();
+      run();
       store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
-      return;
+    } else {
+      // one copy (with two, D = 64 spills 13 registers: 4x30x300 6.4 -> 6.7 us)
+      if (b < p.n_whole)
+        whole_item();
+      else if (!share())
+        return;
+      run();
+      store();
     }
+    return;
   } else {
     // the first heavy_max * h workgroups: head id % h of listed split query
     // tile id / h (doc_prefix_kernel); the others run the usual order and
@@ -1772,11 +1827,15 @@ AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool ma
   w.part_off = (w.heavy_off + (size_t)(1 + kHeavyMax) * sizeof(int4) + 255) & ~(size_t)255;
   int64_t split_items = items - w.split.whole;
   if (limit != 0 && split_items > 0) {
-    const int64_t item_bytes = w.split.parts * (128 * d + 512) * (int64_t)sizeof(float) + (int64_t)sizeof(uint64_t);
-    const int64_t room = (int64_t)limit - (int64_t)w.part_off;
-    split_items = room > 0 ? std::min(split_items, room / item_bytes) : 0;
-    w.split.whole = items - split_items;
-    if (split_items == 0) w.split.parts = 1;
+    // fewer pieces rather than some items whole: those would last as long as an
+    // uncut tail (1x30x3071x128 with 124 of 208 items cut: 148 us, 134 uncut)
+    const int64_t slots = ((int64_t)limit - (int64_t)w.part_off - split_items * (int64_t)sizeof(uint64_t)) /
+                          ((128 * d + 512) * (int64_t)sizeof(float));
+    w.split.parts = (int)std::min<int64_t>(w.split.parts, slots / split_items);
+    if (w.split.parts < 2) {
+      w.split = TailSplit{items, 1};
+      split_items = 0;
+    }
   }
   const int64_t pieces = split_items * w.split.parts;
   // then one 8-byte arrival counter per split item (in-kernel merge)

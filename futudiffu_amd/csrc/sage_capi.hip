@@ -345,16 +345,19 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   // or the scratch of the allocation-free entry point), items are
   // split as in an unmasked launch: the production op is always masked, and at
   // 1x30x4416 its 1050 items leave a third round of 26.  The pieces' slots stay
-  // within that scratch, so every entry point cuts the same items.
+  // within that scratch, so every entry point that has the room cuts the same
+  // items.
   sage::AttnWorkspace ws = sage::attn_workspace(b, h, n, d, mask != 0);
   // a launch whose every item is cut runs whole in a workspace of the summaries
   // alone, the size it needs without the cut
   if (mask == 0 && ws.split.whole == 0 && workspace_bytes < ws.bytes) ws = sage::attn_workspace(b, h, n, d, true);
-  bool masked_split = false;
+  sage::MaskedSplit shares{sage::TailSplit{b * h * nq, 1}, 0, 1};
   if (mask == 1 && merge_in_kernel()) {
     const sage::AttnWorkspace split = sage::attn_workspace(b, h, n, d, false, SAGE_NOALLOC_SCRATCH_BYTES);
-    masked_split = workspace_bytes >= split.bytes;
-    if (masked_split) ws = split;
+    if (workspace_bytes >= split.bytes) {
+      ws = split;
+      shares = sage::masked_split(split.split, b * h * nq, nkv, d);
+    }
   }
   if (!workspace || workspace_bytes < ws.bytes)
     return fail(SAGE_ERR_WORKSPACE, "workspace of %zu bytes needed, got %zu", ws.bytes, workspace_bytes);
@@ -397,13 +400,14 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   p.nt = (int)nkv;
   p.light_last = (nq > 1 && n - (nq - 1) * 128 <= 64) ? 1 : 0;
   // cut the items of the last, partial dispatch round
-  p.n_whole = (int)(b * h * nq);
-  p.split_parts = 1;
-  if (mask == 0 || masked_split) {
-    p.n_whole = (int)ws.split.whole;
-    p.split_parts = ws.split.parts;
+  const sage::TailSplit split = mask == 0 ? ws.split : shares.split;
+  p.n_whole = (int)split.whole;
+  p.split_parts = split.parts;
+  p.share_from = shares.share_from;
+  p.share_min = shares.share_min;
+  if (split.parts > 1) {
     p.part = reinterpret_cast<float*>(wsp + ws.part_off);
-    if (ws.split.parts > 1 && merge_in_kernel()) {
+    if (merge_in_kernel()) {
       p.merge_ctr = reinterpret_cast<uint64_t*>(wsp + ws.ctr_off);
       p.merge_tag = next_merge_tag();
     }

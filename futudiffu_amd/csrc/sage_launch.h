@@ -56,6 +56,10 @@ struct AttnParams {
   // parity only (int8 QK, unmasked): int32 [BH, Np, Np] receives the S^T
   // accumulators of every tile the kernel's own loop consumes (row = query)
   int32_t* s_dump;
+  // tile mask alone: a split item is cut into at most (active tiles) /
+  // share_min pieces, and not at all below share_from active tiles
+  int share_from;
+  int share_min;
 };
 
 // Split query tiles (document ids) that the first workgroups of a launch take
@@ -150,6 +154,41 @@ inline TailSplit tail_split(int64_t n_items, int64_t nt, int64_t d) {
   return t;
 }
 
+// The split of a tile-masked launch without document ids: tail_split's items
+// (reduced to `split` by attn_workspace's limit), each cut into equal shares of
+// its active tiles by the kernel, which alone knows the mask.
+//
+// A share takes at least 4 tiles beside full rounds and at least 12 where every
+// item is cut (the figures of tail_split); a launch whose items cannot have two
+// such shares is not split (4x30x300x128, 5 tiles: 13.2 us whole, 14.8 with
+// workgroups that only exit).  Items of several documents are short and of
+// different lengths, so they leave no long tail of their own.  So with more
+// than short_tail items past the last full round, and below one round, only
+// items of three quarters of the tiles or more are cut; D = 64 runs three
+// workgroups a CU with bf16 P.V, whose rounds are longer, so its line is lower
+// and above 128 items none is cut.  Attention kernel, bf16 P.V, in 1, 2, 3
+// documents, us, without split / every item cut / long items cut:
+//   1x30x2560x128 (88 past)  105 57 42 / 95 55 43 / 95 59 44
+//   1x19x4200x128 (115)     170 89 62 / 150 84 61 / 151 91 65
+//   1x30x1500x128 (104 past one per CU)  42 25 19 / 39 27 23 / 40 25 20
+//   1x17x4200x64 (49)       110 58 41 / 90 48 34 / 91 60 43
+//   1x30x2560x64 (88)        69 37 28 / 63 42 34 / 64 39 30
+//   2x30x1337x64 (148)       40 23 18 / 44 30 19 / 44 24 19
+struct MaskedSplit {
+  TailSplit split;
+  int share_from, share_min;
+};
+
+inline MaskedSplit masked_split(TailSplit split, int64_t n_items, int64_t nt, int64_t d) {
+  const int64_t share_min = split.whole == 0 ? 12 : 4, tail = n_items - split.whole;
+  const int64_t short_tail = d == 64 ? 64 : 96;
+  const bool any = split.whole == 0 || (split.whole >= kResidentWGs && tail <= short_tail);
+  MaskedSplit m{split, any ? 0 : (int)((3 * nt + 3) / 4), (int)share_min};
+  if (m.split.parts > nt / share_min) m.split.parts = (int)(nt / share_min);
+  if (m.split.parts < 2 || (split.whole != 0 && tail > 128)) m.split = TailSplit{n_items, 1};
+  return m;
+}
+
 // Inputs of the q/k/v producer (QKV split + per-head RMSNorm + Flux RoPE +
 // transpose, fused_kernels.py:271-390).  With qkv set, the quantization reads
 // the projection output and applies the producer itself; with qkv null it
@@ -219,9 +258,9 @@ struct AttnWorkspace {
   size_t doc_off, heavy_off, part_off, ctr_off, bytes;
   TailSplit split;
 };
-// `masked`: a launch with a tile mask or document ids, which splits no item
-// and so needs no partial slots.  `limit` (0: none): split only as many of the
-// tail items as keep `bytes` within it, the others stay whole.
+// `masked`: a launch that splits no item (document ids, or a tile mask in a
+// workspace without room for partials).  `limit` (0: none): the tail items in
+// as many pieces as keep `bytes` within it; whole if that is under two.
 AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false, size_t limit = 0);
 size_t attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false);
 hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t pad_fill, uint8_t* mask,

@@ -272,3 +272,30 @@ def test_bf16_document_ids_on_the_pipelined_loop(cuda, lens, D):
     assert (out.cpu().float() - want.float()).abs().max().item() <= 2e-2
     assert O.cosine(out.cpu(), want) >= 0.999
     assert (lse.cpu() - wl.view_as(lse.cpu())).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("B,H,D,lens", [(1, 30, 128, [1003, 771, 1297]), (1, 30, 128, [500, 400, 600]),
+                                        (2, 30, 64, [1337]), (4, 30, 128, [300])])
+def test_tile_masked_launches_left_whole(cuda, B, H, D, lens):
+    """Launches whose items are not cut, with room for partials: 208 items past a
+    round (their partials exceed the scratch in two pieces), short documents
+    below one round, 148 items past a round at D = 64, items of 5 tiles.  The
+    bits of the launch that has no room."""
+    from futudiffu_amd import _lib
+    from futudiffu_amd import sage_attention as SA
+    N = sum(lens)
+    lib = _lib.load()
+    q, k, v = (t.to(cuda) for t in O.make_inputs(B, H, N, D, seed=N))
+    mg = O.build_block_mask(lens, N).to(cuda)
+    print(f"masked launch left whole {B}x{H}x{N}x{D}", flush=True)
+    qz = SA.quantize_qkv(q, k, v, qk="int8", pv="bf16")
+    out, lse = SA.attn_from_quantized(qz, B, H, block_mask=mg)
+    wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+    o1, l1 = torch.empty_like(out), torch.empty_like(lse)
+    _lib.check(lib.sage_attn_fwd(
+        qz.q_codes.data_ptr(), qz.q_scale.data_ptr(), qz.k_codes.data_ptr(), qz.k_scale.data_ptr(),
+        qz.v_op.data_ptr(), None, B, H, N, D, 0, 0, 0, mg.data_ptr(), 0, mg.shape[0], mg.shape[1], None,
+        ws.data_ptr(), wsb, o1.data_ptr(), 0, l1.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out, o1) and torch.equal(lse, l1)
