@@ -1436,6 +1436,14 @@ __device__ __forceinline__ int nth_active(const uint8_t* row, int nt, int k) {
   return nt;
 }
 
+// Workgroups of the attention kernel per CU.  bf16 P.V without document ids
+// at D = 64 fits three (39 KB of LDS, 168 registers; two spill across the tile
+// loop, not in it): left to itself it takes 170 and the third is lost, which at
+// 4x30x1300 costs 78.9 -> 70.7 us (fp8 QK) and 83.3 -> 75.4 us (int8), tile-masked
+// at 1x30x6912 394.1 -> 352.7 and 420.3 -> 385.2 us.
+template <int D, int PV, int MASK>
+constexpr int kAttnWGs = D == 64 && PV == kPV_BF16 && (MASK & 2) == 0 ? 3 : 2;
+
 // Position i of a list of n that XCDs (workgroup i runs on XCD i % 8) take in
 // contiguous ranges.
 __device__ __forceinline__ int64_t xcd_range(int64_t i, int64_t n) {
@@ -1463,7 +1471,7 @@ __device__ __forceinline__ void leave_piece(const AttnParams& p, uint8_t* smem, 
 }
 
 template <int D, int QK, int PV, int GRAN, int MASK, bool DUMP = false>
-__global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnParams p) {
+__global__ void __launch_bounds__(256, (kAttnWGs<D, PV, MASK>)) attn_fwd_kernel(AttnParams p) {
   using SM = Smem<D, PV>;
   constexpr int NC = D / 32;
   __shared__ __attribute__((aligned(16))) uint8_t smem[SM::bytes];

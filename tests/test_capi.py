@@ -501,3 +501,31 @@ def test_noalloc_entry_rejects_shapes_beyond_its_scratch():
     args[9], args[6] = 128, 0
     assert lib.sage_attn_fwd_noalloc(*args) == 1
     assert "positive" in lib.sage_last_error().decode()
+
+
+def test_attention_kernels_keep_their_workgroups_per_cu(tmp_path):
+    """Registers and LDS of the built attention kernels: bf16 P.V at D = 64
+    without document ids runs three workgroups of four waves a CU (512 / 3
+    registers in units of 8, 160 KB of LDS), every other instance two."""
+    from futudiffu_amd import _lib, build
+    tools = os.path.join(os.path.dirname(os.path.dirname(build.hipcc())), "llvm", "bin")
+    objdump, readelf = (os.path.join(tools, t) for t in ("llvm-objdump", "llvm-readelf"))
+    if not (os.path.exists(objdump) and os.path.exists(readelf)):
+        pytest.skip("no ROCm binutils")
+    lib = tmp_path / "lib.so"
+    lib.write_bytes(open(_lib.load()._name, "rb").read())
+    subprocess.run([objdump, "--offloading", str(lib)], cwd=tmp_path, check=True, capture_output=True)
+    seen = 0
+    for obj in tmp_path.glob("lib.so.*gfx950*"):
+        notes = subprocess.run([readelf, "--notes", str(obj)], check=True, capture_output=True, text=True).stdout
+        for k in notes.split("- .agpr_count:")[1:]:
+            field = lambda n: int(re.search(rf"\.{n}:\s+(\d+)", k).group(1))  # noqa: E731
+            m = re.search(r"\.name:\s+_ZN4sage15attn_fwd_kernelILi(\d+)ELi\dELi(\d)ELi\dELi(\d)ELb0", k)
+            if m is None:
+                continue
+            d, pv, mask = (int(x) for x in m.groups())
+            wgs = 3 if d == 64 and pv == 0 and mask < 2 else 2
+            assert field("vgpr_count") <= 512 // wgs // 8 * 8, m.group(0)
+            assert field("group_segment_fixed_size") * wgs <= 160 << 10, m.group(0)
+            seen += 1
+    assert seen == 64
