@@ -151,12 +151,8 @@ BwdWorkspace bwd_workspace(int64_t b, int64_t bh, int64_t n, int64_t d) {
   w.ks = take(rows * 4);
   w.kmean = take((size_t)bh * d * 2);
   w.quant = take(sage::quant_workspace_bytes(bh, n, d));
-  // Five regions of one bf16 image each: the size is part of the interface
-  // (callers keep workspaces of it), the last three are spare since the passes
-  // read dO, Q and V as they are.
   w.kt = take(rows * d * 2);
-  w.lse_pad = take(rows * d * 2);
-  for (int i = 0; i < 3; ++i) take(rows * d * 2);
+  w.lse_pad = take(rows * 4);
   w.neg_delta = take(rows * 4);
   // document-id summaries (used with doc_ids): key tiles, 32- and 128-row blocks
   w.sums = take((size_t)b * ((n + 63) / 64 + np / 32 + np / 128) * sizeof(int4));
