@@ -115,6 +115,33 @@ def test_graph_capture_sage_attn_split_tail(cuda):
         SA.configure_sage(smooth_k=saved[0], qk_quant=saved[1], pv_quant=saved[2])
 
 
+@pytest.mark.parametrize("B,H,N,masked", [(1, 2, 3000, False), (1, 2, 1921, True), (1, 65, 1000, True)])
+def test_graph_capture_cut_items(cuda, B, H, N, masked):
+    """Replays of launches whose items are cut and merged by arrival counters
+    that only the launch itself resets: every item of a launch of few items,
+    unmasked and tile-masked, and the 8 tile-masked items past a full round.
+    The mask changes between replays, and with it the shares in use."""
+    from futudiffu_amd import _lib
+    from futudiffu_amd import sage_attention as SA
+    D = 128
+    sc = 1.0 / math.sqrt(D)
+    lib = _lib.load()
+    assert lib.sage_attn_workspace_bytes(B, H, N, D) > lib.sage_attn_masked_workspace_bytes(B, H, N, D)
+    print(f"graph capture: cut items {B}x{H}x{N}x{D} masked={masked}", flush=True)
+    segments = [[N], [N // 2, N - N // 2], [N], [100, N - 100]]
+
+    def make(i):
+        q, k, v = _inputs(cuda, B, H, N, D, seed=260 + i)
+        return (q, k, v, O.build_block_mask(segments[i], N).to(cuda)) if masked else (q, k, v)
+
+    def fn(q, k, v, m=None):
+        if m is not None:
+            return torch.ops.futudiffu_ii.sage_attn_masked(q, k, v, m, sc)
+        return SA.sage_forward(q, k, v, sc, qk="int8", pv="fp8", smooth_k=True)
+
+    _capture_and_replay(cuda, fn, make, "cut items")
+
+
 def test_graph_capture_sage_attn_ext_doc_ids(cuda):
     """futudiffu_ii::sage_attn_ext with exact document ids (key padding
     included): the summary and prefix kernels, the listed split query tiles
