@@ -32,7 +32,8 @@
 // O and l are kept in a lazily moved frame: they hold sums of 2^(s - m_ref),
 // where the per-row reference point m_ref only moves when a block max exceeds
 // it by more than kTau (then O and l are rescaled, which is rare after the
-// first tiles; the pipelined bf16 loop finds such a block by its sum of P).  The LSE is m_ref + log2(l), the reference's m + log2(l).
+// first tiles; the pipelined bf16 loop finds such a block by its sum of P).  The
+// LSE is m_ref + log2(l), the reference's m + log2(l).
 // fp8 P follows the reference per (row, 64-key block) scaling
 // (sage_kernels.py:1137-1141): with bm the block's row max, the code argument
 // is e = 2^(s - bm) * 448 (= p * 448 / max(p)), and the block's PV product is
@@ -1015,16 +1016,15 @@ __device__ __forceinline__ bool item_tiles(const AttnParams& p, uint8_t* smem, i
   };
   // ---- every scheduled tile is computed by every live wave, so the product
   // of tile i-1 is always pending in iteration i.  The first and the last
-  // tile are peeled off the loop, which leaves its body one straight basic
-  // block for the scheduler: the pending P.V in two chunk-pair halves, each
-  // under half of this tile's score conversion, then the next tile's S^T
-  // under this tile's softmax.  fp8: the pending product's MFMAs and their
-  // dequantization into O; bf16: its MFMAs accumulate into O, after the
-  // frame move the previous softmax decided (deferred to here, so the
-  // softmax never waits for the product in flight).  With document ids
-  // (fp8) the tiles before prefix_end, which some live wave does not see
-  // whole, go through the general body first; every later scheduled tile
-  // is seen whole by every live wave.
+  // tile are peeled off the loop, which leaves its body without a tile test.
+  // fp8: one straight basic block for the scheduler, the pending P.V in NP
+  // chunk pairs, its MFMAs and their dequantization into O under this tile's
+  // score conversion, then the next tile's S^T under this tile's softmax.
+  // bf16: the ten groups of tile_bf16, after the frame move the previous
+  // softmax decided (deferred to here, so the softmax never waits for the
+  // product in flight).  With document ids the tiles before prefix_end, which
+  // some live wave does not see whole, go through the general body first;
+  // every later scheduled tile is seen whole by every live wave.
   constexpr int NP = NC / 2;
   int stage = 0;
   if constexpr (DOC) {
@@ -1717,7 +1717,7 @@ hipError_t launch_attn_d(int qk, int pv, int gran, int mask, const AttnParams& p
 // past the last of them bound the item's tile loop (no scan of the unseen
 // tiles before and after), and one past the last that some live 32-row wave
 // of the tile does not see whole (classify != 1) ends its prefix: the
-// pipelined fp8 loop of the attention kernel takes the tiles from there on,
+// pipelined loop of the attention kernel takes the tiles from there on,
 // the tiles before go through the general tile body with its per-element
 // visibility test.
 // A query tile whose live waves see different key-tile ranges (a document

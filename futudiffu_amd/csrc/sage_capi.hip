@@ -573,7 +573,8 @@ int sage_attn_bwd_layout(const void* q, const void* k, const void* v, const void
     mask |= 1;
   }
   if (doc_ids) mask |= 2;
-  // the dK/dV and dQ launches: 512-thread workgroups, one per 128-row tile
+  // one launch of a dK/dV and a dQ workgroup (256 threads) per 128-row tile; the
+  // quantization's limit below leaves room for the rounding and the cut items
   if ((b * h) * ((n + 127) / 128) > kMaxGridUnits / 2)
     return fail(SAGE_ERR_ARG, "b*h*ceil(n/128) = %lld exceeds the grid limit", (long long)(b * h * ((n + 127) / 128)));
   if (sage::quant_grid_units(b * h, n, d, 0) > kMaxGridUnits)
@@ -646,9 +647,9 @@ int sage_attn_bwd_layout(const void* q, const void* k, const void* v, const void
   p.np = np;
   p.h = (int)h;
   p.sm_scale = sm_scale;
-  // the last dQ items (up to kBwdDqSplit, a multiple of 8) in two key halves
-  // (measured at 1x30x4416x128: 1150.6 -> 1124.5 us with 128; 64 and 256
-  // within the run-to-run spread of 128)
+  // the last dQ items (up to kBwdDqSplit, a multiple of 8) in two key halves:
+  // the backward at 1x30x4416x128 919 -> 880 us, 1x30x1280 115.7 -> 110.0,
+  // 2x4x333x64 18.0 either way; 1x30x3071, whose last round is fuller, 442 -> 449
   const int64_t items = bh * (np / 128);
   p.dq_split = nkv >= 2 && bwd_split_enabled() ? (int)std::min<int64_t>(sage::kBwdDqSplit, items / 8 * 8) : 0;
   p.dq_part = reinterpret_cast<float*>(w + ws.dq_part);

@@ -66,7 +66,8 @@ struct AttnParams {
 // (AttnParams::heavy): kHeavyMax * h workgroups are reserved for them.
 constexpr int kHeavyMax = 2;
 
-// Resident workgroups of the attention kernel on MI355X: 256 CUs x 2.
+// Resident workgroups of the attention kernel on MI355X: 256 CUs x 2 (three a CU
+// with bf16 P.V at D = 64, which the splits below do not count on).
 constexpr int kResidentWGs = 512;
 
 // Floats of one partial slot: O of 128 rows x D (fp32, lane order), then the
@@ -91,10 +92,11 @@ constexpr int64_t kPartFloats = 128 * D + 2 * 256;
 // fits the one round of resident workgroups, else as many as fit, at least 2.
 // Measured at 20 tiles with a separate merge kernel: 2 pieces, 260 items
 // 43.5 -> 34.8 us, 300 items 41.6 -> 36.9, 350 items 41.5 -> 39.1; 400 items
-// lose, 42.1 -> 55.7; cutting every item costs more than it balances (300
-// items: 54.3 / 57.7 / 59.6 us in 2 / 3 / 4 pieces).  With the merge inside
-// the attention kernel, 300 items: 34.4 us in 2 pieces, 31.7 / 31.6 in 3 / 4,
-// 33.1 in 5.
+// lose, 42.1 -> 55.7.  With the merge inside the attention kernel, 300 items:
+// 34.4 us in 2 pieces, 31.7 / 31.6 in 3 / 4, 33.1 in 5; cutting every item
+// costs more than it balances (in 2 / 3 / 4 pieces, by this rule last: 300 items
+// of 20 tiles 51.2 / 51.0 / 62.0 against 30.8 us, 288 of 64 tiles 99.3 / 90.5 /
+// 98.6 against 75.5, 390 of 26 tiles, all whole, 64.8 / 72.5 / 89.4 against 47.6).
 //
 // Launches of no more items than CUs: each item walks all its tiles alone (1.05
 // us a tile) while CUs idle, so every item is cut, from 24 tiles on.  At most

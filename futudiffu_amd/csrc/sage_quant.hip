@@ -161,26 +161,16 @@ __device__ __forceinline__ void row_amax(const float (&x)[PASSES][8], float (&am
 // head; read per head they made up most of the L2 traffic of the
 // producer-fused quantization.
 
-// Sum over the LPR consecutive lanes (8 or 16) that hold one token's channels:
-// a pairwise tree over the lanes in order, with DPP moves of the two halves of
-// the fp64 value (quad xor 1, quad xor 2, half-row mirror, row mirror, as in
-// group_max).  At each step both lanes of a pair add the same two operands, so
-// every lane of the token ends with the same value.
+// DPP move of the two halves of an fp64 value, for the sums over the LPR
+// consecutive lanes (8 or 16) that hold one token's channels: a pairwise tree
+// over the lanes in order, at each step of which both lanes of a pair add the
+// same two operands.
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, false);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, false);
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
-template <int LPR>
-__device__ __forceinline__ double token_sum(double v) {
-  v += dpp_f64<0xB1>(v);   // [1,0,3,2]
-  v += dpp_f64<0x4E>(v);   // [2,3,0,1]
-  v += dpp_f64<0x141>(v);  // half-row mirror: quad q with quad q^1
-  if constexpr (LPR == 16) v += dpp_f64<0x140>(v);  // row mirror: half-row with half-row
-  return v;
 }
 
 // Two fp32 -> two bf16 (round to nearest even, v_cvt_pk_bf16_f32) in one word.

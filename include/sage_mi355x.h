@@ -185,9 +185,11 @@ size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 /* Bytes of device workspace a sage_attn_fwd launch with a tile_mask or
  * doc_ids needs: the summaries only (a few KB; 7 KB for the packed 1x30x6912
  * batch).  A tile-masked launch without doc_ids that is given room for them
- * (sage_attn_workspace_bytes) splits its items like an unmasked one: as
- * many of them as keep the partials within SAGE_NOALLOC_SCRATCH_BYTES, so
- * sage_attn_fwd_noalloc cuts the same ones.  No reference counterpart. */
+ * (sage_attn_workspace_bytes) cuts its last items into shares of their active
+ * tiles where that is faster, in as many as keep all partials within
+ * SAGE_NOALLOC_SCRATCH_BYTES (sage_attn_fwd_noalloc cuts the same ones), or
+ * none.  P is rounded in another frame in a cut item, so its rows can differ in
+ * the last bits between the two workspace sizes.  No reference counterpart. */
 size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
 /* Fused attention forward over pre-quantized operands.
@@ -211,9 +213,9 @@ size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t
  *                 32-bit byte offsets).
  *   h             heads per batch (row z of q belongs to batch z / h).
  *   workspace     device memory of sage_attn_workspace_bytes(b, h, n, d)
- *                 bytes (sage_attn_masked_workspace_bytes when tile_mask or
- *                 doc_ids is given), 16-byte aligned.  Concurrent calls need
- *                 separate workspaces.
+ *                 bytes (at least sage_attn_masked_workspace_bytes when
+ *                 tile_mask or doc_ids is given), 16-byte aligned.  Concurrent
+ *                 calls need separate workspaces.
  *   out_layout    SAGE_OUT_BHND (the reference op's output) or SAGE_OUT_BNHD
  *                 (fuses JointAttention's out.transpose(1, 2).reshape(b, -1,
  *                 H*D), transformer.py:471).  Values are bit-identical
@@ -251,7 +253,8 @@ int sage_attn_fwd(const void* q_codes, const float* q_scale,
  * threads) race; calls ordered on one stream do not.  The stream must belong
  * to the current device.  The first call on a device looks the array's
  * address up (hipGetSymbolAddress).  Other arguments, results and errors as
- * sage_attn_fwd, bit-identical to it. */
+ * sage_attn_fwd, bit-identical to it with a workspace of
+ * sage_attn_workspace_bytes (with document ids, of either size). */
 int sage_attn_fwd_noalloc(const void* q_codes, const float* q_scale,
                           const void* k_codes, const float* k_scale,
                           const void* v_in, const float* v_scale,
