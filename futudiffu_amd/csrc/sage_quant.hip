@@ -1746,6 +1746,7 @@ int64_t quant_grid_units(int64_t bh, int64_t n, int64_t d, int64_t h) {
 // flags of the one-kernel form, uint64 [bh][nch], then (its producer form)
 // the heads' mean flags, uint64 [bh], and means, fp32 [bh][d].
 size_t quant_workspace_bytes(int64_t bh, int64_t n, int64_t d) {
+  if (n <= 0 || d <= 0 || d > 256) return 0;  // refused by every launch; the chunk counts divide by both
   const int64_t nch = k_sum_chunks(n, d);
   return (size_t)(bh * nch * d) * sizeof(double) + (size_t)(bh * nch + bh) * sizeof(uint64_t) +
          (size_t)(bh * d) * sizeof(float);

@@ -126,6 +126,9 @@ for n in (1, 1024, 1473, 4416):
     for d in (-4, 0, 96, 512):
         assert lib.sage_forward_workspace_bytes(1, 2, n, d, 1, 0) == 0
 assert lib.sage_forward_workspace_bytes(1, 2, 0, 128, 1, 0) == 0
+for bh, n, d in ((30, 0, 128), (0, 0, 64), (30, -1, 64), (30, 100, 0), (30, 100, 512)):
+    assert lib.sage_quant_workspace_bytes(bh, n, d) == 0
+lib.sage_attn_bwd_workspace_bytes(1, 30, 0, 128)
 assert lib.sage_attn_workspace_bytes(0, 30, 4416, 128) == lib.sage_attn_workspace_bytes(0, 30, 64, 128) == 256
 '''
 
