@@ -207,13 +207,20 @@ def qkv_postprocess_backward(qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: 
     """Gradient of ``qkv_postprocess`` with respect to ``qkv`` (bf16
     ``[B, N, 3*H*D]``), given the gradients of its outputs ``[B, H, N, D]``:
     the reference's analytical backward (fused_kernels.py:711-783) on the GPU."""
+    return _postprocess_backward_into(torch.empty_like(qkv), qkv, q_norm_weight, k_norm_weight, freqs_cis, grad_q,
+                                      grad_k, grad_v, n_heads, head_dim, norm_eps)
+
+
+def _postprocess_backward_into(dqkv: Tensor, qkv: Tensor, q_norm_weight: Tensor, k_norm_weight: Tensor,
+                               freqs_cis: Tensor, grad_q: Tensor, grad_k: Tensor, grad_v: Tensor, n_heads: int,
+                               head_dim: int, norm_eps: float) -> Tensor:
+    """``qkv_postprocess_backward`` into ``dqkv``, a tensor like ``qkv``."""
     shape = (qkv.shape[0], n_heads, qkv.shape[1], head_dim)
     for name, g in (("grad_q", grad_q), ("grad_k", grad_k), ("grad_v", grad_v)):
         if tuple(g.shape) != shape:
             raise ValueError(f"{name} must be {list(shape)}, got {tuple(g.shape)}")
     B, N, qw, kw, fr = _check_producer(qkv, q_norm_weight, k_norm_weight, freqs_cis, n_heads, head_dim)
     gs = [g.to(device=qkv.device, dtype=torch.bfloat16).contiguous() for g in (grad_q, grad_k, grad_v)]
-    dqkv = torch.empty_like(qkv)
     lib = _lib.load()
     _lib.check(lib.sage_qkv_postprocess_bwd(
         qkv.data_ptr(), qw.data_ptr(), kw.data_ptr(), fr.data_ptr(), gs[0].data_ptr(), gs[1].data_ptr(),
