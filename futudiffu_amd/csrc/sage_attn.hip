@@ -1835,12 +1835,21 @@ AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool ma
   w.part_off = (w.heavy_off + (size_t)(1 + kHeavyMax) * sizeof(int4) + 255) & ~(size_t)255;
   int64_t split_items = items - w.split.whole;
   if (limit != 0 && split_items > 0) {
-    // fewer pieces rather than some items whole: those would last as long as an
-    // uncut tail (1x30x3071x128 with 124 of 208 items cut: 148 us, 134 uncut)
     const int64_t slots = ((int64_t)limit - (int64_t)w.part_off - split_items * (int64_t)sizeof(uint64_t)) /
                           ((128 * d + 512) * (int64_t)sizeof(float));
-    w.split.parts = (int)std::min<int64_t>(w.split.parts, slots / split_items);
-    if (w.split.parts < 2) {
+    if (split_items <= kResidentWGs / 2) {
+      // fewer pieces: items left whole last as long as an uncut tail
+      // (1x30x3071x128, one document, 124 of 208 items cut: 141 us, all 136)
+      w.split.parts = (int)std::min<int64_t>(w.split.parts, slots / split_items);
+    } else {
+      // more items than CUs, so that some share one anyway: as many items as
+      // give a piece to every CU (2x12x4100x128, one document, 280 items: 203 us
+      // uncut, 199 in two pieces each, 196 in three, 179 with 85 of them in three)
+      const int64_t pieces = std::min<int64_t>(slots, kResidentWGs / 2);
+      split_items = std::min(split_items, std::max<int64_t>(pieces, 0) / w.split.parts);
+      w.split.whole = items - split_items;
+    }
+    if (w.split.parts < 2 || split_items == 0) {
       w.split = TailSplit{items, 1};
       split_items = 0;
     }

@@ -341,18 +341,18 @@ int attn_fwd_impl(const void* q_codes, const float* q_scale, const void* k_codes
   // or the scratch of the allocation-free entry point), items are
   // split as in an unmasked launch: the production op is always masked, and at
   // 1x30x4416 its 1050 items leave a third round of 26.  The pieces' slots stay
-  // within that scratch, so every entry point that has the room cuts the same
-  // items.
+  // within kMaskedSplitBytes, so every entry point that has the room cuts the
+  // same items.
   sage::AttnWorkspace ws = sage::attn_workspace(b, h, n, d, mask != 0);
   // a launch whose every item is cut runs whole in a workspace of the summaries
   // alone, the size it needs without the cut
   if (mask == 0 && ws.split.whole == 0 && workspace_bytes < ws.bytes) ws = sage::attn_workspace(b, h, n, d, true);
   sage::MaskedSplit shares{sage::TailSplit{b * h * nq, 1}, 0, 1};
   if (mask == 1 && merge_in_kernel()) {
-    const sage::AttnWorkspace split = sage::attn_workspace(b, h, n, d, false, SAGE_NOALLOC_SCRATCH_BYTES);
+    const sage::AttnWorkspace split = sage::attn_workspace(b, h, n, d, false, sage::kMaskedSplitBytes);
     if (workspace_bytes >= split.bytes) {
       ws = split;
-      shares = sage::masked_split(split.split, b * h * nq, nkv, d);
+      shares = sage::masked_split(split.split, b * h * nq, nkv);
     }
   }
   if (!workspace || workspace_bytes < ws.bytes)
@@ -434,11 +434,13 @@ int sage_attn_fwd(const void* q_codes, const float* q_scale, const void* k_codes
 namespace {
 
 // Device scratch of sage_attn_fwd_noalloc: the document-id summaries and the
-// split-tail partials that sage_attn_fwd keeps in its workspace argument.
+// split-tail partials that sage_attn_fwd keeps in its workspace argument.  An
+// unmasked call may need SAGE_NOALLOC_SCRATCH_BYTES of it; the rest is for the
+// pieces of tile-masked items.
 // Each GPU the library runs on holds its own copy until the process ends.
 // Host code never uses the array's name as an address: its device address
 // comes from hipGetSymbolAddress, once per device, with that device current.
-__device__ __align__(256) uint8_t scratch[SAGE_NOALLOC_SCRATCH_BYTES];
+__device__ __align__(256) uint8_t scratch[sage::kMaskedSplitBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -487,7 +489,7 @@ int sage_attn_fwd_noalloc(const void* q_codes, const float* q_scale, const void*
   st = scratch_of_stream(stream, &ws);
   if (st) return st;
   return attn_fwd_impl(q_codes, q_scale, k_codes, k_scale, v_in, v_scale, b, h, n, d, qk_kind, pv_kind, granularity,
-                       tile_mask, mask_stride_z, mask_nq, mask_nkv, doc_ids, ws, SAGE_NOALLOC_SCRATCH_BYTES, out,
+                       tile_mask, mask_stride_z, mask_nq, mask_nkv, doc_ids, ws, sage::kMaskedSplitBytes, out,
                        out_layout, lse, nullptr, "sage_attn_fwd_noalloc", stream);
 }
 

@@ -160,34 +160,33 @@ inline TailSplit tail_split(int64_t n_items, int64_t nt, int64_t d) {
 // (reduced to `split` by attn_workspace's limit), each cut into equal shares of
 // its active tiles by the kernel, which alone knows the mask.
 //
-// A share takes at least 4 tiles beside full rounds and at least 12 where every
-// item is cut (the figures of tail_split); a launch whose items cannot have two
-// such shares is not split (4x30x300x128, 5 tiles: 13.2 us whole, 14.8 with
-// workgroups that only exit).  Items of several documents are short and of
-// different lengths, so they leave no long tail of their own.  So with more
-// than short_tail items past the last full round, and below one round, only
-// items of three quarters of the tiles or more are cut; D = 64 runs three
-// workgroups a CU with bf16 P.V, whose rounds are longer, so its line is lower
-// and above 128 items none is cut.  Attention kernel, bf16 P.V, in 1, 2, 3
-// documents, us, without split / every item cut / long items cut:
-//   1x30x2560x128 (88 past)  105 57 42 / 95 55 43 / 95 59 44
-//   1x19x4200x128 (115)     170 89 62 / 150 84 61 / 151 91 65
-//   1x30x1500x128 (104 past one per CU)  42 25 19 / 39 27 23 / 40 25 20
-//   1x17x4200x64 (49)       110 58 41 / 90 48 34 / 91 60 43
-//   1x30x2560x64 (88)        69 37 28 / 63 42 34 / 64 39 30
-//   2x30x1337x64 (148)       40 23 18 / 44 30 19 / 44 24 19
+// Beside full rounds, or past one item per CU, a share takes at least 4 tiles,
+// and items of fewer than 12 stay whole: a piece's start, partial and share of
+// the merge cost more than so short an item leaves idle.  Where every item is
+// cut, or more than 128 beside full rounds (whose pieces share CUs), it takes at
+// least 12.  A launch whose items cannot have two shares is not split
+// (4x30x300x128, 5 tiles: 13.2 us whole, 14.8 with workgroups that only exit).
+// Measured over 356 launches of 1 to 4 documents of 800 to 6912 tokens together,
+// geometric mean of the attention kernel's time over the uncut launch's, every
+// item cut into shares of 4 or more / these rules, for bf16 and fp8 P.V:
+//   past one per CU       D=128 0.97 / 0.95, 0.89 / 0.89;  D=64 0.91 / 0.90, 0.87 / 0.87
+//   1 to 128 past a round D=128 1.01 / 1.00, 0.97 / 0.96;  D=64 0.96 / 0.95, 0.96 / 0.96
+//   more                  D=128 1.03 / 0.98, 1.00 / 0.96;  D=64 1.02 / 0.98, 1.01 / 0.97
 struct MaskedSplit {
   TailSplit split;
   int share_from, share_min;
 };
 
-inline MaskedSplit masked_split(TailSplit split, int64_t n_items, int64_t nt, int64_t d) {
-  const int64_t share_min = split.whole == 0 ? 12 : 4, tail = n_items - split.whole;
-  const int64_t short_tail = d == 64 ? 64 : 96;
-  const bool any = split.whole == 0 || (split.whole >= kResidentWGs && tail <= short_tail);
-  MaskedSplit m{split, any ? 0 : (int)((3 * nt + 3) / 4), (int)share_min};
-  if (m.split.parts > nt / share_min) m.split.parts = (int)(nt / share_min);
-  if (m.split.parts < 2 || (split.whole != 0 && tail > 128)) m.split = TailSplit{n_items, 1};
+// Bytes of workspace a tile-masked split may take, of the unmasked launch's:
+// two pieces of 256 items at D = 128.  The allocation-free entry point's array
+// has them, so that every entry with the room cuts the same items.
+inline constexpr size_t kMaskedSplitBytes = (size_t)34 << 20;
+
+inline MaskedSplit masked_split(TailSplit split, int64_t n_items, int64_t nt) {
+  const bool few = split.whole != 0 && n_items % kResidentWGs - (n_items < kResidentWGs ? split.whole : 0) <= 128;
+  MaskedSplit m{split, few ? 12 : 0, few ? 4 : 12};
+  if (m.split.parts > nt / m.share_min) m.split.parts = (int)(nt / m.share_min);
+  if (m.split.parts < 2) m.split = TailSplit{n_items, 1};
   return m;
 }
 

@@ -186,9 +186,7 @@ size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
  * doc_ids needs: the summaries only (a few KB; 7 KB for the packed 1x30x6912
  * batch).  A tile-masked launch without doc_ids that is given room for them
  * (sage_attn_workspace_bytes) cuts its last items into shares of their active
- * tiles where that is faster, in as many as keep all partials within
- * SAGE_NOALLOC_SCRATCH_BYTES (sage_attn_fwd_noalloc cuts the same ones), or
- * none.  P is rounded in another frame in a cut item, so its rows can differ in
+ * tiles where that is faster (sage_attn_fwd_noalloc cuts the same ones).  P is rounded in another frame in a cut item, so its rows can differ in
  * the last bits between the two workspace sizes.  No reference counterpart. */
 size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
@@ -232,17 +230,17 @@ int sage_attn_fwd(const void* q_codes, const float* q_scale,
                   void* out, int out_layout, float* lse,
                   hipStream_t stream);
 
-/* Bytes of device scratch behind sage_attn_fwd_noalloc (per GPU). */
+/* Largest workspace of a call that sage_attn_fwd_noalloc takes. */
 #define SAGE_NOALLOC_SCRATCH_BYTES (16u << 20)
 
 /* sage_attn_fwd without the workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
- * workspace lives in a fixed device array of SAGE_NOALLOC_SCRATCH_BYTES per
- * GPU, held until the process ends; launches whose workspace (as
+ * workspace lives in a fixed device array per GPU (34 MiB: those bytes and room
+ * for the pieces of tile-masked items), held until the process ends; launches whose workspace (as
  * sage_attn_fwd: sage_attn_workspace_bytes unmasked,
  * sage_attn_masked_workspace_bytes with a tile mask or document ids) exceeds
- * it are rejected with SAGE_ERR_WORKSPACE before any launch (the unmasked
+ * SAGE_NOALLOC_SCRATCH_BYTES are rejected with SAGE_ERR_WORKSPACE before any launch (the unmasked
  * 1x30x4416x128 headline needs 6.9 MB, the masked packed 1x30x6912 batch
  * 7 KB).  The call allocates and frees
  * nothing and needs no memory cleared beforehand: every byte of scratch it

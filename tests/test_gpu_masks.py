@@ -274,13 +274,44 @@ def test_bf16_document_ids_on_the_pipelined_loop(cuda, lens, D):
     assert (lse.cpu() - wl.view_as(lse.cpu())).abs().max().item() <= 2e-3
 
 
+@pytest.mark.parametrize("H,D,pv,lens", [(24, 128, "fp8", [1000, 500]), (52, 128, "bf16", [1600]),
+                                         (60, 64, "bf16", [1537]), (60, 128, "fp8", [1500, 37])])
+def test_tile_masked_launches_cut(cuda, H, D, pv, lens):
+    """Launches whose items are cut: 32 past one per CU (those of 16 tiles, not
+    those of 8), 164 past a round in two shares each, and 268 of which 85 are
+    cut.  Against the uncut launch (a workspace of the masked size), to the
+    rounding of P in another frame."""
+    from futudiffu_amd import _lib
+    from futudiffu_amd import sage_attention as SA
+    B, N = 1, sum(lens)
+    lib = _lib.load()
+    q, k, v = (t.to(cuda) for t in O.make_inputs(B, H, N, D, seed=N + D))
+    mg = O.build_block_mask(lens, N).to(cuda)
+    print(f"masked launch cut {B}x{H}x{N}x{D} {pv}", flush=True)
+    qz = SA.quantize_qkv(q, k, v, qk="int8", pv=pv)
+    out, lse = SA.attn_from_quantized(qz, B, H, block_mask=mg)
+    wsb = int(lib.sage_attn_masked_workspace_bytes(B, H, N, D))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=cuda)
+    o1, l1 = torch.empty_like(out), torch.empty_like(lse)
+    _lib.check(lib.sage_attn_fwd(
+        qz.q_codes.data_ptr(), qz.q_scale.data_ptr(), qz.k_codes.data_ptr(), qz.k_scale.data_ptr(),
+        qz.v_op.data_ptr(), SA._ptr(qz.v_scale), B, H, N, D, 0, SA._PV[pv], 0, mg.data_ptr(), 0, mg.shape[0],
+        mg.shape[1], None, ws.data_ptr(), wsb, o1.data_ptr(), 0, l1.data_ptr(),
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert not torch.equal(out, o1)  # some item is cut
+    # the bound of test_tile_masked_tail_split: one bf16 step of an output up to 2
+    assert (out.float() - o1.float()).abs().max().item() <= 8e-3
+    assert (lse - l1).abs().max().item() <= 1e-4
+
+
 @pytest.mark.parametrize("B,H,D,lens", [(1, 30, 128, [1003, 771, 1297]), (1, 30, 128, [500, 400, 600]),
                                         (2, 30, 64, [1337]), (4, 30, 128, [300])])
 def test_tile_masked_launches_left_whole(cuda, B, H, D, lens):
     """Launches whose items are not cut, with room for partials: 208 items past a
-    round (their partials exceed the scratch in two pieces), short documents
-    below one round, 148 items past a round at D = 64, items of 5 tiles.  The
-    bits of the launch that has no room."""
+    round of at most 21 active tiles (two shares take 24), items of at most 10
+    below one round (they are cut from 12 on), 148 items past a round of 21
+    tiles, items of 5 tiles.  The bits of the launch that has no room."""
     from futudiffu_amd import _lib
     from futudiffu_amd import sage_attention as SA
     N = sum(lens)

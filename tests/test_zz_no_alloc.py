@@ -75,3 +75,6 @@ def test_noalloc_packed_batch_masked(cuda):
     _case(cuda, lib, 1, 30, 6912, 128, seed=73, pv="fp8", doc_segments=segs)
     print("noalloc packed 1x30x6912x128 int8/fp8 with the tile mask", flush=True)
     _case(cuda, lib, 1, 30, 6912, 128, seed=74, pv="fp8", tile_segments=segs)
+    # 164 tile-masked items past a round in two shares: 22 MB of partials
+    print("noalloc 1x52x1600x128 int8/bf16 with the tile mask", flush=True)
+    _case(cuda, lib, 1, 52, 1600, 128, seed=75, pv="bf16", tile_segments=[1600])
