@@ -1326,13 +1326,10 @@ __device__ __forceinline__ void store_partial_coherent(float* slot, const f32x16
 // had completed before they counted.  The item's slots are split_parts apart
 // from the next item's; its first `parts` are in use.  fac: LDS [8][128] floats.
 template <int D>
-__device__ __forceinline__ void merge_pieces(const AttnParams& p, int64_t si, int parts, float* fac) {
+__device__ __forceinline__ void merge_pieces(const AttnParams& p, int bh, int qt, int64_t si, int parts, float* fac) {
   constexpr int NC = D / 32;
   constexpr int kMaxParts = 8;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, h = lane >> 5, r = lane & 31;
-  const int nq = (int)(p.np / kRowsPerWG);
-  const int64_t pos = p.n_whole + si;
-  const int bh = (int)(pos / nq), qt = (int)(pos % nq);
   const int64_t q0 = (int64_t)qt * kRowsPerWG + 32 * w;
   const uint32_t* slots = reinterpret_cast<const uint32_t*>(p.part + si * p.split_parts * kPartFloats<D>);
   auto ld = [](const uint32_t* a) __attribute__((always_inline)) {
@@ -1452,11 +1449,12 @@ __device__ __forceinline__ int64_t xcd_range(int64_t i, int64_t n) {
   return x * per + (x < rem ? x : rem) + local;
 }
 
-// The end of a piece of split item si: its partial into `slot`, and where it
-// is the last of the item's `parts` to arrive, the merge.
+// The end of a piece of split item si, (bh, qt): its partial into `slot`, and
+// where it is the last of the item's `parts` to arrive, the merge.
 template <int D>
-__device__ __forceinline__ void leave_piece(const AttnParams& p, uint8_t* smem, int64_t slot, int64_t si, int parts,
-                                            const f32x16 (&o)[D / 32], float m_ref, float l_acc) {
+__device__ __forceinline__ void leave_piece(const AttnParams& p, uint8_t* smem, int bh, int qt, int64_t slot,
+                                            int64_t si, int parts, const f32x16 (&o)[D / 32], float m_ref,
+                                            float l_acc) {
   store_partial_coherent<D>(p.part + slot * kPartFloats<D>, o, m_ref, l_acc);
   wait_vmem();  // this piece's partial is at the coherence point before it counts
   __syncthreads();
@@ -1465,7 +1463,7 @@ __device__ __forceinline__ void leave_piece(const AttnParams& p, uint8_t* smem, 
   __syncthreads();
   if (*last == 0) return;
   __syncthreads();  // every wave has read the decision before the factors reuse the LDS
-  merge_pieces<D>(p, si, parts, reinterpret_cast<float*>(smem));
+  merge_pieces<D>(p, bh, qt, si, parts, reinterpret_cast<float*>(smem));
   if (threadIdx.x == 0)
     __hip_atomic_store(p.merge_ctr + si, p.merge_tag << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1504,7 +1502,7 @@ __global__ void __launch_bounds__(256, (kAttnWGs<D, PV, MASK>)) attn_fwd_kernel(
         store_partial<D>(p.part + c * kPartFloats<D>, o, m_ref, l_acc);
         return;
       }
-      leave_piece<D>(p, smem, c, si, p.split_parts, o, m_ref, l_acc);
+      leave_piece<D>(p, smem, bh, qt, c, si, p.split_parts, o, m_ref, l_acc);
       return;
     }
     const int64_t pos = xcd_range(b, p.n_whole);
@@ -1514,11 +1512,16 @@ __global__ void __launch_bounds__(256, (kAttnWGs<D, PV, MASK>)) attn_fwd_kernel(
     // A tile-masked item's pieces are equal shares of its active tiles, at
     // least share_min of them, and none where it has fewer than share_from:
     // it uses only as many of its workgroups as that gives, the others exit.
-    // The first pieces of all items come first, dealt to XCDs like a launch of
-    // their own: for the items that stay whole they are the launch's
-    // remaining items in their usual places, and the workgroups that exit come
-    // after (interleaved with the pieces of one item in a row, 1x30x1500x128
-    // in 2, 3 documents: 28.3, 25.3 us with bf16 P.V against 26.3, 20.0 uncut).
+    // The first pieces of all items come first: for the items that stay whole
+    // they are the launch's remaining items in their usual places, and the
+    // workgroups that exit come after (interleaved with the pieces of one item
+    // in a row, 1x30x1500x128 in 2, 3 documents: 28.3, 25.3 us with bf16 P.V
+    // against 26.3, 20.0 uncut).  Below two full rounds every XCD cuts the last
+    // items of its own range, whose K and V it has read (2x12x3000x128 in four
+    // documents 49.1 -> 40.4 us, 1x30x2200x64 fp8 P.V in three 34.6 -> 26.6,
+    // against the last heads' items dealt to all XCDs); after more rounds both
+    // are alike in the kernel, and the last heads' items are 1 % faster per op
+    // (packed 1x30x6912 350.5 against 354.9 us).
     // The loop starts at the first active tile and ends after the last:
     // walking the others one scalar load at a time took 10 us per short
     // document of the packed 6912-token batch.
@@ -1526,23 +1529,28 @@ __global__ void __launch_bounds__(256, (kAttnWGs<D, PV, MASK>)) attn_fwd_kernel(
     int64_t si = 0;
     int part = 0, parts = 1, count;
     int2 ends;
-    auto whole_item = [&]() __attribute__((always_inline)) {
-      if (p.split_parts > 1) {
-        const int64_t pos = xcd_range(b, p.n_whole);
-        bh = (int)(pos / nq);
-        qt = (int)(pos % nq);
+    const int items = p.bh * nq;
+    auto place = [&](int i) __attribute__((always_inline)) {  // (bh, qt) of place i: whole items, then cut ones
+      if (items < 2 * kResidentWGs || p.split_parts == 1) {
+        item_of(i, items, p.bh, nq, p.light_last, bh, qt);
       } else {
-        item_of((int)b, (int)gridDim.x, p.bh, nq, p.light_last, bh, qt);
+        const int pos = i < p.n_whole ? (int)xcd_range(i, p.n_whole)
+                                      : p.n_whole + (int)xcd_range(i - p.n_whole, items - p.n_whole);
+        bh = pos / nq;
+        qt = pos % nq;
       }
+    };
+    auto whole_item = [&]() __attribute__((always_inline)) {
+      place((int)b);
       ends = active_ends(mask_row(p, bh, qt), p.nt, count);
     };
     auto share = [&]() __attribute__((always_inline)) -> bool {  // false: not used
-      const int64_t c = b - p.n_whole, n_cut = (int64_t)p.bh * nq - p.n_whole;
-      part = (int)(c / n_cut);
-      si = xcd_range(c - part * n_cut, n_cut);
-      const int64_t pos = p.n_whole + si;
-      bh = (int)(pos / nq);
-      qt = (int)(pos % nq);
+      const int stride = (items - p.n_whole + 7) & ~7;  // of the parts: an item's run on one XCD
+      const int c = (int)b - p.n_whole;
+      part = c / stride;
+      si = c - part * stride;
+      if (p.n_whole + si >= items) return false;
+      place((int)(p.n_whole + si));
       const uint8_t* row = mask_row(p, bh, qt);
       ends = active_ends(row, p.nt, count);
       parts = count < p.share_from ? 1 : max(1, min(p.split_parts, count / p.share_min));
@@ -1560,7 +1568,7 @@ __global__ void __launch_bounds__(256, (kAttnWGs<D, PV, MASK>)) attn_fwd_kernel(
       if (parts == 1)
         store_rows_final<D, PV>(p, smem, bh, qt, o, m_ref, l_acc);
       else
-        leave_piece<D>(p, smem, si * p.split_parts + part, si, parts, o, m_ref, l_acc);
+        leave_piece<D>(p, smem, bh, qt, si * p.split_parts + part, si, parts, o, m_ref, l_acc);
     };
     if constexpr (PV == kPV_FP8) {
       // a copy of the loop for each (sharing one, D = 64 runs 3 % slower:
@@ -1685,7 +1693,9 @@ hipError_t launch_attn_g(int mask, const AttnParams& p, hipStream_t st) {
   const int64_t items = (int64_t)p.bh * (p.np / kRowsPerWG);
   const int64_t n_split = items - p.n_whole;  // 0 with document ids
   // with document ids the first heavy_max * h workgroups take the listed split query tiles
-  const dim3 grid((unsigned)(p.n_whole + n_split * p.split_parts + ((mask & 2) ? (int64_t)p.heavy_max * p.h : 0)));
+  // a tile-masked launch's parts are a multiple of the XCD count apart
+  const int64_t cut = mask == 1 ? (n_split + 7) / 8 * 8 : n_split;
+  const dim3 grid((unsigned)(p.n_whole + cut * p.split_parts + ((mask & 2) ? (int64_t)p.heavy_max * p.h : 0)));
   // the accumulator dump exists for the per-token, unmasked kernels
   constexpr bool kDumpable = GRAN == kGRAN_TOKEN;
   if (p.s_dump != nullptr) {

@@ -167,11 +167,13 @@ inline TailSplit tail_split(int64_t n_items, int64_t nt, int64_t d) {
 // least 12.  A launch whose items cannot have two shares is not split
 // (4x30x300x128, 5 tiles: 13.2 us whole, 14.8 with workgroups that only exit).
 // Measured over 356 launches of 1 to 4 documents of 800 to 6912 tokens together,
-// geometric mean of the attention kernel's time over the uncut launch's, every
-// item cut into shares of 4 or more / these rules, for bf16 and fp8 P.V:
-//   past one per CU       D=128 0.97 / 0.95, 0.89 / 0.89;  D=64 0.91 / 0.90, 0.87 / 0.87
-//   1 to 128 past a round D=128 1.01 / 1.00, 0.97 / 0.96;  D=64 0.96 / 0.95, 0.96 / 0.96
-//   more                  D=128 1.03 / 0.98, 1.00 / 0.96;  D=64 1.02 / 0.98, 1.01 / 0.97
+// geometric mean of the attention kernel's time over the uncut launch's, for bf16
+// and fp8 P.V (slower ones by 12 % at most):
+//   past one per CU       D=128 0.94, 0.89;  D=64 0.90, 0.87
+//   1 to 128 past a round D=128 0.97, 0.95;  D=64 0.94, 0.93
+//   more                  D=128 0.98, 0.96;  D=64 0.98, 0.96
+// Shares of 4 everywhere are 3 to 9 % slower than these where more are past a
+// round, and 1 to 2 % elsewhere (short items).
 struct MaskedSplit {
   TailSplit split;
   int share_from, share_min;

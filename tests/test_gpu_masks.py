@@ -274,12 +274,11 @@ def test_bf16_document_ids_on_the_pipelined_loop(cuda, lens, D):
     assert (lse.cpu() - wl.view_as(lse.cpu())).abs().max().item() <= 2e-3
 
 
-@pytest.mark.parametrize("H,D,pv,lens", [(24, 128, "fp8", [1000, 500]), (52, 128, "bf16", [1600]),
+@pytest.mark.parametrize("H,D,pv,lens", [(24, 128, "fp8", [500, 1000]), (52, 128, "bf16", [1600]),
                                          (60, 64, "bf16", [1537]), (60, 128, "fp8", [1500, 37])])
 def test_tile_masked_launches_cut(cuda, H, D, pv, lens):
-    """Launches whose items are cut: 32 past one per CU (those of 16 tiles, not
-    those of 8), 164 past a round in two shares each, and 268 of which 85 are
-    cut.  Against the uncut launch (a workspace of the masked size), to the
+    """Launches whose items are cut: 32 past one per CU, of 16 active tiles, 164
+    past a round in two shares each, and 268 of which 85 are cut.  Against the uncut launch (a workspace of the masked size), to the
     rounding of P in another frame."""
     from futudiffu_amd import _lib
     from futudiffu_amd import sage_attention as SA
