@@ -532,3 +532,21 @@ def test_attention_kernels_keep_their_workgroups_per_cu(tmp_path):
             assert field("group_segment_fixed_size") * wgs <= 160 << 10, m.group(0)
             seen += 1
     assert seen == 64
+
+
+def test_attention_kernels_start_on_8_kib(tmp_path):
+    """The code of every built attention kernel starts on 8 KiB, so that its
+    place, which small launches feel, does not follow unrelated changes."""
+    from futudiffu_amd import _lib, build
+    tools = os.path.join(os.path.dirname(os.path.dirname(build.hipcc())), "llvm", "bin")
+    objdump, readelf = (os.path.join(tools, t) for t in ("llvm-objdump", "llvm-readelf"))
+    if not (os.path.exists(objdump) and os.path.exists(readelf)):
+        pytest.skip("no ROCm binutils")
+    lib = tmp_path / "lib.so"
+    lib.write_bytes(open(_lib.load()._name, "rb").read())
+    subprocess.run([objdump, "--offloading", str(lib)], cwd=tmp_path, check=True, capture_output=True)
+    starts = []
+    for obj in tmp_path.glob("lib.so.*gfx950*"):
+        syms = subprocess.run([readelf, "--dyn-syms", "-W", str(obj)], check=True, capture_output=True, text=True).stdout
+        starts += [int(m, 16) for m in re.findall(r"([0-9a-f]{16}) +\d+ FUNC .*attn_fwd_kernel", syms)]
+    assert len(starts) > 64 and not any(a % 8192 for a in starts)
