@@ -262,8 +262,10 @@ struct AttnWorkspace {
   TailSplit split;
 };
 // `masked`: a launch that splits no item (document ids, or a tile mask in a
-// workspace without room for partials).  `limit` (0: none): the tail items in
-// as many pieces as keep `bytes` within it; whole if that is under two.
+// workspace without room for partials).  `limit` (0: none): the partials
+// kept within it, by fewer pieces an item up to one item per CU and by fewer
+// items beyond (then no more pieces than CUs); none if that leaves under two
+// pieces.
 AttnWorkspace attn_workspace(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false, size_t limit = 0);
 size_t attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d, bool masked = false);
 hipError_t launch_tile_mask(const int32_t* doc, int64_t nb, int64_t n, int32_t pad_fill, uint8_t* mask,

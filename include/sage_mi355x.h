@@ -174,9 +174,9 @@ int sage_quantize_from_qkv(const void* qkv, const float* q_norm_w, const float* 
  * the 128-row items that an unmasked launch splits (the items past the last
  * whole round of 512 resident workgroups; below one round the items past one
  * per CU; every item of a launch of fewer items than CUs and enough key tiles)
- * and an 8-byte arrival counter per split item (the last piece to finish merges the item's partials; the
- * counters need no clearing, each call tags them with a value no earlier
- * call used).  Enough for every launch of that shape; a launch of fewer items
+ * and an 8-byte arrival counter per split item (the last piece to finish merges
+ * the item's partials; the counters need no clearing, each call tags them with
+ * a value no earlier call used).  Enough for every launch of that shape; a launch of fewer items
  * than CUs also takes a workspace of the summaries alone, and runs its items
  * whole then.  No reference counterpart (the Triton launch needs no
  * workspace). */
@@ -186,8 +186,9 @@ size_t sage_attn_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
  * doc_ids needs: the summaries only (a few KB; 7 KB for the packed 1x30x6912
  * batch).  A tile-masked launch without doc_ids that is given room for them
  * (sage_attn_workspace_bytes) cuts its last items into shares of their active
- * tiles where that is faster (sage_attn_fwd_noalloc cuts the same ones).  P is rounded in another frame in a cut item, so its rows can differ in
- * the last bits between the two workspace sizes.  No reference counterpart. */
+ * tiles where that is faster (sage_attn_fwd_noalloc cuts the same ones).  P is
+ * rounded in another frame in a cut item, so its rows can differ in the last
+ * bits between the two workspace sizes.  No reference counterpart. */
 size_t sage_attn_masked_workspace_bytes(int64_t b, int64_t h, int64_t n, int64_t d);
 
 /* Fused attention forward over pre-quantized operands.
